@@ -551,6 +551,25 @@ static bool try_launch_row(const vf_lbm_parameter& p, const BoxArgs& a, const K1
     return true;
 }
 
+// Whether the in-place node kernel takes its workgroups in XCD block ranges (xcd_block): where the
+// spans of a plane share cache lines at their ends (a plane is not a whole number of lines) the
+// ranges keep both sharers in one L2. Measured on MI355X, ranges against launch order, us per step:
+//   cache-resident   66^3 FP32 11.8 / 12.9, FP16 10.0 / 12.3; 130 x 70 x 70 FP32 23.2 / 26.5;
+//                    194 x 98 x 98 FP32 62.5 / 70.8, FP16 41.9 / 44.1; 258 x 130 x 130 FP16 91 / 98
+//   streaming FP32   258 x 130 x 130 190 / 206; 300 x 301 x 150 582 / 644; 251 x 187 x 133 285 / 285
+//   streaming 16-bit 251 x 187 x 133 186 / 158; 300 x 301 x 150 340 / 324; 333 x 200 x 290 495 / 456
+// A 16-bit span is half as long, so on a lattice larger than the cache eight distant regions cost
+// its streams more DRAM efficiency than the shared lines do: those keep the launch order. A level
+// that fits by itself inside a hierarchy that does not (258 x 130 x 130 FP16 in the two-level step)
+// takes the ranges: 315 us per coarse step against 319 in launch order.
+template <class S> static bool node_xcd_ranges(const vf_lbm_parameter& p)
+{
+    const int choice = p.kernelChoice.rowXcdRanges;
+    if (choice == 1 || choice == 2) return choice == 1;
+    return xcd_planes(p.nx, p.ny, sizeof(S), 0) &&
+           (sizeof(S) == 4 || 27 * p.numberOfNodes * sizeof(S) <= kCacheResidentBytes);
+}
+
 template <class S, bool EVEN>
 static void launch_box_t(const vf_lbm_parameter& p, bool macro, hipStream_t s)
 {
@@ -562,14 +581,7 @@ static void launch_box_t(const vf_lbm_parameter& p, bool macro, hipStream_t s)
     if (try_launch_row<S, EVEN>(p, a, r, macro, nullptr, s)) return;
     const dim3 grid(plane_blocks(p.nx, p.ny), p.nz), bx(kBoxBlock);
     const FusedBB none{};
-    // XCD block ranges where the working set streams and planes share cache lines at their ends
-    // (or where pinned): inside the two-level step they take the 258 x 130 x 130 FP16 coarse
-    // level's fetched bytes from 1.21 to 0.99 x algorithmic at the same time (107 against
-    // 104-109 us); on a cache-resident lattice (the sphere channel) they cost 59 -> 61 us
-    const uint64_t ws = p.workingSetBytes ? p.workingSetBytes : 27 * p.numberOfNodes * sizeof(S);
-    const bool xcd = p.kernelChoice.rowXcdRanges == 1 ||
-                     (p.kernelChoice.rowXcdRanges == 0 && ws > kCacheResidentBytes &&
-                      xcd_planes(p.nx, p.ny, sizeof(S), 0));
+    const bool xcd = node_xcd_ranges<S>(p);
     if (mask && macro) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, true, true>), grid, dim3(bx), 0, s, f, a, r, none);
     else if (mask && xcd) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, true, false, false, true>), grid, dim3(bx), 0, s, f, a, r, none);
     else if (mask) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, true, false>), grid, dim3(bx), 0, s, f, a, r, none);
@@ -590,7 +602,9 @@ static bool launch_box_bb_t(const vf_lbm_parameter& p, bool macro, const FusedBB
     S* f = static_cast<S*>(p.distributions);
     const bool mask = p.fluidMask != nullptr;
     const dim3 grid(plane_blocks(p.nx, p.ny), p.nz), bx(kBoxBlock);
+    const bool xcd = node_xcd_ranges<S>(p);
     if (mask && macro) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, true, true, true>), grid, dim3(bx), 0, s, f, a, r, bb);
+    else if (mask && xcd) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, true, false, true, true>), grid, dim3(bx), 0, s, f, a, r, bb);
     else if (mask) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, true, false, true>), grid, dim3(bx), 0, s, f, a, r, bb);
     else if (macro) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, false, true, true>), grid, dim3(bx), 0, s, f, a, r, bb);
     else hipLaunchKernelGGL((k17_box_kernel<S, EVEN, false, false, true>), grid, dim3(bx), 0, s, f, a, r, bb);
