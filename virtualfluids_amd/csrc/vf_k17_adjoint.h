@@ -9,13 +9,19 @@
 //     -> backward chimera x, y, z -> post-collision populations,
 //
 // and the reverse walks it backwards: the backward chimera lines are linear in their inputs
-// for a fixed velocity (3x3 transposes plus a velocity term), the moment algebra is
-// differentiated term by term, the limiter x -> x N / (|x| + L) has the derivative
-// N L / (|x| + L)^2, and the forward chimera lines and the macroscopic sums close the chain.
-// Every forward intermediate the reverse needs is recomputed from f (nothing is stored per
+// for a fixed velocity (3x3 transposes), the moment algebra is differentiated term by term, the
+// limiter x -> x N / (|x| + L) has the derivative N L / (|x| + L)^2, and the transposed forward
+// chimera lines and the macroscopic sums close the chain. The velocity adjoint needs no
+// intermediate of the passes: with true central moments M_abc (the shifted ones plus the rest
+// moments of the weights) and the velocity as the centre,
+//   d M_abc / d u_x = -a M_(a-1)bc,   d f / d u_x = B(a N_(a-1)bc)  (B the backward chimera),
+// so it is a short sum of products of moments and their adjoints on either side of the cumulant
+// stage. Every forward intermediate the reverse needs is recomputed from f (nothing is stored per
 // node between steps). Arrays inside this file are indexed idx(a, b, c) = a + 3 b + 9 c: for
 // populations (a, b, c) is the velocity plus one per axis, for moments the orders per axis.
 #pragma once
+
+#include <type_traits>
 
 #include "vf_k17.h"
 
@@ -44,57 +50,49 @@ VF_HD constexpr int dir_of_idx(int i)
          : i == idx(2, 0, 0) ? dPMM : dMMM;
 }
 
-// Chimera weights K of a line: x lines (b, c) -> v(b) v(c); y lines (a, c) -> w(a) v(c);
-// z lines (a, b) -> w(a) w(b), with v = (1, 0, 1/3) and w = (1/6, 2/3, 1/6).
-VF_HD constexpr float kv(int i) { return i == 1 ? 0.0f : (i == 0 ? 1.0f : 1.0f / 3.0f); }
-VF_HD constexpr float kw(int i) { return i == 1 ? 2.0f / 3.0f : 1.0f / 6.0f; }
+// moments of the weights: kr(a) kr(b) kr(c) is what the shifted moment abc lacks of the true one
+VF_HD constexpr float kr(int i) { return i == 1 ? 0.0f : (i == 0 ? 1.0f : 1.0f / 3.0f); }
 
-// forward chimera line: (a, b, c) -> (s, d - u (s+K), e - 2 u d + (s+K) u^2)
-VF_HD void line_fwd(float& a, float& b, float& c, float u, float K)
+// Transposed backward chimera line. The line (a, b, c) -> (lo, mid, hi) is the inverse of the
+// central moments about u; (A, B, C) hold the adjoints of lo, mid, hi on entry and of a, b, c on
+// return: C = (L + H)/2 - M, B = 2 u C + (H - L)/2, A = M + u (u C + (H - L)/2).
+VF_HD void line_bwd_t(float& A, float& B, float& C, float u, float u2)
 {
-    const float e = a + c, d = c - a, s = e + b, sK = s + K;
-    a = s;
-    b = d - u * sK;
-    c = e - 2.0f * u * d + sK * u * u;
+    const float h = 0.5f * (C - A);
+    const float c = __builtin_fmaf(0.5f, A + C, -B);
+    A = __builtin_fmaf(u, __builtin_fmaf(u, c, h), B);
+    B = __builtin_fmaf(u2, c, h); // u2 = 2 u
+    C = c;
 }
 
-// its reverse: (a, b, c) are the line's inputs, (A, B, C) the adjoints of its outputs;
-// returns the adjoints of the inputs in (A, B, C) and adds the velocity term to ub
-VF_HD void line_fwd_rev(float a, float b, float c, float u, float K, float& A, float& B, float& C, float& ub)
+// Transposed forward chimera line (s, d - u s, e - 2 u d + u^2 s of a, b, c with s = a + b + c,
+// d = c - a, e = a + c): (A, B, C) hold the adjoints of the moments on entry, of the line's
+// inputs on return; dj is an adjoint of d from elsewhere (the momentum sums).
+VF_HD void line_fwd_t(float& A, float& B, float& C, float u, float m2u, float usq)
 {
-    const float e = a + c, d = c - a, s = e + b, sK = s + K;
-    ub += -sK * B + (2.0f * u * sK - 2.0f * d) * C;
-    const float sb = A - u * B + u * u * C;
-    const float db = B - 2.0f * u * C;
-    const float eb = C + sb;
-    A = eb - db;
-    B = sb;
-    C = eb + db;
+    const float s = __builtin_fmaf(usq, C, __builtin_fmaf(-u, B, A));
+    const float d = __builtin_fmaf(m2u, C, B);
+    const float e = C + s;
+    A = e - d;
+    B = s;
+    C = e + d;
 }
-
-// backward chimera line (the inverse transform): lo = a0 (a+K) + b0 b + c/2,
-// hi = a2 (a+K) + b2 b + c/2, mid = a - lo - hi
-VF_HD void line_bwd(float& a, float& b, float& c, float u, float K)
+VF_HD void line_fwd_t(float& A, float& B, float& C, float u, float m2u, float usq, float dj)
 {
-    const float a0 = 0.5f * (u * u - u), b0 = u - 0.5f, a2 = 0.5f * (u * u + u), b2 = u + 0.5f;
-    const float aK = a + K;
-    const float lo = a0 * aK + b0 * b + 0.5f * c;
-    const float hi = a2 * aK + b2 * b + 0.5f * c;
-    const float mid = (a - lo) - hi;
-    a = lo;
-    b = mid;
-    c = hi;
+    const float s = __builtin_fmaf(usq, C, __builtin_fmaf(-u, B, A));
+    const float d = __builtin_fmaf(m2u, C, B) + dj;
+    const float e = C + s;
+    A = e - d;
+    B = s;
+    C = e + d;
 }
-
-VF_HD void line_bwd_rev(float a, float b, float u, float K, float& A, float& B, float& C, float& ub)
+// ... where the second moment is not used
+VF_HD void line_fwd01_t(float& A, float& B, float& C, float u)
 {
-    const float a0 = 0.5f * (u * u - u), b0 = u - 0.5f, a2 = 0.5f * (u * u + u), b2 = u + 0.5f;
-    const float aK = a + K;
-    const float L = A, M = B, H = C;
-    ub += (L - M) * (b0 * aK + b) + (H - M) * (b2 * aK + b);
-    A = a0 * L + a2 * H + (1.0f - a0 - a2) * M;
-    B = b0 * L + b2 * H - (b0 + b2) * M;
-    C = 0.5f * (L + H) - M;
+    const float s = __builtin_fmaf(-u, B, A), d = B;
+    A = s - d;
+    B = s;
+    C = s + d;
 }
 
 // ---- forward state --------------------------------------------------------------------------
@@ -127,27 +125,47 @@ VF_HD void macro_of(const float (&p)[27], const K17Rates& r, float vscale, Macro
     m.vz = jz * rs + r.fz;
 }
 
-// z pass (all 27 outputs are used downstream)
-VF_HD void pass_z(float (&p)[27], float vz)
+// Forward chimera passes z, y, x of the moments the cumulant stage reads (k17_collide's lines: a
+// moment of fourth order or higher is replaced there, never read). p: populations on entry, on
+// return the moments of order <= 3 at their idx (the other entries hold nothing).
+VF_HD void forward_moments(float (&p)[27], float vx, float vy, float vz)
 {
+    const float vx2 = vx * vx, vy2 = vy * vy, vz2 = vz * vz;
+    {
+        const float m2u = -2.0f * vz;
+        auto z = [&](int i, int j, auto num) {
+            constexpr int K = decltype(num)::value;
+            fwd<K, 36>(p[idx(i, j, 0)], p[idx(i, j, 1)], p[idx(i, j, 2)], vz, vz2, m2u);
+        };
+        using C1 = std::integral_constant<int, 1>;
+        using C4 = std::integral_constant<int, 4>;
+        using C16 = std::integral_constant<int, 16>;
+        z(0, 0, C1{}); z(1, 0, C4{}); z(2, 0, C1{});
+        z(0, 1, C4{}); z(1, 1, C16{}); z(2, 1, C4{});
+        z(0, 2, C1{}); z(1, 2, C4{}); z(2, 2, C1{});
+    }
+    {
+        const float m2u = -2.0f * vy;
+        fwd<1, 6>(p[idx(0, 0, 0)], p[idx(0, 1, 0)], p[idx(0, 2, 0)], vy, vy2, m2u);
+        fwd<2, 3>(p[idx(1, 0, 0)], p[idx(1, 1, 0)], p[idx(1, 2, 0)], vy, vy2, m2u);
+        fwd<1, 6>(p[idx(2, 0, 0)], p[idx(2, 1, 0)], p[idx(2, 2, 0)], vy, vy2, m2u);
 #pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int j = 0; j < 3; ++j) line_fwd(p[idx(i, j, 0)], p[idx(i, j, 1)], p[idx(i, j, 2)], vz, kw(i) * kw(j));
-}
-VF_HD void pass_y(float (&p)[27], float vy)
-{
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int k = 0; k < 3; ++k) line_fwd(p[idx(i, 0, k)], p[idx(i, 1, k)], p[idx(i, 2, k)], vy, kw(i) * kv(k));
-}
-VF_HD void pass_x(float (&p)[27], float vx)
-{
-#pragma unroll
-    for (int j = 0; j < 3; ++j)
-#pragma unroll
-        for (int k = 0; k < 3; ++k) line_fwd(p[idx(0, j, k)], p[idx(1, j, k)], p[idx(2, j, k)], vx, kv(j) * kv(k));
+        for (int i = 0; i < 3; ++i) fwd<0, 1>(p[idx(i, 0, 1)], p[idx(i, 1, 1)], p[idx(i, 2, 1)], vy, vy2, m2u);
+        fwd01<1, 18>(p[idx(0, 0, 2)], p[idx(0, 1, 2)], p[idx(0, 2, 2)], vy);
+        fwd01<2, 9>(p[idx(1, 0, 2)], p[idx(1, 1, 2)], p[idx(1, 2, 2)], vy);
+        fwd01<1, 18>(p[idx(2, 0, 2)], p[idx(2, 1, 2)], p[idx(2, 2, 2)], vy);
+    }
+    {
+        const float m2u = -2.0f * vx;
+        fwd<1, 1>(p[idx(0, 0, 0)], p[idx(1, 0, 0)], p[idx(2, 0, 0)], vx, vx2, m2u);
+        fwd<0, 1>(p[idx(0, 1, 0)], p[idx(1, 1, 0)], p[idx(2, 1, 0)], vx, vx2, m2u);
+        fwd01<1, 3>(p[idx(0, 2, 0)], p[idx(1, 2, 0)], p[idx(2, 2, 0)], vx);
+        fwd<0, 1>(p[idx(0, 0, 1)], p[idx(1, 0, 1)], p[idx(2, 0, 1)], vx, vx2, m2u);
+        fwd01<0, 1>(p[idx(0, 1, 1)], p[idx(1, 1, 1)], p[idx(2, 1, 1)], vx);
+        p[idx(0, 2, 1)] = (p[idx(0, 2, 1)] + p[idx(2, 2, 1)]) + p[idx(1, 2, 1)];
+        fwd01<1, 3>(p[idx(0, 0, 2)], p[idx(1, 0, 2)], p[idx(2, 0, 2)], vx);
+        p[idx(0, 1, 2)] = (p[idx(0, 1, 2)] + p[idx(2, 1, 2)]) + p[idx(1, 1, 2)];
+    }
 }
 
 // Moments of the cumulant stage that the relaxation reads, and everything derived from them.
@@ -484,68 +502,104 @@ VF_HD void mid_reverse(const Mid& s, const Macro& mc, const K17Rates& r, const f
     }
 }
 
-// backward chimera x, y, z on moments M (idx order), giving populations in idx order
-VF_HD void backward_chimera(float (&M)[27], float vx, float vy, float vz)
+// Transposed backward chimera: A holds the adjoints of the populations on entry (idx order) and
+// of the moments N that entered the passes on return; the velocity's part, sum a A_abc N_(a-1)bc
+// per axis over the true moments, is added to vxb, vyb, vzb.
+VF_HD void backward_chimera_t(float (&A)[27], float vx, float vy, float vz)
 {
+    const float vx2 = 2.0f * vx, vy2 = 2.0f * vy, vz2 = 2.0f * vz;
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = 0; j < 3; ++j) line_bwd_t(A[idx(i, j, 0)], A[idx(i, j, 1)], A[idx(i, j, 2)], vz, vz2);
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) line_bwd_t(A[idx(i, 0, k)], A[idx(i, 1, k)], A[idx(i, 2, k)], vy, vy2);
 #pragma unroll
     for (int j = 0; j < 3; ++j)
 #pragma unroll
-        for (int k = 0; k < 3; ++k) line_bwd(M[idx(0, j, k)], M[idx(1, j, k)], M[idx(2, j, k)], vx, kv(j) * kv(k));
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int k = 0; k < 3; ++k) line_bwd(M[idx(i, 0, k)], M[idx(i, 1, k)], M[idx(i, 2, k)], vy, kw(i) * kv(k));
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int j = 0; j < 3; ++j) line_bwd(M[idx(i, j, 0)], M[idx(i, j, 1)], M[idx(i, j, 2)], vz, kw(i) * kw(j));
+        for (int k = 0; k < 3; ++k) line_bwd_t(A[idx(0, j, k)], A[idx(1, j, k)], A[idx(2, j, k)], vx, vx2);
 }
-
-// its reverse: N the moments entering the passes; A holds the adjoints of the outputs on entry
-// and the adjoints of N on return; the velocity terms are added to vxb, vyb, vzb
+VF_HD void backward_velocity_adjoint(const float (&N)[27], const float (&A)[27], float& vxb, float& vyb, float& vzb)
+{
+    float x2 = 0.0f, y2 = 0.0f, z2 = 0.0f; // the second-order halves
+#pragma unroll
+    for (int b = 0; b < 3; ++b)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const float k = kr(b) * kr(c);
+            vxb += A[idx(1, b, c)] * (k ? N[idx(0, b, c)] + k : N[idx(0, b, c)]);
+            vyb += A[idx(b, 1, c)] * (k ? N[idx(b, 0, c)] + k : N[idx(b, 0, c)]);
+            vzb += A[idx(b, c, 1)] * (k ? N[idx(b, c, 0)] + k : N[idx(b, c, 0)]);
+            x2 += A[idx(2, b, c)] * N[idx(1, b, c)];
+            y2 += A[idx(b, 2, c)] * N[idx(b, 1, c)];
+            z2 += A[idx(b, c, 2)] * N[idx(b, c, 1)];
+        }
+    vxb += 2.0f * x2;
+    vyb += 2.0f * y2;
+    vzb += 2.0f * z2;
+}
 VF_HD void backward_chimera_rev(const float (&N)[27], float vx, float vy, float vz, float (&A)[27], float& vxb,
                                 float& vyb, float& vzb)
 {
+    backward_chimera_t(A, vx, vy, vz);
+    backward_velocity_adjoint(N, A, vxb, vyb, vzb);
+}
+
+// The forward chimera's part of the velocity adjoint, -sum a mb_abc M_(a-1)bc per axis over the
+// true moments; mb is nonzero up to third order only (forward_moments).
+VF_HD void forward_velocity_adjoint(const Mid& s, const float (&mb)[27], float& vxb, float& vyb, float& vzb)
+{
+    const float t = 1.0f / 3.0f;
+    const float rho = s.m000 + 1.0f, m200 = s.m200 + t, m020 = s.m020 + t, m002 = s.m002 + t;
+    vxb -= mb[idx(1, 0, 0)] * rho + mb[idx(1, 1, 0)] * s.m010 + mb[idx(1, 0, 1)] * s.m001 + mb[idx(1, 1, 1)] * s.m011 +
+           mb[idx(1, 2, 0)] * m020 + mb[idx(1, 0, 2)] * m002 +
+           2.0f * (mb[idx(2, 0, 0)] * s.m100 + mb[idx(2, 1, 0)] * s.m110 + mb[idx(2, 0, 1)] * s.m101);
+    vyb -= mb[idx(0, 1, 0)] * rho + mb[idx(1, 1, 0)] * s.m100 + mb[idx(0, 1, 1)] * s.m001 + mb[idx(1, 1, 1)] * s.m101 +
+           mb[idx(2, 1, 0)] * m200 + mb[idx(0, 1, 2)] * m002 +
+           2.0f * (mb[idx(0, 2, 0)] * s.m010 + mb[idx(1, 2, 0)] * s.m110 + mb[idx(0, 2, 1)] * s.m011);
+    vzb -= mb[idx(0, 0, 1)] * rho + mb[idx(1, 0, 1)] * s.m100 + mb[idx(0, 1, 1)] * s.m010 + mb[idx(1, 1, 1)] * s.m110 +
+           mb[idx(2, 0, 1)] * m200 + mb[idx(0, 2, 1)] * m020 +
+           2.0f * (mb[idx(0, 0, 2)] * s.m001 + mb[idx(1, 0, 2)] * s.m101 + mb[idx(0, 1, 2)] * s.m011);
+}
+
+// Transposed forward chimera x, y, z: mb holds the adjoints of the moments of order <= 3 on entry
+// and of the populations on return. drhob, jxb, jyb, jzb: the adjoints of the density and momentum
+// sums, which are the zeroth moment and the first differences of the same lines.
+VF_HD void forward_chimera_t(float (&mb)[27], float vx, float vy, float vz, float drhob, float jxb, float jyb,
+                             float jzb)
+{
+    const float vx2 = vx * vx, vy2 = vy * vy, vz2 = vz * vz;
+    mb[idx(0, 0, 0)] += drhob;
     {
-        float Y[27];  // input of the z pass = N after the x and y passes
+        const float m2u = -2.0f * vx;
+        line_fwd_t(mb[idx(0, 0, 0)], mb[idx(1, 0, 0)], mb[idx(2, 0, 0)], vx, m2u, vx2, jxb);
+        line_fwd_t(mb[idx(0, 1, 0)], mb[idx(1, 1, 0)], mb[idx(2, 1, 0)], vx, m2u, vx2);
+        line_fwd_t(mb[idx(0, 0, 1)], mb[idx(1, 0, 1)], mb[idx(2, 0, 1)], vx, m2u, vx2);
+        line_fwd01_t(mb[idx(0, 2, 0)], mb[idx(1, 2, 0)], mb[idx(2, 2, 0)], vx);
+        line_fwd01_t(mb[idx(0, 1, 1)], mb[idx(1, 1, 1)], mb[idx(2, 1, 1)], vx);
+        line_fwd01_t(mb[idx(0, 0, 2)], mb[idx(1, 0, 2)], mb[idx(2, 0, 2)], vx);
+        mb[idx(1, 2, 1)] = mb[idx(2, 2, 1)] = mb[idx(0, 2, 1)];
+        mb[idx(1, 1, 2)] = mb[idx(2, 1, 2)] = mb[idx(0, 1, 2)];
+    }
+    {
+        const float m2u = -2.0f * vy;
 #pragma unroll
-        for (int i = 0; i < 27; ++i) Y[i] = N[i];
-#pragma unroll
-        for (int j = 0; j < 3; ++j)
-#pragma unroll
-            for (int k = 0; k < 3; ++k) line_bwd(Y[idx(0, j, k)], Y[idx(1, j, k)], Y[idx(2, j, k)], vx, kv(j) * kv(k));
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-#pragma unroll
-            for (int k = 0; k < 3; ++k) line_bwd(Y[idx(i, 0, k)], Y[idx(i, 1, k)], Y[idx(i, 2, k)], vy, kw(i) * kv(k));
+        for (int i = 0; i < 3; ++i) {
+            line_fwd_t(mb[idx(i, 0, 0)], mb[idx(i, 1, 0)], mb[idx(i, 2, 0)], vy, m2u, vy2, jyb);
+            line_fwd_t(mb[idx(i, 0, 1)], mb[idx(i, 1, 1)], mb[idx(i, 2, 1)], vy, m2u, vy2);
+            line_fwd01_t(mb[idx(i, 0, 2)], mb[idx(i, 1, 2)], mb[idx(i, 2, 2)], vy);
+        }
+    }
+    {
+        const float m2u = -2.0f * vz;
 #pragma unroll
         for (int i = 0; i < 3; ++i)
 #pragma unroll
             for (int j = 0; j < 3; ++j)
-                line_bwd_rev(Y[idx(i, j, 0)], Y[idx(i, j, 1)], vz, kw(i) * kw(j), A[idx(i, j, 0)], A[idx(i, j, 1)],
-                             A[idx(i, j, 2)], vzb);
+                line_fwd_t(mb[idx(i, j, 0)], mb[idx(i, j, 1)], mb[idx(i, j, 2)], vz, m2u, vz2, jzb);
     }
-    {
-        float X[27];  // input of the y pass = N after the x pass
-#pragma unroll
-        for (int i = 0; i < 27; ++i) X[i] = N[i];
-#pragma unroll
-        for (int j = 0; j < 3; ++j)
-#pragma unroll
-            for (int k = 0; k < 3; ++k) line_bwd(X[idx(0, j, k)], X[idx(1, j, k)], X[idx(2, j, k)], vx, kv(j) * kv(k));
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-#pragma unroll
-            for (int k = 0; k < 3; ++k)
-                line_bwd_rev(X[idx(i, 0, k)], X[idx(i, 1, k)], vy, kw(i) * kv(k), A[idx(i, 0, k)], A[idx(i, 1, k)],
-                             A[idx(i, 2, k)], vyb);
-    }
-#pragma unroll
-    for (int j = 0; j < 3; ++j)
-#pragma unroll
-        for (int k = 0; k < 3; ++k)
-            line_bwd_rev(N[idx(0, j, k)], N[idx(1, j, k)], vx, kv(j) * kv(k), A[idx(0, j, k)], A[idx(1, j, k)],
-                         A[idx(2, j, k)], vxb);
 }
 
 } // namespace adj
@@ -558,19 +612,14 @@ VF_HD void k17_vjp(const float (&f)[27], const float (&g)[27], const K17Rates& r
                    float vscale = 1.0f, float* sb = nullptr)
 {
     using namespace adj;
-    float p[27];
-#pragma unroll
-    for (int i = 0; i < 27; ++i) p[i] = f[dir_of_idx(i)];
-    Macro mc;
-    macro_of(p, r, vscale, mc);
-
-    // forward to the moments m, and the cumulant stage
     float m[27];
 #pragma unroll
-    for (int i = 0; i < 27; ++i) m[i] = p[i];
-    pass_z(m, mc.vz);
-    pass_y(m, mc.vy);
-    pass_x(m, mc.vx);
+    for (int i = 0; i < 27; ++i) m[i] = f[dir_of_idx(i)];
+    Macro mc;
+    macro_of(m, r, vscale, mc);
+
+    // forward to the moments m, and the cumulant stage
+    forward_moments(m, mc.vx, mc.vy, mc.vz);
     Mid s;
     float N[27];
     mid_forward(m, mc, r, s, N);
@@ -589,56 +638,20 @@ VF_HD void k17_vjp(const float (&f)[27], const float (&g)[27], const K17Rates& r
     vxb += 2.0f * mc.vx * vx2b;
     vyb += 2.0f * mc.vy * vy2b;
     vzb += 2.0f * mc.vz * vz2b;
+    forward_velocity_adjoint(s, mb, vxb, vyb, vzb);
 
-    // ---- reverse of the forward chimera (x, y, z) -------------------------------------------
-    // the x pass reads the y pass output, the y pass the z pass output
-    float Zo[27], Yo[27];
-#pragma unroll
-    for (int i = 0; i < 27; ++i) Zo[i] = p[i];
-    pass_z(Zo, mc.vz);
-#pragma unroll
-    for (int i = 0; i < 27; ++i) Yo[i] = Zo[i];
-    pass_y(Yo, mc.vy);
-#pragma unroll
-    for (int j = 0; j < 3; ++j)
-#pragma unroll
-        for (int k = 0; k < 3; ++k)
-            line_fwd_rev(Yo[idx(0, j, k)], Yo[idx(1, j, k)], Yo[idx(2, j, k)], mc.vx, kv(j) * kv(k), mb[idx(0, j, k)],
-                         mb[idx(1, j, k)], mb[idx(2, j, k)], vxb);
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int k = 0; k < 3; ++k)
-            line_fwd_rev(Zo[idx(i, 0, k)], Zo[idx(i, 1, k)], Zo[idx(i, 2, k)], mc.vy, kw(i) * kv(k), mb[idx(i, 0, k)],
-                         mb[idx(i, 1, k)], mb[idx(i, 2, k)], vyb);
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int j = 0; j < 3; ++j)
-            line_fwd_rev(p[idx(i, j, 0)], p[idx(i, j, 1)], p[idx(i, j, 2)], mc.vz, kw(i) * kw(j), mb[idx(i, j, 0)],
-                         mb[idx(i, j, 1)], mb[idx(i, j, 2)], vzb);
-
-    // ---- reverse of the macroscopic values ----------------------------------------------
+    // ---- reverse of the macroscopic values and the forward chimera --------------------------
     if (ub) {
         ub[0] = vxb;
         ub[1] = vyb;
         ub[2] = vzb;
     }
     const float rs = mc.R * vscale;
-    const float jxb = vxb * rs, jyb = vyb * rs, jzb = vzb * rs;
     const float vj = vxb * mc.jx + vyb * mc.jy + vzb * mc.jz;
     Rb += vscale * vj;
     if (sb) *sb = mc.R * vj;
     drhob += -Rb * mc.R * mc.R;
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            const float sb = drhob + float(i - 1) * jxb + float(j - 1) * jyb;
-            mb[idx(i, j, 0)] += sb - jzb;
-            mb[idx(i, j, 1)] += sb;
-            mb[idx(i, j, 2)] += sb + jzb;
-        }
+    forward_chimera_t(mb, mc.vx, mc.vy, mc.vz, drhob, vxb * rs, vyb * rs, vzb * rs);
 #pragma unroll
     for (int i = 0; i < 27; ++i) fb[dir_of_idx(i)] = mb[i];
 }
