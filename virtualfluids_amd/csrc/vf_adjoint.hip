@@ -24,24 +24,24 @@ namespace {
 
 constexpr int kAdjBlock = 256;
 
-template <class S, bool EVEN>
-__device__ __forceinline__ void adj_gather(const S* __restrict__ f, const float* __restrict__ lam, uint64_t N,
+// state v[d] and adjoint of the post-collision values g[inv(d)], both from the cell of pre[d]
+template <class S, bool EVEN, bool BUF>
+__device__ __forceinline__ void adj_gather(const SlotIO<S, BUF>& f, const SlotIO<float, BUF>& lam,
                                            const uint32_t (&n)[8], float (&v)[27], float (&g)[27])
 {
 #pragma unroll
     for (int d = 0; d < 27; ++d) {
-        const uint64_t cell = (uint64_t)slot<EVEN>(d) * N + n[node_sel(d)];
-        v[d] = Codec<S>::load(f + cell);
-        g[inv(d)] = lam[cell];
+        v[d] = f.load(slot<EVEN>(d), n[node_sel(d)] * (uint32_t)sizeof(S));
+        g[inv(d)] = lam.load(slot<EVEN>(d), n[node_sel(d)] * (uint32_t)sizeof(float));
     }
 }
 
-template <bool EVEN>
-__device__ __forceinline__ void adj_scatter(float* __restrict__ lam, uint64_t N, const uint32_t (&n)[8],
+template <bool EVEN, bool BUF>
+__device__ __forceinline__ void adj_scatter(const SlotIO<float, BUF>& lam, const uint32_t (&n)[8],
                                             const float (&fb)[27])
 {
 #pragma unroll
-    for (int d = 0; d < 27; ++d) lam[(uint64_t)slot<EVEN>(d) * N + n[node_sel(d)]] = fb[d];
+    for (int d = 0; d < 27; ++d) lam.store(slot<EVEN>(d), n[node_sel(d)] * (uint32_t)sizeof(float), fb[d]);
 }
 
 struct AdjBoxArgs {
@@ -92,7 +92,7 @@ __device__ __forceinline__ void brinkman_adjoint(const float* porosity, float* p
     if (porosity && porosityAdj) porosityAdj[k] += -0.5f * sb;
 }
 
-template <class S, bool EVEN, bool MASK, bool SHIFT, bool XCD = false>
+template <class S, bool EVEN, bool MASK, bool SHIFT, bool BUF, bool XCD = false>
 __global__ __launch_bounds__(kAdjBlock) void k17_adjoint_box_kernel(const S* __restrict__ f, float* __restrict__ lam,
                                                                     AdjBoxArgs a, K17Rates r)
 {
@@ -108,10 +108,12 @@ __global__ __launch_bounds__(kAdjBlock) void k17_adjoint_box_kernel(const S* __r
     const uint32_t n[8] = {row00 + x, row00 + xp, row10 + x, row10 + xp, row01 + x, row01 + xp, row11 + x, row11 + xp};
     if (MASK && a.mask[n[0]] == 0) return;
     float v[27], g[27], fb[27], ub[3], sb = 0.0f;
-    adj_gather<S, EVEN>(f, lam, a.N, n, v, g);
+    const SlotIO<S, BUF> fio(f, a.N);
+    const SlotIO<float, BUF> lio(lam, a.N);
+    adj_gather<S, EVEN, BUF>(fio, lio, n, v, g);
     const float vs = a.porosity ? 1.0f - 0.5f * a.porosity[n[0]] : 1.0f;
-    k17_vjp(v, g, r, fb, SHIFT ? ub : nullptr, vs, a.porosity ? &sb : nullptr);
-    adj_scatter<EVEN>(lam, a.N, n, fb);
+    k17_vjp(v, g, r, fb, SHIFT ? ub : nullptr, vs, &sb);
+    adj_scatter<EVEN, BUF>(lio, n, fb);
     if (SHIFT) {
         a.shiftAdj[n[0]] += ub[0];
         a.shiftAdj[a.N + n[0]] += ub[1];
@@ -257,7 +259,7 @@ __global__ __launch_bounds__(kAdjRowMaxThreads) void k17_adjoint_row_kernel(cons
     if (fluid) {
         float ub[3], sb = 0.0f;
         const float vs = a.porosity ? 1.0f - 0.5f * a.porosity[k] : 1.0f;
-        k17_vjp(v, g, r, fb, SHIFT ? ub : nullptr, vs, a.porosity ? &sb : nullptr);
+        k17_vjp(v, g, r, fb, SHIFT ? ub : nullptr, vs, &sb);
         if (SHIFT) {
             a.shiftAdj[k] += ub[0];
             a.shiftAdj[a.N + k] += ub[1];
@@ -345,10 +347,12 @@ __global__ __launch_bounds__(kAdjBlock) void k17_adjoint_indexed_kernel(const S*
     n[6] = a.nbz[n[2]];
     n[7] = a.nbz[n[3]];
     float v[27], g[27], fb[27], ub[3], sb = 0.0f;
-    adj_gather<S, EVEN>(f, lam, a.N, n, v, g);
+    const SlotIO<S, false> fio(f, a.N);
+    const SlotIO<float, false> lio(lam, a.N);
+    adj_gather<S, EVEN, false>(fio, lio, n, v, g);
     const float vs = a.porosity ? 1.0f - 0.5f * a.porosity[k] : 1.0f;
-    k17_vjp(v, g, r, fb, SHIFT ? ub : nullptr, vs, a.porosity ? &sb : nullptr);
-    adj_scatter<EVEN>(lam, a.N, n, fb);
+    k17_vjp(v, g, r, fb, SHIFT ? ub : nullptr, vs, &sb);
+    adj_scatter<EVEN, false>(lio, n, fb);
     if (SHIFT) {
         a.shiftAdj[k] += ub[0];
         a.shiftAdj[a.N + k] += ub[1];
@@ -388,17 +392,25 @@ void launch_row_b(const AdjBoxArgs& a, const K17Rates& r, const S* f, float* lam
     else hipLaunchKernelGGL((k17_adjoint_row_kernel<S, EVEN, false, false, BUF>), grid, block, 0, s, f, lam, a, r);
 }
 
+template <class S, bool EVEN, bool BUF>
+void launch_scalar_b(const AdjBoxArgs& a, const K17Rates& r, const S* f, float* lam, bool mask, bool shift, dim3 grid,
+                     hipStream_t s, bool xcd)
+{
+    const dim3 block(kAdjBlock);
+    if (xcd && mask && !shift) hipLaunchKernelGGL((k17_adjoint_box_kernel<S, EVEN, true, false, BUF, true>), grid, block, 0, s, f, lam, a, r);
+    else if (xcd && !mask && !shift) hipLaunchKernelGGL((k17_adjoint_box_kernel<S, EVEN, false, false, BUF, true>), grid, block, 0, s, f, lam, a, r);
+    else if (mask && shift) hipLaunchKernelGGL((k17_adjoint_box_kernel<S, EVEN, true, true, BUF>), grid, block, 0, s, f, lam, a, r);
+    else if (mask) hipLaunchKernelGGL((k17_adjoint_box_kernel<S, EVEN, true, false, BUF>), grid, block, 0, s, f, lam, a, r);
+    else if (shift) hipLaunchKernelGGL((k17_adjoint_box_kernel<S, EVEN, false, true, BUF>), grid, block, 0, s, f, lam, a, r);
+    else hipLaunchKernelGGL((k17_adjoint_box_kernel<S, EVEN, false, false, BUF>), grid, block, 0, s, f, lam, a, r);
+}
 template <class S, bool EVEN>
 void launch_scalar(const AdjBoxArgs& a, const K17Rates& r, const S* f, float* lam, bool mask, bool shift, dim3 grid,
                    hipStream_t s, bool xcd = false)
 {
-    const dim3 block(kAdjBlock);
-    if (xcd && mask && !shift) hipLaunchKernelGGL((k17_adjoint_box_kernel<S, EVEN, true, false, true>), grid, block, 0, s, f, lam, a, r);
-    else if (xcd && !mask && !shift) hipLaunchKernelGGL((k17_adjoint_box_kernel<S, EVEN, false, false, true>), grid, block, 0, s, f, lam, a, r);
-    else if (mask && shift) hipLaunchKernelGGL((k17_adjoint_box_kernel<S, EVEN, true, true>), grid, block, 0, s, f, lam, a, r);
-    else if (mask) hipLaunchKernelGGL((k17_adjoint_box_kernel<S, EVEN, true, false>), grid, block, 0, s, f, lam, a, r);
-    else if (shift) hipLaunchKernelGGL((k17_adjoint_box_kernel<S, EVEN, false, true>), grid, block, 0, s, f, lam, a, r);
-    else hipLaunchKernelGGL((k17_adjoint_box_kernel<S, EVEN, false, false>), grid, block, 0, s, f, lam, a, r);
+    // the buffer form needs kRowSplit slots of the adjoint (the larger element) within 32-bit offsets
+    if (slots_fit_buffers(a.N, sizeof(float))) launch_scalar_b<S, EVEN, true>(a, r, f, lam, mask, shift, grid, s, xcd);
+    else launch_scalar_b<S, EVEN, false>(a, r, f, lam, mask, shift, grid, s, xcd);
 }
 
 template <class S, bool EVEN>
@@ -409,11 +421,13 @@ void launch_box(const vf_lbm_parameter& p, float* lam, float* shift, float* padj
     const K17Rates r = make_k17_rates(p);
     const bool mask = p.fluidMask != nullptr;
     const S* f = static_cast<const S*>(p.distributions);
-    // A row is one workgroup of ceil(nx / 64) waves. At ~245 VGPRs a CU holds 8 waves of this
-    // kernel, so only rows of 1, 2, 4 or 8 whole waves fill it; those take the row kernel (256^3
-    // FP32: 0.99 against 1.09 ms). Every other width takes the scalar kernel, whose plane-flat
-    // workgroups keep every lane busy (258 x 130 x 130 FP16: 247 us, against 371 us for 256
-    // columns in the row kernel and a tail launch for the last two; measured on MI355X).
+    // A row is one workgroup of ceil(nx / 64) waves, and at ~135 VGPRs a CU holds 12 waves of this
+    // kernel: rows of 1 to 4 whole waves take the row kernel (256^3 FP32 920 against 1039 us in the
+    // scalar kernel, FP16 765 / 848; 192 x 192 x 128 FP32 279 / 306, 128^3 117 / 128). Longer rows
+    // leave too few workgroups to overlap loads and arithmetic (384 x 192 x 128 FP32 789 / 600, 512 x
+    // 128 x 128 630 / 529), and
+    // rows that are not whole waves idle lanes (258 x 130 x 130 FP16 524 / 250): those take the
+    // scalar kernel, whose plane-flat workgroups keep every lane busy.
     // kernelChoice.adjointKernel pins the scalar kernel, whole rows (ROW_WHOLE), or the row kernel
     // over the whole waves of any row with the scalar kernel on the columns beyond (ROW: a row
     // whose last wave would carry fewer than 32 lanes is split there, 258 = 256 + 2).
@@ -423,13 +437,13 @@ void launch_box(const vf_lbm_parameter& p, float* lam, float* shift, float* padj
     if (p.nx > 64 && p.nx % 64 != 0 && p.nx % 64 < 32 && kc.adjointKernel == VF_ADJOINT_KERNEL_ROW)
         rowEnd = p.nx - p.nx % 64;
     const int waves = (int)((rowEnd + 63) / 64);
-    const bool wholeWaves = p.nx % 64 == 0 && 8 % waves == 0;
+    const bool wholeWaves = p.nx % 64 == 0 && waves <= 4;
     if (rowEnd <= (uint32_t)kAdjRowMaxThreads && (wholeWaves || pinnedRow) && kc.adjointKernel != VF_ADJOINT_KERNEL_NODE) {
         // the buffer form needs kRowSplit slots of the adjoint (the larger element) within
         // 32-bit offsets
         AdjBoxArgs ar = a;
         ar.rowEnd = rowEnd;
-        if ((uint64_t)kRowSplit * a.N * sizeof(float) <= 0xffffffffull && kc.rowAddressing != VF_ROW_ADDRESSING_GLOBAL)
+        if (slots_fit_buffers(a.N, sizeof(float)) && kc.rowAddressing != VF_ROW_ADDRESSING_GLOBAL)
             launch_row_b<S, EVEN, true>(ar, r, f, lam, mask, shift != nullptr, s);
         else
             launch_row_b<S, EVEN, false>(ar, r, f, lam, mask, shift != nullptr, s);

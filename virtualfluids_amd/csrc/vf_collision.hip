@@ -25,24 +25,18 @@
 namespace vfa {
 
 // ---- device: gather / scatter over the 8 cell nodes -------------------------------------
-template <class S, bool EVEN>
-__device__ __forceinline__ void gather(const S* __restrict__ f, uint64_t N, const uint32_t (&n)[8], float (&v)[27])
+template <class S, bool EVEN, bool BUF>
+__device__ __forceinline__ void gather(const SlotIO<S, BUF>& f, const uint32_t (&n)[8], float (&v)[27])
 {
 #pragma unroll
-    for (int d = 0; d < 27; ++d) {
-        const char* base = reinterpret_cast<const char*>(f) + (uint64_t)slot<EVEN>(d) * N * sizeof(S);
-        v[d] = Codec<S>::load(reinterpret_cast<const S*>(base + n[node_sel(d)] * (uint32_t)sizeof(S)));
-    }
+    for (int d = 0; d < 27; ++d) v[d] = f.load(slot<EVEN>(d), n[node_sel(d)] * (uint32_t)sizeof(S));
 }
 
-template <class S, bool EVEN>
-__device__ __forceinline__ void scatter(S* __restrict__ f, uint64_t N, const uint32_t (&n)[8], const float (&v)[27])
+template <class S, bool EVEN, bool BUF>
+__device__ __forceinline__ void scatter(const SlotIO<S, BUF>& f, const uint32_t (&n)[8], const float (&v)[27])
 {
 #pragma unroll
-    for (int d = 0; d < 27; ++d) {
-        char* base = reinterpret_cast<char*>(f) + (uint64_t)slot<EVEN>(d) * N * sizeof(S);
-        Codec<S>::store(reinterpret_cast<S*>(base + n[node_sel(d)] * (uint32_t)sizeof(S)), v[inv(d)]);
-    }
+    for (int d = 0; d < 27; ++d) f.store(slot<EVEN>(d), n[node_sel(d)] * (uint32_t)sizeof(S), v[inv(d)]);
 }
 
 struct BoxArgs {
@@ -82,8 +76,8 @@ struct FusedBB {
 // from the stored values, list by list, writing the incoming population inv(d) of every wall
 // link d into the cell the next step reads (slot d with this step's parity, at the node of
 // inv(d)'s cell).
-template <class S, bool EVEN>
-__device__ __forceinline__ void bounce_back_epilogue(S* __restrict__ f, uint64_t N, const uint32_t (&n)[8],
+template <class S, bool EVEN, bool BUF>
+__device__ __forceinline__ void bounce_back_epilogue(const SlotIO<S, BUF>& f, const uint32_t (&n)[8],
                                                      const float (&v)[27], const FusedBB& bb)
 {
     const int32_t e = bb.nodeEntry[n[0]];
@@ -107,7 +101,7 @@ __device__ __forceinline__ void bounce_back_epilogue(S* __restrict__ f, uint64_t
         for (int d = 1; d < 27; ++d) {
             if (!(links >> d & 1u)) continue;
             const float val = velocity ? velocity_bounce_back(post[d], d, Ux, Uy, Uz) : post[d];
-            Codec<S>::store(f + (uint64_t)slot<EVEN>(d) * N + n[node_sel(inv(d))], val);
+            f.store(slot<EVEN>(d), n[node_sel(inv(d))] * (uint32_t)sizeof(S), val);
         }
     }
 }
@@ -132,7 +126,7 @@ template <bool XCD> __device__ __forceinline__ bool plane_node(const PlaneDiv& p
     return true;
 }
 
-template <class S, bool EVEN, bool MASK, bool MACRO, bool BB = false, bool XCD = false>
+template <class S, bool EVEN, bool BUF, bool MASK, bool MACRO, bool BB = false, bool XCD = false>
 __global__ __launch_bounds__(kBoxBlock) void k17_box_kernel(S* __restrict__ f, BoxArgs a, K17Rates r, FusedBB bb)
 {
     int x, y, z;
@@ -148,7 +142,8 @@ __global__ __launch_bounds__(kBoxBlock) void k17_box_kernel(S* __restrict__ f, B
     if (MASK && a.mask[n[0]] == 0) return;
 
     float v[27];
-    gather<S, EVEN>(f, a.N, n, v);
+    const SlotIO<S, BUF> io(f, a.N);
+    gather<S, EVEN, BUF>(io, n, v);
     MacroOut mo;
     k17_collide(v, r, mo, brinkman_scale(a.porosity, n[0]));
     if (MACRO) {
@@ -157,14 +152,14 @@ __global__ __launch_bounds__(kBoxBlock) void k17_box_kernel(S* __restrict__ f, B
         a.vy[n[0]] = mo.vy;
         a.vz[n[0]] = mo.vz;
     }
-    scatter<S, EVEN>(f, a.N, n, v);
-    if (BB) bounce_back_epilogue<S, EVEN>(f, a.N, n, v, bb);
+    scatter<S, EVEN, BUF>(io, n, v);
+    if (BB) bounce_back_epilogue<S, EVEN, BUF>(io, n, v, bb);
 }
 
 // Out-of-place variant: reads `in`, writes the stepped state to `out` (same layout). Masked
 // nodes copy their 27 cells unchanged, so `out` is the complete state the in-place step
 // would leave. Used to replay a segment of steps while keeping every intermediate state.
-template <class S, bool EVEN, bool MASK, bool XCD = false>
+template <class S, bool EVEN, bool BUF, bool MASK, bool XCD = false>
 __global__ __launch_bounds__(kBoxBlock) void k17_box_into_kernel(const S* __restrict__ in, S* __restrict__ out,
                                                                  BoxArgs a, K17Rates r)
 {
@@ -179,18 +174,19 @@ __global__ __launch_bounds__(kBoxBlock) void k17_box_into_kernel(const S* __rest
     const uint32_t row11 = (uint32_t)a.nx * ((uint32_t)yp + (uint32_t)a.ny * (uint32_t)zp);
     const uint32_t n[8] = {row00 + x, row00 + xp, row10 + x, row10 + xp, row01 + x, row01 + xp, row11 + x, row11 + xp};
     float v[27];
-    gather<S, EVEN>(in, a.N, n, v);
+    const SlotIO<S, BUF> src(in, a.N), dst(out, a.N);
+    gather<S, EVEN, BUF>(src, n, v);
     if (MASK && a.mask[n[0]] == 0) {
         // unchanged cells: value of pre(d) back into its own cell (scatter writes v[inv(d)])
         float w[27];
 #pragma unroll
         for (int d = 0; d < 27; ++d) w[inv(d)] = v[d];
-        scatter<S, EVEN>(out, a.N, n, w);
+        scatter<S, EVEN, BUF>(dst, n, w);
         return;
     }
     MacroOut mo;
     k17_collide(v, r, mo, brinkman_scale(a.porosity, n[0]));
-    scatter<S, EVEN>(out, a.N, n, v);
+    scatter<S, EVEN, BUF>(dst, n, v);
 }
 
 // ---- row kernel: one workgroup per x-row, V consecutive x-nodes per lane ----------------
@@ -399,7 +395,7 @@ struct IndexedArgs {
 
 constexpr int kIndexedBlock = 256;
 
-template <class S, bool EVEN, bool MACRO, bool BODYFORCE>
+template <class S, bool EVEN, bool BUF, bool MACRO, bool BODYFORCE>
 __global__ __launch_bounds__(kIndexedBlock) void k17_indexed_kernel(S* __restrict__ f, IndexedArgs a, K17Rates r)
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -426,7 +422,8 @@ __global__ __launch_bounds__(kIndexedBlock) void k17_indexed_kernel(S* __restric
         a.bfz[k] = 0.0f;
     }
     float v[27];
-    gather<S, EVEN>(f, a.N, n, v);
+    const SlotIO<S, BUF> io(f, a.N);
+    gather<S, EVEN, BUF>(io, n, v);
     MacroOut mo;
     k17_collide(v, rr, mo, brinkman_scale(a.porosity, k));
     if (MACRO) {
@@ -435,7 +432,7 @@ __global__ __launch_bounds__(kIndexedBlock) void k17_indexed_kernel(S* __restric
         a.vy[k] = mo.vy;
         a.vz[k] = mo.vz;
     }
-    scatter<S, EVEN>(f, a.N, n, v);
+    scatter<S, EVEN, BUF>(io, n, v);
 }
 
 // ---- host launchers ----------------------------------------------------------------------
@@ -503,7 +500,7 @@ static void launch_row_t(const BoxArgs& a, const K17Rates& r, bool mask, bool ma
                          const vf_kernel_choice& kc, hipStream_t s)
 {
     // the larger descriptor spans kRowSplit slots; buffer offsets are 32-bit
-    if ((uint64_t)kRowSplit * a.N * sizeof(S) <= 0xffffffffull && kc.rowAddressing != VF_ROW_ADDRESSING_GLOBAL)
+    if (slots_fit_buffers(a.N, sizeof(S)) && kc.rowAddressing != VF_ROW_ADDRESSING_GLOBAL)
         launch_row_b<S, V, EVEN, true>(a, r, mask, macro, f, out, ws, kc, s);
     else
         launch_row_b<S, V, EVEN, false>(a, r, mask, macro, f, out, ws, kc, s);
@@ -551,23 +548,58 @@ static bool try_launch_row(const vf_lbm_parameter& p, const BoxArgs& a, const K1
     return true;
 }
 
-// Whether the in-place node kernel takes its workgroups in XCD block ranges (xcd_block): where the
-// spans of a plane share cache lines at their ends (a plane is not a whole number of lines) the
-// ranges keep both sharers in one L2. Measured on MI355X, ranges against launch order, us per step:
-//   cache-resident   66^3 FP32 11.8 / 12.9, FP16 10.0 / 12.3; 130 x 70 x 70 FP32 23.2 / 26.5;
-//                    194 x 98 x 98 FP32 62.5 / 70.8, FP16 41.9 / 44.1; 258 x 130 x 130 FP16 91 / 98
-//   streaming FP32   258 x 130 x 130 190 / 206; 300 x 301 x 150 582 / 644; 251 x 187 x 133 285 / 285
-//   streaming 16-bit 251 x 187 x 133 186 / 158; 300 x 301 x 150 340 / 324; 333 x 200 x 290 495 / 456
-// A 16-bit span is half as long, so on a lattice larger than the cache eight distant regions cost
-// its streams more DRAM efficiency than the shared lines do: those keep the launch order. A level
-// that fits by itself inside a hierarchy that does not (258 x 130 x 130 FP16 in the two-level step)
-// takes the ranges: 315 us per coarse step against 319 in launch order.
-template <class S> static bool node_xcd_ranges(const vf_lbm_parameter& p)
+// Launch order and residency of the node kernels.
+//
+// XCD block ranges (xcd_block): where the spans of a plane share cache lines at their ends (a plane
+// is not a whole number of lines) the ranges keep both sharers in one L2. Beyond the cache they
+// also make eight distant regions of every stream, which costs DRAM efficiency: a 16-bit lattice
+// (its spans half as long) is better off in launch order, and so is an FP32 lattice of more
+// than twice the cache at two resident workgroups per CU. Measured on MI355X, us per step in
+// place, ranges against launch order, each at its best cap:
+//   cache-resident   66^3 FP32 11.8 / 12.9, FP16 10.0 / 12.3; 130 x 70 x 70 FP32 22.9 / 26.2;
+//                    194 x 98 x 98 FP32 63.0 / 68.6; 258 x 130 x 130 FP16 90 / 98
+//   streaming FP32   258 x 130 x 130 187 / 196; 251 x 187 x 133 280 / 271; 300 x 301 x 150 582 / 569;
+//                    333 x 200 x 290 855 / 805; 150 x 300 x 310 601 / 580
+//   streaming 16-bit 251 x 187 x 133 183 / 158; 300 x 301 x 150 332 / 327; 333 x 200 x 290 502 / 462
+// A 16-bit level that fits by itself inside a hierarchy that does not (258 x 130 x 130 FP16 in the
+// two-level step) takes the ranges: 315 us per coarse step against 319 in launch order.
+//
+// Resident workgroups per CU (0: as many as registers allow, eight): fewer concurrent spans per
+// stream serve HBM better, until the loads in flight no longer cover its latency. Eight against
+// the cap here: FP32 in place 258 x 130 x 130 192 -> 188 (4), 333 x 200 x 290 1006 -> 805 (2); out of
+// place 255 -> 198 (3, masked), 333 x 200 x 290 945 -> 900 (3); 16-bit in place 333 x 200 x 290 500 ->
+// 462 (4), out of place 542 -> 498 (4). Lattices of less than half the cache are latency-bound
+// (26 MB: 9.7 -> 10.7 at 4) and take every wave.
+struct NodeLaunch {
+    bool xcd;
+    size_t lds; // reserved at launch to impose the cap
+};
+template <class S> static NodeLaunch node_launch(const vf_lbm_parameter& p, bool into)
 {
+    const uint64_t own = 27 * p.numberOfNodes * sizeof(S);
     const int choice = p.kernelChoice.rowXcdRanges;
-    if (choice == 1 || choice == 2) return choice == 1;
-    return xcd_planes(p.nx, p.ny, sizeof(S), 0) &&
-           (sizeof(S) == 4 || 27 * p.numberOfNodes * sizeof(S) <= kCacheResidentBytes);
+    const bool ordered = !into && own > (sizeof(S) == 4 ? 2 * kCacheResidentBytes : kCacheResidentBytes);
+    const bool xcd = choice == 1 || choice == 2 ? choice == 1
+                                                : xcd_planes(p.nx, p.ny, sizeof(S), 0) && !ordered;
+    int cap = 0;
+    if (own > kCacheResidentBytes / 2) cap = sizeof(S) == 2 ? 4 : into ? 3 : xcd || own <= kCacheResidentBytes ? 4 : 2;
+    return {xcd, lds_reserve_for(cap)};
+}
+
+template <class S, bool EVEN, bool BUF>
+static void launch_node_b(const vf_lbm_parameter& p, const BoxArgs& a, const K17Rates& r, bool macro, hipStream_t s)
+{
+    S* f = static_cast<S*>(p.distributions);
+    const bool mask = p.fluidMask != nullptr;
+    const dim3 grid(plane_blocks(p.nx, p.ny), p.nz), bx(kBoxBlock);
+    const FusedBB none{};
+    const auto [xcd, lds] = node_launch<S>(p, false);
+    if (mask && macro) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, BUF, true, true>), grid, dim3(bx), lds, s, f, a, r, none);
+    else if (mask && xcd) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, BUF, true, false, false, true>), grid, dim3(bx), lds, s, f, a, r, none);
+    else if (mask) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, BUF, true, false>), grid, dim3(bx), lds, s, f, a, r, none);
+    else if (macro) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, BUF, false, true>), grid, dim3(bx), lds, s, f, a, r, none);
+    else if (xcd) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, BUF, false, false, false, true>), grid, dim3(bx), lds, s, f, a, r, none);
+    else hipLaunchKernelGGL((k17_box_kernel<S, EVEN, BUF, false, false>), grid, dim3(bx), lds, s, f, a, r, none);
 }
 
 template <class S, bool EVEN>
@@ -576,18 +608,24 @@ static void launch_box_t(const vf_lbm_parameter& p, bool macro, hipStream_t s)
     BoxArgs a{p.numberOfNodes, p.nx, p.ny, p.nz, p.fluidMask, p.rho, p.velocityX, p.velocityY, p.velocityZ,
               p.porosity, make_plane_div(p.nx, p.ny)};
     const K17Rates r = make_k17_rates(p);
+    if (try_launch_row<S, EVEN>(p, a, r, macro, nullptr, s)) return;
+    if (slots_fit_buffers(a.N, sizeof(S))) launch_node_b<S, EVEN, true>(p, a, r, macro, s);
+    else launch_node_b<S, EVEN, false>(p, a, r, macro, s);
+}
+
+template <class S, bool EVEN, bool BUF>
+static void launch_node_bb_b(const vf_lbm_parameter& p, const BoxArgs& a, const K17Rates& r, bool macro,
+                             const FusedBB& bb, hipStream_t s)
+{
     S* f = static_cast<S*>(p.distributions);
     const bool mask = p.fluidMask != nullptr;
-    if (try_launch_row<S, EVEN>(p, a, r, macro, nullptr, s)) return;
     const dim3 grid(plane_blocks(p.nx, p.ny), p.nz), bx(kBoxBlock);
-    const FusedBB none{};
-    const bool xcd = node_xcd_ranges<S>(p);
-    if (mask && macro) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, true, true>), grid, dim3(bx), 0, s, f, a, r, none);
-    else if (mask && xcd) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, true, false, false, true>), grid, dim3(bx), 0, s, f, a, r, none);
-    else if (mask) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, true, false>), grid, dim3(bx), 0, s, f, a, r, none);
-    else if (macro) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, false, true>), grid, dim3(bx), 0, s, f, a, r, none);
-    else if (xcd) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, false, false, false, true>), grid, dim3(bx), 0, s, f, a, r, none);
-    else hipLaunchKernelGGL((k17_box_kernel<S, EVEN, false, false>), grid, dim3(bx), 0, s, f, a, r, none);
+    const auto [xcd, lds] = node_launch<S>(p, false);
+    if (mask && macro) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, BUF, true, true, true>), grid, dim3(bx), lds, s, f, a, r, bb);
+    else if (mask && xcd) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, BUF, true, false, true, true>), grid, dim3(bx), lds, s, f, a, r, bb);
+    else if (mask) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, BUF, true, false, true>), grid, dim3(bx), lds, s, f, a, r, bb);
+    else if (macro) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, BUF, false, true, true>), grid, dim3(bx), lds, s, f, a, r, bb);
+    else hipLaunchKernelGGL((k17_box_kernel<S, EVEN, BUF, false, false, true>), grid, dim3(bx), lds, s, f, a, r, bb);
 }
 
 // The node kernel with the bounce-back epilogue. Returns false where the dense-box collision
@@ -599,20 +637,13 @@ static bool launch_box_bb_t(const vf_lbm_parameter& p, bool macro, const FusedBB
     BoxArgs a{p.numberOfNodes, p.nx, p.ny, p.nz, p.fluidMask, p.rho, p.velocityX, p.velocityY, p.velocityZ,
               p.porosity, make_plane_div(p.nx, p.ny)};
     const K17Rates r = make_k17_rates(p);
-    S* f = static_cast<S*>(p.distributions);
-    const bool mask = p.fluidMask != nullptr;
-    const dim3 grid(plane_blocks(p.nx, p.ny), p.nz), bx(kBoxBlock);
-    const bool xcd = node_xcd_ranges<S>(p);
-    if (mask && macro) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, true, true, true>), grid, dim3(bx), 0, s, f, a, r, bb);
-    else if (mask && xcd) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, true, false, true, true>), grid, dim3(bx), 0, s, f, a, r, bb);
-    else if (mask) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, true, false, true>), grid, dim3(bx), 0, s, f, a, r, bb);
-    else if (macro) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, false, true, true>), grid, dim3(bx), 0, s, f, a, r, bb);
-    else hipLaunchKernelGGL((k17_box_kernel<S, EVEN, false, false, true>), grid, dim3(bx), 0, s, f, a, r, bb);
+    if (slots_fit_buffers(a.N, sizeof(S))) launch_node_bb_b<S, EVEN, true>(p, a, r, macro, bb, s);
+    else launch_node_bb_b<S, EVEN, false>(p, a, r, macro, bb, s);
     return true;
 }
 
-template <class S, bool EVEN>
-static void launch_indexed_t(const vf_lbm_parameter& p, const uint32_t* idx, uint32_t n, bool macro, bool force,
+template <class S, bool EVEN, bool BUF>
+static void launch_indexed_b(const vf_lbm_parameter& p, const uint32_t* idx, uint32_t n, bool macro, bool force,
                              hipStream_t s)
 {
     IndexedArgs a{p.numberOfNodes, p.neighborX, p.neighborY, p.neighborZ, idx, n,
@@ -621,10 +652,17 @@ static void launch_indexed_t(const vf_lbm_parameter& p, const uint32_t* idx, uin
     const K17Rates r = make_k17_rates(p);
     dim3 grid((n + kIndexedBlock - 1) / kIndexedBlock);
     S* f = static_cast<S*>(p.distributions);
-    if (macro && force) hipLaunchKernelGGL((k17_indexed_kernel<S, EVEN, true, true>), grid, dim3(kIndexedBlock), 0, s, f, a, r);
-    else if (macro) hipLaunchKernelGGL((k17_indexed_kernel<S, EVEN, true, false>), grid, dim3(kIndexedBlock), 0, s, f, a, r);
-    else if (force) hipLaunchKernelGGL((k17_indexed_kernel<S, EVEN, false, true>), grid, dim3(kIndexedBlock), 0, s, f, a, r);
-    else hipLaunchKernelGGL((k17_indexed_kernel<S, EVEN, false, false>), grid, dim3(kIndexedBlock), 0, s, f, a, r);
+    if (macro && force) hipLaunchKernelGGL((k17_indexed_kernel<S, EVEN, BUF, true, true>), grid, dim3(kIndexedBlock), 0, s, f, a, r);
+    else if (macro) hipLaunchKernelGGL((k17_indexed_kernel<S, EVEN, BUF, true, false>), grid, dim3(kIndexedBlock), 0, s, f, a, r);
+    else if (force) hipLaunchKernelGGL((k17_indexed_kernel<S, EVEN, BUF, false, true>), grid, dim3(kIndexedBlock), 0, s, f, a, r);
+    else hipLaunchKernelGGL((k17_indexed_kernel<S, EVEN, BUF, false, false>), grid, dim3(kIndexedBlock), 0, s, f, a, r);
+}
+template <class S, bool EVEN>
+static void launch_indexed_t(const vf_lbm_parameter& p, const uint32_t* idx, uint32_t n, bool macro, bool force,
+                             hipStream_t s)
+{
+    if (slots_fit_buffers(p.numberOfNodes, sizeof(S))) launch_indexed_b<S, EVEN, true>(p, idx, n, macro, force, s);
+    else launch_indexed_b<S, EVEN, false>(p, idx, n, macro, force, s);
 }
 
 template <template <class, bool> class L, class... A>
@@ -650,6 +688,21 @@ static int dispatch_storage(const vf_lbm_parameter& p, A&&... args)
 template <class S, bool EVEN> struct BoxL {
     static void run(const vf_lbm_parameter& p, bool macro, hipStream_t s) { launch_box_t<S, EVEN>(p, macro, s); }
 };
+template <class S, bool EVEN, bool BUF>
+static void launch_into_b(const vf_lbm_parameter& p, const BoxArgs& a, const K17Rates& r, S* out, hipStream_t s)
+{
+    const dim3 grid(plane_blocks(p.nx, p.ny), p.nz), bx(kBoxBlock);
+    const S* in = static_cast<const S*>(p.distributions);
+    const auto [xcd, lds] = node_launch<S>(p, true);
+    if (p.fluidMask && xcd)
+        hipLaunchKernelGGL((k17_box_into_kernel<S, EVEN, BUF, true, true>), grid, dim3(bx), lds, s, in, out, a, r);
+    else if (p.fluidMask)
+        hipLaunchKernelGGL((k17_box_into_kernel<S, EVEN, BUF, true>), grid, dim3(bx), lds, s, in, out, a, r);
+    else if (xcd)
+        hipLaunchKernelGGL((k17_box_into_kernel<S, EVEN, BUF, false, true>), grid, dim3(bx), lds, s, in, out, a, r);
+    else
+        hipLaunchKernelGGL((k17_box_into_kernel<S, EVEN, BUF, false>), grid, dim3(bx), lds, s, in, out, a, r);
+}
 template <class S, bool EVEN> struct BoxIntoL {
     static void run(const vf_lbm_parameter& p, void* out, hipStream_t s)
     {
@@ -657,17 +710,8 @@ template <class S, bool EVEN> struct BoxIntoL {
                   make_plane_div(p.nx, p.ny)};
         const K17Rates r = make_k17_rates(p);
         if (try_launch_row<S, EVEN>(p, a, r, false, static_cast<S*>(out), s)) return;
-        const dim3 grid(plane_blocks(p.nx, p.ny), p.nz), bx(kBoxBlock);
-        const S* in = static_cast<const S*>(p.distributions);
-        const bool xcd = xcd_planes(p.nx, p.ny, sizeof(S), p.kernelChoice.rowXcdRanges);
-        if (p.fluidMask && xcd)
-            hipLaunchKernelGGL((k17_box_into_kernel<S, EVEN, true, true>), grid, dim3(bx), 0, s, in, (S*)out, a, r);
-        else if (p.fluidMask)
-            hipLaunchKernelGGL((k17_box_into_kernel<S, EVEN, true>), grid, dim3(bx), 0, s, in, (S*)out, a, r);
-        else if (xcd)
-            hipLaunchKernelGGL((k17_box_into_kernel<S, EVEN, false, true>), grid, dim3(bx), 0, s, in, (S*)out, a, r);
-        else
-            hipLaunchKernelGGL((k17_box_into_kernel<S, EVEN, false>), grid, dim3(bx), 0, s, in, (S*)out, a, r);
+        if (slots_fit_buffers(a.N, sizeof(S))) launch_into_b<S, EVEN, true>(p, a, r, static_cast<S*>(out), s);
+        else launch_into_b<S, EVEN, false>(p, a, r, static_cast<S*>(out), s);
     }
 };
 template <class S, bool EVEN> struct IndexedL {

@@ -28,6 +28,66 @@ __host__ __device__ constexpr int shifted_index(int d)
 // slots span less than 4 GiB.
 constexpr int kRowSplit = 14;
 
+// host: whether kRowSplit slots of N elements of elemBytes lie within 32-bit buffer offsets
+inline bool slots_fit_buffers(uint64_t N, size_t elemBytes) { return kRowSplit * N * elemBytes <= 0xffffffffull; }
+
+// The population slots of a one-node-per-thread kernel: load / store of one element of slot `sl`
+// at byte offset `off` of the slot. BUF: through the two buffer descriptors above, whose address
+// is descriptor + scalar slot offset + 32-bit lane offset; the global form (lattices beyond
+// slots_fit_buffers) keeps a 64-bit address per direction in vector registers between the load and
+// the store (28 64-bit adds and 54 registers a node: the adjoint 1330 -> 1194 vector operations
+// and 147 -> 137 registers with the buffers, the collision 692 -> 657, with the bounce-back epilogue
+// 1275 -> 1098: 64^3 cavity 16.8 -> 14.0 us a step).
+template <class S, bool BUF> struct SlotIO {
+    S* f;
+    uint64_t slotBytes;
+    __amdgpu_buffer_rsrc_t lo, hi;
+
+    __device__ __forceinline__ SlotIO(const S* f_, uint64_t N) : f(const_cast<S*>(f_)), slotBytes(N * sizeof(S))
+    {
+        if constexpr (BUF) {
+            lo = __builtin_amdgcn_make_buffer_rsrc(f, (short)0, (int)0xffffffff, 0x00020000);
+            hi = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<char*>(f) + kRowSplit * slotBytes, (short)0,
+                                                   (int)0xffffffff, 0x00020000);
+        }
+    }
+    __device__ __forceinline__ uint32_t soff(int sl) const
+    {
+        return (uint32_t)(sl >= kRowSplit ? sl - kRowSplit : sl) * (uint32_t)slotBytes;
+    }
+    __device__ __forceinline__ S* at(int sl, uint32_t off) const
+    {
+        return reinterpret_cast<S*>(reinterpret_cast<char*>(f) + (uint64_t)sl * slotBytes + off);
+    }
+    __device__ __forceinline__ float load(int sl, uint32_t off) const
+    {
+        if constexpr (BUF) {
+            if constexpr (sizeof(S) == 4)
+                return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(sl >= kRowSplit ? hi : lo, off, soff(sl), 0));
+            else {
+                const unsigned short w = __builtin_amdgcn_raw_buffer_load_b16(sl >= kRowSplit ? hi : lo, off, soff(sl), 0);
+                return Codec<S>::load(reinterpret_cast<const S*>(&w));
+            }
+        } else {
+            return Codec<S>::load(at(sl, off));
+        }
+    }
+    __device__ __forceinline__ void store(int sl, uint32_t off, float v) const
+    {
+        if constexpr (BUF) {
+            if constexpr (sizeof(S) == 4)
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), sl >= kRowSplit ? hi : lo, off, soff(sl), 0);
+            else {
+                unsigned short w;
+                Codec<S>::store(reinterpret_cast<S*>(&w), v);
+                __builtin_amdgcn_raw_buffer_store_b16(w, sl >= kRowSplit ? hi : lo, off, soff(sl), 0);
+            }
+        } else {
+            Codec<S>::store(at(sl, off), v);
+        }
+    }
+};
+
 // Workgroup b of a launch runs on XCD b % 8; each of the eight XCDs has its own L2. With
 // xcd_block the XCDs take contiguous ranges of R blocks instead (XCD j: [j q + min(j, R % 8),
 // ...) with q = R / 8), so that neighbouring rows meet in one L2. Rows whose bytes are not a
@@ -48,10 +108,9 @@ inline uint32_t xcd_rows(int nx, size_t elemBytes, int choice)
     return ((size_t)nx * elemBytes) % 128 != 0;
 }
 
-// host: the same for the plane-flat out-of-place kernel, whose workgroups take consecutive spans
-// of a plane: spans share their end lines with the next one where a plane's bytes are not a
-// whole number of lines (on MI355X, 258 x 130 x 130 FP16 out of place 140 -> 125 us alone and
-// 121-130 -> 118 us inside the two-level step; the sphere channel's 194 x 98 x 98 FP32 92 -> 87)
+// host: the same for the plane-flat node kernels, whose workgroups take consecutive spans of a
+// plane: spans share their end lines with the next one where a plane's bytes are not a whole number
+// of lines
 inline uint32_t xcd_planes(int nx, int ny, size_t elemBytes, int choice)
 {
     if (choice == 1 || choice == 2) return choice == 1;
