@@ -71,6 +71,32 @@ struct FusedBB {
     const float* vz[3];
 };
 
+// The bounce-back links of this thread's node, list by list. The table loads are issued before the
+// collision, which hides them: issued after the scatter they cost a node with wall links three
+// memory latencies in a row at the end of its wave (entry, links, list index).
+struct NodeLinks {
+    uint32_t links[3];
+    float U[3][3]; // wall velocity of each list (velocity lists only)
+};
+__device__ __forceinline__ NodeLinks node_links(const FusedBB& bb, int32_t e)
+{
+    NodeLinks n{};
+    if (e >= 0) {
+#pragma unroll
+        for (int l = 0; l < 3; ++l) n.links[l] = bb.entryLinks[3 * e + l];
+#pragma unroll
+        for (int l = 0; l < 3; ++l) {
+            if (!bb.vx[l]) continue;
+            const int32_t i = bb.entryIndex[3 * e + l];
+            if (i < 0) continue;
+            n.U[l][0] = bb.vx[l][i];
+            n.U[l][1] = bb.vy[l][i];
+            n.U[l][2] = bb.vz[l][i];
+        }
+    }
+    return n;
+}
+
 // The post-collision bounce-back of one node, from its post-collision values v (as the
 // collision left them in registers): exactly what NoSlipBounceBack / VelocityBounceBack compute
 // from the stored values, list by list, writing the incoming population inv(d) of every wall
@@ -78,29 +104,21 @@ struct FusedBB {
 // inv(d)'s cell).
 template <class S, bool EVEN, bool BUF>
 __device__ __forceinline__ void bounce_back_epilogue(const SlotIO<S, BUF>& f, const uint32_t (&n)[8],
-                                                     const float (&v)[27], const FusedBB& bb)
+                                                     const float (&v)[27], const FusedBB& bb, const NodeLinks& nl)
 {
-    const int32_t e = bb.nodeEntry[n[0]];
-    if (e < 0) return;
+    if (!(nl.links[0] | nl.links[1] | nl.links[2])) return;
     float post[27];
 #pragma unroll
     for (int d = 0; d < 27; ++d) post[d] = Codec<S>::round(v[d]); // the stored post-collision values
 #pragma unroll
     for (int l = 0; l < 3; ++l) {
-        const uint32_t links = bb.entryLinks[3 * e + l];
+        const uint32_t links = nl.links[l];
         if (!links) continue;
-        float Ux = 0.0f, Uy = 0.0f, Uz = 0.0f;
         const bool velocity = bb.vx[l] != nullptr;
-        if (velocity) {
-            const int32_t i = bb.entryIndex[3 * e + l];
-            Ux = bb.vx[l][i];
-            Uy = bb.vy[l][i];
-            Uz = bb.vz[l][i];
-        }
 #pragma unroll
         for (int d = 1; d < 27; ++d) {
             if (!(links >> d & 1u)) continue;
-            const float val = velocity ? velocity_bounce_back(post[d], d, Ux, Uy, Uz) : post[d];
+            const float val = velocity ? velocity_bounce_back(post[d], d, nl.U[l][0], nl.U[l][1], nl.U[l][2]) : post[d];
             f.store(slot<EVEN>(d), n[node_sel(inv(d))] * (uint32_t)sizeof(S), val);
         }
     }
@@ -139,11 +157,15 @@ __global__ __launch_bounds__(kBoxBlock) void k17_box_kernel(S* __restrict__ f, B
     const uint32_t row01 = (uint32_t)a.nx * ((uint32_t)y + (uint32_t)a.ny * (uint32_t)zp);
     const uint32_t row11 = (uint32_t)a.nx * ((uint32_t)yp + (uint32_t)a.ny * (uint32_t)zp);
     const uint32_t n[8] = {row00 + x, row00 + xp, row10 + x, row10 + xp, row01 + x, row01 + xp, row11 + x, row11 + xp};
+    int32_t entry = -1;
+    if (BB) entry = bb.nodeEntry[n[0]];
     if (MASK && a.mask[n[0]] == 0) return;
 
     float v[27];
     const SlotIO<S, BUF> io(f, a.N);
     gather<S, EVEN, BUF>(io, n, v);
+    NodeLinks links{};
+    if (BB) links = node_links(bb, entry);
     MacroOut mo;
     k17_collide(v, r, mo, brinkman_scale(a.porosity, n[0]));
     if (MACRO) {
@@ -153,7 +175,7 @@ __global__ __launch_bounds__(kBoxBlock) void k17_box_kernel(S* __restrict__ f, B
         a.vz[n[0]] = mo.vz;
     }
     scatter<S, EVEN, BUF>(io, n, v);
-    if (BB) bounce_back_epilogue<S, EVEN, BUF>(io, n, v, bb);
+    if (BB) bounce_back_epilogue<S, EVEN, BUF>(io, n, v, bb, links);
 }
 
 // Out-of-place variant: reads `in`, writes the stepped state to `out` (same layout). Masked
