@@ -478,6 +478,41 @@ int vf_DragLiftSum(const vf_lbm_parameter* para, const vf_q_boundary_conditions*
  * overwritten. */
 int vf_KineticEnergy(const vf_lbm_parameter* para, const uint32_t* neighborInverse, double* out2, void* stream);
 
+/* ---------------------------------------------------------------------------------
+ * Sequences of launches (no counterpart in the reference: its time loop calls the launchers one by
+ * one). vf_run_launches enqueues the n entries of `list` in order, `repeats` times, on one stream:
+ * what calling the entry points one by one does, without a caller's round trip per launch (on
+ * MI355X about 2.6 us of host time a launch, below the shortest kernels of a step). It returns the
+ * first error of an entry (the entries before it are enqueued), and changes no state but the
+ * parities its VF_LAUNCH_SWAP entries flip.
+ * --------------------------------------------------------------------------------- */
+enum vf_launch_kind {
+    VF_LAUNCH_BOX = 0,             /* vf_k17_run_box(level, collisionTemplate) */
+    VF_LAUNCH_BOX_BOUNCE_BACK = 1, /* vf_k17_run_box_bounce_back(level, collisionTemplate, bounceBack) */
+    VF_LAUNCH_INDICES = 2,         /* vf_k17_run_on_indices over the level's fluid nodes, collisionTemplate */
+    VF_LAUNCH_BC = 3,              /* bc(level, list) */
+    VF_LAUNCH_SWAP = 4,            /* flips level->isEvenTimestep (no launch) */
+    VF_LAUNCH_COARSE_TO_FINE = 5,  /* vf_ScaleCoarseToFineCompressible(level, fine, cells, offsets) */
+    VF_LAUNCH_FINE_TO_COARSE = 6   /* vf_ScaleFineToCoarseCompressible(level, fine, cells, offsets) */
+};
+/* The launchers of one boundary-condition list */
+typedef int (*vf_bc_launcher)(const vf_lbm_parameter* para, const vf_q_boundary_conditions* bc, void* stream);
+/* All pointers are host pointers, read when the sequence runs; fields a kind does not use are
+ * ignored. */
+typedef struct vf_launch {
+    int32_t kind;              /* enum vf_launch_kind */
+    int32_t collisionTemplate; /* collisions */
+    vf_lbm_parameter* level;   /* the coarse level for the scaling kinds */
+    const vf_lbm_parameter* fine;
+    vf_bc_launcher bc;
+    const vf_q_boundary_conditions* list;
+    const vf_post_bounce_back* bounceBack;
+    const vf_interpolation_cells* cells;
+    const vf_interpolation_cell_neighbor* offsets; /* or NULL */
+} vf_launch;
+
+int vf_run_launches(const vf_launch* list, uint32_t n, uint32_t repeats, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

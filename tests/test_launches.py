@@ -1,0 +1,108 @@
+"""Sequences of launches (vf_run_launches): argument checks on the CPU, and on the GPU the same
+fields as launching every kernel from Python for short and long runs, both parities, a given
+stream, a lattice changed between runs and a run inside a captured graph."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from virtualfluids_amd import capi
+from virtualfluids_amd.grid import cavity, channel
+
+
+def test_bad_entries_are_rejected_before_anything_runs():
+    lib = capi.load()
+    p = capi.LBMParameter()
+    p.isEvenTimestep = 1
+    good = capi.Launch(kind=capi.LAUNCH_SWAP, level=ctypes.pointer(p))
+    for bad in (capi.Launch(kind=7, level=ctypes.pointer(p)), capi.Launch(kind=-1, level=ctypes.pointer(p)),
+                capi.Launch(kind=capi.LAUNCH_SWAP), capi.Launch(kind=capi.LAUNCH_BC, level=ctypes.pointer(p)),
+                capi.Launch(kind=capi.LAUNCH_COARSE_TO_FINE, level=ctypes.pointer(p))):
+        arr = (capi.Launch * 2)(good, bad)
+        assert lib.vf_run_launches(arr, 2, 1, None) == capi.VF_ERR_INVALID_ARGUMENT
+        assert p.isEvenTimestep == 1
+    assert lib.vf_run_launches(None, 1, 1, None) == capi.VF_ERR_INVALID_ARGUMENT
+    assert lib.vf_run_launches(None, 0, 1, None) == capi.VF_OK
+    # an entry's own error stops the sequence: its collision has no populations
+    arr = (capi.Launch * 2)(capi.Launch(kind=capi.LAUNCH_BOX, level=ctypes.pointer(p)), good)
+    assert lib.vf_run_launches(arr, 2, 3, None) == capi.VF_ERR_INVALID_ARGUMENT
+    assert p.isEvenTimestep == 1
+    assert lib.vf_run_launches((capi.Launch * 1)(good), 1, 3, None) == capi.VF_OK
+    assert p.isEvenTimestep == 0
+
+
+def _factory(bounce_back):
+    from virtualfluids_amd.simulation import BoundaryConditionFactory as F
+
+    fac = F()
+    if bounce_back:
+        fac.set_velocity_boundary_condition(F.VelocityBC.VelocityBounceBack)
+        fac.set_no_slip_boundary_condition(F.NoSlipBC.NoSlipBounceBack)
+    else:
+        fac.set_velocity_boundary_condition(F.VelocityBC.VelocityInterpolatedCompressible)
+        fac.set_no_slip_boundary_condition(F.NoSlipBC.NoSlipInterpolatedCompressible)
+        fac.set_pressure_boundary_condition(F.PressureBC.PressureNonEquilibriumCompressible)
+    return fac
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bounce_back,box", [(True, True), (False, True), (False, False)])
+def test_runs_match_host_launches(gpu, bounce_back, box):
+    import torch
+
+    from virtualfluids_amd.lattice import Lattice
+    from virtualfluids_amd.simulation import Simulation
+
+    sims = []
+    for _ in range(2):
+        g = cavity(9) if bounce_back else channel((17, 9, 7), inflow=0.03)
+        L = Lattice(g, 1.7, box=box)
+        z = np.zeros(g.N)
+        L.init_equilibrium(z, np.where(g.geo == 19, 0.02, 0.0), z, z)
+        sims.append(Simulation(L, _factory(bounce_back)))
+    a, b = sims
+    stream = torch.cuda.Stream()
+    phi = torch.linspace(0.0, 0.05, a.lattice.N, device="cuda")
+    for i, n in enumerate((1, 2, 3, 16, 37, 0)):
+        if i == 4:  # the lattice changes between runs
+            a.lattice.set_porosity(phi)
+            b.lattice.set_porosity(phi)
+        if i == 3:
+            stream.wait_stream(torch.cuda.current_stream())
+            a.run(n, stream=stream)
+            torch.cuda.current_stream().wait_stream(stream)
+        else:
+            a.run(n)
+        b.run(n, graphs=False)
+        assert a.lattice.even == b.lattice.even and a.t == b.t
+        assert torch.equal(a.lattice.f, b.lattice.f), f"after {n} steps"
+
+
+@pytest.mark.gpu
+def test_run_inside_a_captured_graph(gpu):
+    import torch
+
+    from virtualfluids_amd.graphs import capture
+    from virtualfluids_amd.lattice import Lattice
+    from virtualfluids_amd.launches import LaunchList
+    from virtualfluids_amd.simulation import Simulation
+
+    sims = []
+    for _ in range(2):
+        g = channel((17, 9, 7), inflow=0.03)
+        L = Lattice(g, 1.7)
+        z = np.zeros(g.N)
+        L.init_equilibrium(z, np.where(g.geo == 19, 0.02, 0.0), z, z)
+        sims.append(Simulation(L, _factory(False)))
+    a, b = sims
+    a.run(2)
+    b.run(2)
+    steps = LaunchList()
+    a.add_launches(steps)
+    graph = capture(lambda st: steps.run(4, st), torch.cuda.Stream())
+    for i in range(3):
+        graph.replay()
+        b.run(4, graphs=False)
+        assert torch.equal(a.lattice.f, b.lattice.f), f"replay {i}"
+        _ = b.lattice.f.float().sum().item()
+    torch.cuda.synchronize()

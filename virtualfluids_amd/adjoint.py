@@ -6,8 +6,8 @@ UpdateGrid27 (collision, velocity BC, no-slip BC, geometry BC, parity swap, pres
 src/gpu/core/Calculation/UpdateGrid27.cpp:54-96) and returns the final buffer. Its backward
 sweeps the steps in reverse with the adjoint kernels (vf_k17_adjoint[_box] and the BC
 adjoints): pressure BC, then geometry, no-slip and velocity, then the collision. The forward keeps a
-copy of the buffer every `checkpoint_every` steps and steps in place, replaying one HIP graph
-per parity; the backward replays one segment at a time from its checkpoint (out of place on
+copy of the buffer every `checkpoint_every` steps and steps in place, the launches enqueued
+natively; the backward replays one segment at a time from its checkpoint (out of place on
 the dense box, so the replay writes each intermediate state once and copies nothing) and walks
 the segment backwards. Memory: steps/K + K + 1
 buffers of the storage type. Gradients flow to f0 and, when given, to the wall velocities of
@@ -28,8 +28,8 @@ import torch
 
 from . import capi
 from .grid import CX, CY, CZ, INV
-from .graphs import StepGraphs as _StepGraphs
 from .lattice import Lattice, stream_handle
+from .launches import LaunchList, StepLaunches
 from .simulation import BoundaryConditionFactory
 
 
@@ -151,6 +151,17 @@ class Stepper:
             capi.call(self.pressure, ctypes.byref(_param(L, target, not even)), ctypes.byref(bc.struct), s)
         return target
 
+    def add_launches(self, out: LaunchList, param):
+        """Append the launches of forward(buf, even, None, ...) to `out`: param is a struct of the
+        level (_param) on that buffer, whose parity the list swaps."""
+        out.collide(param, self.L.box)
+        for _, fn, bc in self._groups():
+            out.bc(param, fn, bc.struct)
+        out.swap(param)
+        bc = self._bc("pressure")
+        if self.pressure and bc is not None:
+            out.bc(param, self.pressure, bc.struct)
+
     def adjoint(self, before: torch.Tensor, after: torch.Tensor, lam: torch.Tensor, even: bool, ubar, rbar, padj,
                 stream, saved=None):
         """Reverse of one step: `before`/`after` are the states around it, `even` its parity;
@@ -189,7 +200,11 @@ class _K17Steps(torch.autograd.Function):
         # the values this forward used: the backward replays with them, whatever the lattice
         # holds by then (another segment or objective may have set its own)
         ctx.params = _bc_snapshot(L)
-        run = _StepGraphs(lambda ev, st: stepper.forward(buf, ev, None, st), graphs)
+        launches = None
+        if graphs:
+            launches = LaunchList(), _param(L, buf, even0)
+            stepper.add_launches(*launches)
+        run = StepLaunches(lambda ev, st: stepper.forward(buf, ev, None, st), launches)
         checkpoints = []
         # the trailing segments whose states fit keep_bytes are stepped out of place and kept, so
         # the backward walks them without a replay
@@ -235,7 +250,6 @@ class _K17Steps(torch.autograd.Function):
                     (observe_from - i) if observe is not None else steps)
             even = run.run(n, even)
             i += n
-        run.close()
         ctx.stepper, ctx.steps, ctx.K = stepper, steps, checkpoint_every
         ctx.checkpoints = checkpoints
         ctx.kept = kept
@@ -311,8 +325,8 @@ def k17_steps(f0: torch.Tensor, lattice: Lattice, steps: int, checkpoint_every: 
 
     The lattice's own buffer and parity are not touched (its BC parameter arrays take the given
     values); `even` is the parity of the first step (default: the lattice's current parity).
-    graphs: the forward sweep replays HIP graphs of the steps (False: every launch from the
-    host; the results are the same bit for bit).
+    graphs: the library enqueues the forward sweep's launches itself (False: every launch from
+    Python; the results are the same bit for bit).
     observe(buf, even) -> scalar tensor, a differentiable function of the buffer and its parity
     (KineticEnergyObservation, or any torch function such as a momentum-exchange drag), is
     summed over the states after steps observe_from .. steps-1; then the call returns (buffer,
@@ -365,7 +379,8 @@ class _TwoLevelSteps(torch.autograd.Function):
         if por_f is not None:
             Lf.set_porosity(por_f.detach())
         ctx.params = (_bc_snapshot(Lc), _bc_snapshot(Lf))
-        run = _StepGraphs(lambda ev, st: _two_level_step_in_place(sc, sf, cells, C, F, ev, st), graphs)
+        run = StepLaunches(lambda ev, st: _two_level_step_in_place(sc, sf, cells, C, F, ev, st),
+                           _level_launches([sc, sf], [cells], [C, F], even0) if graphs else None)
         checkpoints = []
         # the trailing segments whose states fit keep_bytes are stepped out of place and kept, so
         # the backward walks them without a replay (the states of a coarse step: two fine
@@ -418,7 +433,6 @@ class _TwoLevelSteps(torch.autograd.Function):
             n = min(K - i % K, steps - i, (observe_from - i) if observe is not None else steps)
             even = run.run(n, even)
             i += n
-        run.close()
         ctx.sc, ctx.sf, ctx.cells, ctx.steps, ctx.K = sc, sf, cells, steps, K
         ctx.in_place = in_place
         ctx.observe, ctx.observe_from = observe, observe_from
@@ -619,8 +633,8 @@ def k17_two_level_steps(fc0: torch.Tensor, ff0: torch.Tensor, coarse: Lattice, f
     parity, is summed over the coarse states after steps observe_from .. steps-1 and returned as
     the third output (FP64); its gradient enters the reverse sweep step by step, so a time
     average over thousands of steps needs no stored states beyond the checkpoints.
-    graphs: the forward sweep replays one HIP graph per coarse parity (False: every launch from
-    the host; the results are the same bit for bit).
+    graphs: the library enqueues the forward sweep's launches itself (False: every launch from
+    Python; the results are the same bit for bit).
     keep_bytes: device memory the forward may keep for the backward. The trailing checkpoint
     segments whose coarse steps' states (two fine buffers, the coarse buffer and the BC lists'
     post-collision values per coarse step) fit in it are stepped out of place and keep every
@@ -677,6 +691,28 @@ def _level_step_in_place(steppers, cells, bufs, level, even, stream):
     steppers[level].forward(bufs[level], even, None, stream)
     if finer:
         _refresh_interface(steppers, cells, level, bufs[level], bufs[level + 1], bufs[level + 1], even, stream)
+
+
+def _level_launches(steppers, cells, bufs, even):
+    """The launches of a coarse step in place on bufs (_level_step_in_place) and the coarsest level's
+    parameter struct, for StepLaunches. Finer levels start each coarse step with the even parity and
+    are back at it after their two steps."""
+    params = [_param(s.L, b, even if level == 0 else True) for level, (s, b) in enumerate(zip(steppers, bufs))]
+    out = LaunchList()
+
+    def add(level):
+        finer = level + 1 < len(steppers)
+        if finer:
+            add(level + 1)
+            add(level + 1)
+        steppers[level].add_launches(out, params[level])
+        if finer:
+            cf, fc = cells[level]
+            out.fine_to_coarse(params[level], params[level + 1], fc)
+            out.coarse_to_fine(params[level], params[level + 1], cf)
+
+    add(0)
+    return out, params[0]
 
 
 def _level_step_record(steppers, cells, bufs, level, even, stream, post_lists):
@@ -750,7 +786,8 @@ class _MultiLevelSteps(torch.autograd.Function):
                 L.set_porosity(p.detach())
         # the values this forward used: the backward replays with them
         ctx.params = [_bc_snapshot(L) for L in lats]
-        run = _StepGraphs(lambda ev, st: _level_step_in_place(steppers, cells, bufs, 0, ev, st), graphs)
+        run = StepLaunches(lambda ev, st: _level_step_in_place(steppers, cells, bufs, 0, ev, st),
+                           _level_launches(steppers, cells, bufs, even0) if graphs else None)
         checkpoints = []
         # the trailing segments whose records fit keep_bytes are stepped out of place and kept, so
         # the backward walks them without a replay. A step of level l (2^l per coarse step) keeps
@@ -795,7 +832,6 @@ class _MultiLevelSteps(torch.autograd.Function):
             n_run = min(K - i % K, steps - i, (observe_from - i) if observe is not None else steps)
             even = run.run(n_run, even)
             i += n_run
-        run.close()
         ctx.meta = meta
         ctx.checkpoints = checkpoints
         ctx.flags = (velocity is not None, rho_bc is not None, [p is not None for p in pors])
@@ -870,8 +906,8 @@ def k17_multilevel_steps(f0s, lattices, interfaces, steps: int, checkpoint_every
     A coarse step follows UpdateGrid27::updateGrid (src/gpu/core/Calculation/UpdateGrid27.cpp:54-96):
     every finer level takes two steps per step of the level above it (even parity first, so every
     finer level starts with the even parity), then the level steps and refreshes the interface to
-    its finer level (fine -> coarse, coarse -> fine). The forward works in place and replays HIP
-    graphs of the coarse step (graphs=False: launches from the host, the same bit for bit); the
+    its finer level (fine -> coarse, coarse -> fine). The forward works in place, the
+    launches enqueued natively (graphs=False: from Python, the same bit for bit); the
     backward replays each checkpoint segment out of place, keeping every level's intermediate
     states, and walks it in reverse: per step of a level, the interface adjoints, the level's step
     adjoint, then its finer level's two steps. For two levels it computes what k17_two_level_steps

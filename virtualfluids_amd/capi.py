@@ -133,6 +133,27 @@ class InterpolationSources(ctypes.Structure):
     _fields_ = [("node", _vp), ("first", _vp), ("lanes", _vp), ("numberOfNodes", ctypes.c_uint32)]
 
 
+# vf_launch_kind
+(LAUNCH_BOX, LAUNCH_BOX_BOUNCE_BACK, LAUNCH_INDICES, LAUNCH_BC, LAUNCH_SWAP, LAUNCH_COARSE_TO_FINE,
+ LAUNCH_FINE_TO_COARSE) = range(7)
+
+
+class Launch(ctypes.Structure):
+    """vf_launch: one entry of a sequence of launches (vf_run_launches)."""
+
+    _fields_ = [
+        ("kind", ctypes.c_int32),
+        ("collisionTemplate", ctypes.c_int32),
+        ("level", ctypes.POINTER(LBMParameter)),
+        ("fine", ctypes.POINTER(LBMParameter)),
+        ("bc", _vp),
+        ("list", ctypes.POINTER(QBoundaryConditions)),
+        ("bounceBack", ctypes.POINTER(PostBounceBack)),
+        ("cells", ctypes.POINTER(InterpolationCells)),
+        ("offsets", ctypes.POINTER(InterpolationCellNeighbor)),
+    ]
+
+
 # VF_ABI_VERSION of include/virtualfluids_amd.h that these structs mirror
 ABI_VERSION = 6
 
@@ -180,6 +201,7 @@ SIGNATURES = {
     "vf_PressureNonEquilibriumCompressibleAdjoint": [_P, _Q, _vp, _vp, ctypes.c_int32, _vp],
     "vf_InitNavierStokesCompressibleNonEquilibrium": [_P, _vp, _vp],
     "vf_ScaleFineToCoarseCompressible": [_P, _P, _vp, _vp, _vp],
+    "vf_run_launches": [_vp, ctypes.c_uint32, ctypes.c_uint32, _vp],
 }
 
 _lib = None

@@ -282,38 +282,54 @@ class Simulation:
 
         L = self.lattice
         L.collide(stream=stream)
-        if self.groups is None:
-            self.groups = post_launch_groups(L, [("velocity", self.velocity_fn), ("noslip", self.noslip_fn),
-                                                 ("geometry", self.geometry_fn)])
-        for _, fn, bc in self.groups:
+        for _, fn, bc in self._post_groups():
             capi.call(fn, L.pref(), ctypes.byref(bc.struct), stream_handle(stream))
+
+    def _post_groups(self):
+        """The post-collision launches (post_launch_groups), built on first use."""
+        if self.groups is None:
+            self.groups = post_launch_groups(self.lattice, [("velocity", self.velocity_fn),
+                                                            ("noslip", self.noslip_fn),
+                                                            ("geometry", self.geometry_fn)])
+        return self.groups
 
     def step(self, stream=None):
         self._launch(stream)
         self.t += 1
 
+    def add_launches(self, out):
+        """Append the launches of one step (what _launch makes) to a LaunchList."""
+        L = self.lattice
+        if self.fused is not None:
+            out.collide_bounce_back(L.param, self.fused.struct)
+        else:
+            out.collide(L.param, L.box)
+            for _, fn, bc in self._post_groups():
+                out.bc(L.param, fn, bc.struct)
+        out.swap(L.param)
+        bc = L.bcs.get("pressure")
+        if self.pressure_fn and bc is not None and bc.n:
+            out.bc(L.param, self.pressure_fn, bc.struct)
+
     def run(self, steps: int, stream=None, graphs: bool = True):
-        """`steps` time steps. With graphs (and no explicit stream) the steps' launches are
-        captured once, 16 steps to a graph, and replayed (virtualfluids_amd.graphs.StepGraphs):
-        the same kernels with the same arguments, without a host round trip per launch;
-        graphs=False launches every kernel from the host."""
-        if not graphs or stream is not None or steps < 3:
+        """`steps` time steps. With graphs (the default) the library enqueues the steps' launches
+        itself (virtualfluids_amd.launches): the same kernels with the same arguments, without a host
+        round trip per launch; without an explicit stream a run of three or more steps returns once
+        they are done. graphs=False launches every kernel from Python."""
+        if not graphs:
             for _ in range(steps):
                 self.step(stream)
             return
-        from .graphs import StepGraphs
+        import torch
 
-        L = self.lattice
+        from .launches import LaunchList
 
-        def launch(even, st):
-            L.even = even
-            self._launch(st)
-
-        # the steps' parity swaps are host state, which a replay does not run: set it after
-        run = StepGraphs(launch)
-        L.even = run.run(steps, L.even)
-        run.close()
-        self.t += steps
+        out = LaunchList()
+        self.add_launches(out)
+        out.run(steps, stream)
+        self.t += max(steps, 0)
+        if stream is None and steps >= 3:
+            torch.cuda.current_stream().synchronize()
 
 
 class MultiLevelSimulation:
@@ -365,35 +381,39 @@ class MultiLevelSimulation:
         self._update(0, stream)
         self.t += 1
 
+    def _add_launches(self, level: int, out):
+        """Append the launches of one step of `level` (what _update makes) to a LaunchList."""
+        fine = len(self.lattices) - 1
+        if level != fine:
+            self._add_launches(level + 1, out)
+            self._add_launches(level + 1, out)
+        self.levels[level].add_launches(out)
+        if level != fine:
+            cf, fc = self.cells[level]
+            coarse_p, fine_p = self.lattices[level].param, self.lattices[level + 1].param
+            if self.manager.scaling_fine_to_coarse:
+                out.fine_to_coarse(coarse_p, fine_p, fc)
+            if self.manager.scaling_coarse_to_fine:
+                out.coarse_to_fine(coarse_p, fine_p, cf)
+
     def run(self, steps: int, stream=None, graphs: bool = True):
-        """`steps` coarse steps. With graphs (and no explicit stream) pairs of coarse steps
-        replay one HIP graph after two steps from the host (after a pair every level's parity
-        is back where it started); graphs=False launches every kernel from the host. The
-        fields are the same bit for bit."""
-        if not graphs or stream is not None or steps < 4:
+        """`steps` coarse steps. With graphs (the default) the library enqueues the steps' launches
+        itself (virtualfluids_amd.launches); without an explicit stream a run of four or more steps
+        returns once they are done. graphs=False launches every kernel from Python. The fields are
+        the same bit for bit."""
+        if not graphs:
             for _ in range(steps):
                 self.step(stream)
             return
         import torch
 
-        from .graphs import capture
+        from .launches import LaunchList
 
-        for _ in range(2):
-            self.step()
-        steps -= 2
-        pairs = steps // 2
-        if pairs:
-            saved_t = [lv.t for lv in self.levels]
-            g = capture(lambda st: (self._update(0, st), self._update(0, st)), torch.cuda.Stream())
-            # the capture ran the host side of a pair (parities are back); no step was taken
-            for lv, t in zip(self.levels, saved_t):
-                lv.t = t
-            for _ in range(pairs):
-                g.replay()
-            torch.cuda.current_stream().synchronize()  # before the graph is released
-            del g
-            for level, lv in enumerate(self.levels):
-                lv.t += 2 * pairs * 2 ** level
-            self.t += 2 * pairs
-        if steps % 2:
-            self.step()
+        out = LaunchList()
+        self._add_launches(0, out)
+        out.run(steps, stream)
+        for level, lv in enumerate(self.levels):
+            lv.t += max(steps, 0) * 2 ** level
+        self.t += max(steps, 0)
+        if stream is None and steps >= 4:
+            torch.cuda.current_stream().synchronize()
