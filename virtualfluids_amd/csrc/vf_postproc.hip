@@ -20,7 +20,9 @@ namespace vfa {
 
 namespace {
 
-constexpr int kSumThreads = 256;
+// One workgroup sums a list (a fixed order without a workspace): its 16 waves are all the
+// loads in flight there are
+constexpr int kSumThreads = 1024;
 
 __device__ __forceinline__ double wave_sum(double v)
 {
@@ -70,13 +72,25 @@ __global__ __launch_bounds__(kSumThreads) void drag_sum_kernel(const S* __restri
     for (uint32_t i = threadIdx.x; i < nbc; i += kSumThreads) {
         uint32_t n[8];
         cell_nodes(a, (uint32_t)k[i], n);
+        // every distance, then every active link's two populations, each before the first is used:
+        // a chain of 26 distance -> population latencies per node otherwise (sphere channel, 3 000
+        // nodes: 82 us with 256 threads and the chain, 25 us so)
+        uint32_t active = 0;
+#pragma unroll
+        for (int e = 1; e < 27; ++e) active |= (link_active(q[(uint64_t)e * nbc + i]) ? 1u : 0u) << e;
+        float out[27], back[27];
 #pragma unroll
         for (int e = 1; e < 27; ++e) {
-            if (!link_active(q[(uint64_t)e * nbc + i])) continue;
             const uint32_t m = n[node_sel(inv(e))];
-            const double out = (double)Codec<S>::load(slot_ptr(const_cast<S*>(f), a.N, e, even) + m);
-            const double back = (double)Codec<S>::load(slot_ptr(const_cast<S*>(f), a.N, inv(e), even) + m);
-            const double s = out + back;
+            out[e] = back[e] = 0.0f;
+            if (active >> e & 1u) {
+                out[e] = Codec<S>::load(slot_ptr(const_cast<S*>(f), a.N, e, even) + m);
+                back[e] = Codec<S>::load(slot_ptr(const_cast<S*>(f), a.N, inv(e), even) + m);
+            }
+        }
+#pragma unroll
+        for (int e = 1; e < 27; ++e) {
+            const double s = (double)out[e] + (double)back[e];
             acc[0] += cx(e) * s;
             acc[1] += cy(e) * s;
             acc[2] += cz(e) * s;
@@ -107,33 +121,60 @@ __device__ __forceinline__ bool interior_fluid(const Addr& a, const uint32_t* nb
 {
     auto fl = [&](uint32_t j) { return geo[j] == VF_GEO_FLUID; };
     if (!fl(k)) return false;
-    if (a.nbx) {
-        const uint32_t m = nbinv[k];
-        return fl(a.nbx[k]) && fl(a.nby[k]) && fl(a.nbz[k]) && fl(m) && fl(a.nbz[a.nby[m]]) && fl(a.nbz[a.nbx[m]]) &&
-               fl(a.nby[a.nbx[m]]);
-    }
-    const uint32_t nx = (uint32_t)a.nx, ny = (uint32_t)a.ny, nz = (uint32_t)a.nz;
-    const uint32_t x = k % nx, t = k / nx, y = t % ny, z = t / ny;
-    const uint32_t xp = x + 1 == nx ? 0 : x + 1, xm = x == 0 ? nx - 1 : x - 1;
-    const uint32_t yp = y + 1 == ny ? 0 : y + 1, ym = y == 0 ? ny - 1 : y - 1;
-    const uint32_t zp = z + 1 == nz ? 0 : z + 1, zm = z == 0 ? nz - 1 : z - 1;
-    auto at = [&](uint32_t xx, uint32_t yy, uint32_t zz) { return xx + nx * (yy + ny * zz); };
-    return fl(at(xp, y, z)) && fl(at(xm, y, z)) && fl(at(x, yp, z)) && fl(at(x, ym, z)) && fl(at(x, y, zp)) &&
-           fl(at(x, y, zm)) && fl(at(xm, ym, zm));
+    const uint32_t m = nbinv[k];
+    return fl(a.nbx[k]) && fl(a.nby[k]) && fl(a.nbz[k]) && fl(m) && fl(a.nbz[a.nby[m]]) && fl(a.nbz[a.nbx[m]]) &&
+           fl(a.nby[a.nbx[m]]);
 }
 
-__global__ __launch_bounds__(256) void kinetic_energy_kernel(Addr a, const uint32_t* nbinv, const uint32_t* geo,
-                                                             const float* vx, const float* vy, const float* vz,
-                                                             const float* rho, double* out)
+__device__ __forceinline__ double node_energy(const float* vx, const float* vy, const float* vz, const float* rho,
+                                              uint32_t k)
 {
-    __shared__ double part[4][2];
+    const double ux = vx[k], uy = vy[k], uz = vz[k];
+    return 0.5 * (ux * ux + uy * uy + uz * uz) * ((double)rho[k] + 1.0);
+}
+
+// BOX: nodes numbered over the planes of a dense box (plane_sum_grid), so that the seven neighbours
+// are offsets; their types and the node's fields are loaded together (one by one
+// behind the previous test they are eight memory latencies a node). Bound by HBM: 20 bytes a node.
+// 256^3: 156 us with the chain, a division per coordinate and 2048 workgroups, 66 us so.
+template <bool BOX>
+__global__ __launch_bounds__(kReduceThreads) void kinetic_energy_kernel(Addr a, const uint32_t* nbinv, const uint32_t* geo,
+                                                             const float* vx, const float* vy, const float* vz,
+                                                             const float* rho, PlaneDiv plane, double* out)
+{
+    __shared__ double part[kReduceThreads / 64][2];
     double e = 0.0, c = 0.0;
-    for (uint64_t kk = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; kk < a.N; kk += (uint64_t)gridDim.x * blockDim.x) {
-        const uint32_t k = (uint32_t)kk;
-        if (!interior_fluid(a, nbinv, geo, k)) continue;
-        const double ux = vx[k], uy = vy[k], uz = vz[k];
-        e += 0.5 * (ux * ux + uy * uy + uz * uz) * ((double)rho[k] + 1.0);
-        c += 1.0;
+    if constexpr (BOX) {
+        const uint32_t nx = plane.nx, ny = (uint32_t)a.ny, nz = (uint32_t)a.nz, P = plane.planeNodes;
+        const uint32_t per = (P + kReduceThreads - 1) / kReduceThreads;
+        for (uint64_t i = blockIdx.x; i < (uint64_t)per * nz; i += gridDim.x) {
+            const uint32_t z = (uint32_t)(i / per), t = (uint32_t)(i % per) * kReduceThreads + threadIdx.x;
+            if (t >= P) continue;
+            const uint32_t y = plane_row(t, plane), x = t - y * nx;
+            const uint32_t xp = x + 1 == nx ? t + 1 - nx : t + 1, xm = x == 0 ? t + nx - 1 : t - 1;
+            const uint32_t yp = y + 1 == ny ? x : t + nx, ym = y == 0 ? t + (P - nx) : t - nx;
+            const uint32_t xym = y == 0 ? xm + (P - nx) : xm - nx;
+            const uint32_t zo = P * z, zp = P * (z + 1 == nz ? 0 : z + 1), zm = P * (z == 0 ? nz - 1 : z - 1);
+            const uint32_t k = zo + t;
+            const uint32_t g[8] = {geo[k],       geo[zo + xp], geo[zo + xm], geo[zo + yp],
+                                   geo[zo + ym], geo[zp + t],  geo[zm + t],  geo[zm + xym]};
+            const double en = node_energy(vx, vy, vz, rho, k);
+            bool in = true;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) in &= g[j] == VF_GEO_FLUID;
+            if (in) {
+                e += en;
+                c += 1.0;
+            }
+        }
+    } else {
+        for (uint64_t kk = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; kk < a.N;
+             kk += (uint64_t)gridDim.x * blockDim.x) {
+            const uint32_t k = (uint32_t)kk;
+            if (!interior_fluid(a, nbinv, geo, k)) continue;
+            e += node_energy(vx, vy, vz, rho, k);
+            c += 1.0;
+        }
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     e = wave_sum(e);
@@ -144,7 +185,8 @@ __global__ __launch_bounds__(256) void kinetic_energy_kernel(Addr a, const uint3
     }
     __syncthreads();
     if (threadIdx.x < 2) {
-        const double s = part[0][threadIdx.x] + part[1][threadIdx.x] + part[2][threadIdx.x] + part[3][threadIdx.x];
+        double s = 0.0;
+        for (int w = 0; w < kReduceThreads / 64; ++w) s += part[w][threadIdx.x];
         atomicAdd(out + threadIdx.x, s);
     }
 }
@@ -264,10 +306,16 @@ extern "C" int vf_KineticEnergy(const vf_lbm_parameter* p, const uint32_t* neigh
         return VF_ERR_INVALID_ARGUMENT;
     }
     hipStream_t s = (hipStream_t)stream;
-    const uint64_t blocks = (p->numberOfNodes + 255) / 256;
     hipLaunchKernelGGL(zero2_kernel, dim3(1), dim3(64), 0, s, out2);
-    hipLaunchKernelGGL(kinetic_energy_kernel, dim3((unsigned)(blocks < 2048 ? blocks : 2048)), dim3(256), 0, s,
-                       make_addr(*p), neighborInverse, p->typeOfGridNode, p->velocityX, p->velocityY, p->velocityZ,
-                       p->rho, out2);
+    if (!p->neighborX) {
+        const dim3 grid = plane_sum_grid(p->nx, p->ny, p->nz);
+        hipLaunchKernelGGL(kinetic_energy_kernel<true>, grid, dim3(kReduceThreads), 0, s, make_addr(*p), neighborInverse,
+                           p->typeOfGridNode, p->velocityX, p->velocityY, p->velocityZ, p->rho,
+                           make_plane_div(p->nx, p->ny), out2);
+    } else {
+        hipLaunchKernelGGL(kinetic_energy_kernel<false>, flat_sum_grid(p->numberOfNodes), dim3(kReduceThreads), 0, s,
+                           make_addr(*p), neighborInverse, p->typeOfGridNode, p->velocityX, p->velocityY,
+                           p->velocityZ, p->rho, PlaneDiv{}, out2);
+    }
     return check_launch("kineticEnergyKernel execution failed");
 }

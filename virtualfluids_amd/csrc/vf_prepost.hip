@@ -7,6 +7,7 @@
 //   reductions   sums of drho, momentum and kinetic energy accumulated in FP64: per-wave
 //                shuffles, one LDS pass per workgroup, one FP64 atomic per workgroup.
 #include "vf_lattice.h"
+#include "vf_rowio.h"
 
 namespace vfa {
 
@@ -125,16 +126,38 @@ __device__ __forceinline__ bool is_valid_fluid(uint32_t t)
     return t == VF_GEO_FLUID || t == VF_GEO_PM_0 || t == VF_GEO_PM_1 || t == VF_GEO_PM_2;
 }
 
-// Moments of one node accumulated in FP64 (every population converted before the add).
-template <class S> __device__ __forceinline__ void node_moments(const S* f, const Addr& a, uint32_t k, bool even,
-                                                               double& drho, double& jx, double& jy, double& jz)
+// The cell nodes of node t of plane z (t = x + nx y) of a dense box
+__device__ __forceinline__ void plane_cell_nodes(const PlaneDiv& p, int ny, int nz, uint32_t t, uint32_t z,
+                                                 uint32_t (&n)[8])
 {
-    uint32_t n[8];
-    cell_nodes(a, k, n);
+    const uint32_t y = plane_row(t, p), x = t - y * p.nx, P = p.planeNodes;
+    const uint32_t xp = x + 1 == p.nx ? 0 : x + 1;
+    const uint32_t r0 = t - x, r1 = y + 1 == (uint32_t)ny ? 0 : r0 + p.nx;
+    const uint32_t z0 = P * z, z1 = z + 1 == (uint32_t)nz ? 0 : z0 + P;
+    n[0] = z0 + r0 + x; n[1] = z0 + r0 + xp; n[2] = z0 + r1 + x; n[3] = z0 + r1 + xp;
+    n[4] = z1 + r0 + x; n[5] = z1 + r0 + xp; n[6] = z1 + r1 + x; n[7] = z1 + r1 + xp;
+}
+
+// The 27 pre-collision populations of a node: through buffer descriptors (BUF) or 64-bit addresses
+template <class S, bool BUF>
+__device__ __forceinline__ void load_cell(const SlotIO<S, BUF>& io, const uint32_t (&n)[8], bool even, float (&v)[27])
+{
+    if (even) {
+#pragma unroll
+        for (int d = 0; d < 27; ++d) v[d] = io.load(d, n[node_sel(d)] * (uint32_t)sizeof(S));
+    } else {
+#pragma unroll
+        for (int d = 0; d < 27; ++d) v[d] = io.load(inv(d), n[node_sel(d)] * (uint32_t)sizeof(S));
+    }
+}
+
+// Moments of one node accumulated in FP64 (every population converted before the add).
+__device__ __forceinline__ void node_moments(const float (&f)[27], double& drho, double& jx, double& jy, double& jz)
+{
     drho = jx = jy = jz = 0.0;
 #pragma unroll
     for (int d = 0; d < 27; ++d) {
-        const double v = (double)read_pre(f, a, n, d, even);
+        const double v = (double)f[d];
         drho += v;
         if (cx(d)) jx += double(cx(d)) * v;
         if (cy(d)) jy += double(cy(d)) * v;
@@ -142,20 +165,33 @@ template <class S> __device__ __forceinline__ void node_moments(const S* f, cons
     }
 }
 
-template <class S>
-__global__ __launch_bounds__(256) void macroscopic_kernel(const S* __restrict__ f, Addr a, const uint32_t* geo, float* rho,
-                                                          float* vx, float* vy, float* vz, float* press, int even_flag)
+// BOX: nodes numbered over the planes of a dense box (one per thread, grid.y the plane), populations
+// through buffer descriptors where they reach. Bound by HBM: 27 populations, the type and five
+// fields a node. 256^3 FP32: 429 us with a division per coordinate and every field written twice
+// (zero, then the value).
+template <class S, bool BOX, bool BUF>
+__global__ __launch_bounds__(256) void macroscopic_kernel(const S* __restrict__ f, Addr a, PlaneDiv plane,
+                                                          const uint32_t* geo, float* rho, float* vx, float* vy,
+                                                          float* vz, float* press, int even_flag)
 {
-    const uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= a.N) return;
-    rho[k] = vx[k] = vy[k] = vz[k] = 0.0f;
-    if (press) press[k] = 0.0f;
-    if (geo && !is_valid_fluid(geo[k])) return;
+    uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     uint32_t n[8];
-    cell_nodes(a, (uint32_t)k, n);
+    if constexpr (BOX) {
+        if (k >= plane.planeNodes) return;
+        plane_cell_nodes(plane, a.ny, a.nz, (uint32_t)k, blockIdx.y, n);
+        k = n[0];
+    } else {
+        if (k >= a.N) return;
+    }
+    if (geo && !is_valid_fluid(geo[k])) {
+        rho[k] = vx[k] = vy[k] = vz[k] = 0.0f;
+        if (press) press[k] = 0.0f;
+        return;
+    }
+    if constexpr (!BOX) cell_nodes(a, (uint32_t)k, n);
+    const SlotIO<S, BUF> io(f, a.N);
     float fv[27];
-#pragma unroll
-    for (int d = 0; d < 27; ++d) fv[d] = read_pre(f, a, n, d, even_flag != 0);
+    load_cell<S, BUF>(io, n, even_flag != 0, fv);
     float drho = 0.0f, jx = 0.0f, jy = 0.0f, jz = 0.0f, e1 = 0.0f, e2 = 0.0f, e3 = 0.0f;
 #pragma unroll
     for (int d = 0; d < 27; ++d) {
@@ -191,26 +227,48 @@ __device__ __forceinline__ double wave_sum(double v)
     return v;
 }
 
-// out[0..3] += sum drho, jx, jy, jz; out[4] += sum 1/2 (1+drho) |u|^2 (when KE)
-template <class S, bool KE>
-__global__ __launch_bounds__(256) void moments_reduce_kernel(const S* __restrict__ f, Addr a, const uint32_t* geo,
-                                                             int even_flag, double* out)
+// out[0..3] += sum drho, jx, jy, jz; out[4] += sum 1/2 (1+drho) |u|^2 (when KE).
+// BOX, BUF as in macroscopic_kernel; a workgroup steps through the planes (plane_sum_grid). Bound
+// by HBM: 27 populations and the type a node (256^3 FP32 327 us, FP16 197 -> 174 us).
+template <class S, bool KE, bool BOX, bool BUF>
+__global__ __launch_bounds__(kReduceThreads) void moments_reduce_kernel(const S* __restrict__ f, Addr a, PlaneDiv plane,
+                                                             const uint32_t* geo, int even_flag, double* out)
 {
     constexpr int NV = KE ? 5 : 4;
-    __shared__ double part[4][NV];
+    __shared__ double part[kReduceThreads / 64][NV];
     double acc[NV];
 #pragma unroll
     for (int j = 0; j < NV; ++j) acc[j] = 0.0;
-    for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k < a.N; k += (uint64_t)gridDim.x * blockDim.x) {
-        if (geo && geo[k] != VF_GEO_FLUID) continue;
+    const SlotIO<S, BUF> io(f, a.N);
+    auto add = [&](const uint32_t (&n)[8]) {
+        float fv[27];
+        load_cell<S, BUF>(io, n, even_flag != 0, fv);
         double drho, jx, jy, jz;
-        node_moments(f, a, (uint32_t)k, even_flag != 0, drho, jx, jy, jz);
+        node_moments(fv, drho, jx, jy, jz);
         acc[0] += drho;
         acc[1] += jx;
         acc[2] += jy;
         acc[3] += jz;
         if (KE) {
             acc[NV - 1] += 0.5 * (jx * jx + jy * jy + jz * jz) / (1.0 + drho);
+        }
+    };
+    uint32_t n[8];
+    if constexpr (BOX) {
+        const uint32_t per = (plane.planeNodes + kReduceThreads - 1) / kReduceThreads;
+        for (uint64_t i = blockIdx.x; i < (uint64_t)per * (uint32_t)a.nz; i += gridDim.x) {
+            const uint32_t z = (uint32_t)(i / per), t = (uint32_t)(i % per) * kReduceThreads + threadIdx.x;
+            if (t >= plane.planeNodes) continue;
+            plane_cell_nodes(plane, a.ny, a.nz, t, z, n);
+            if (geo && geo[n[0]] != VF_GEO_FLUID) continue;
+            add(n);
+        }
+    } else {
+        for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k < a.N;
+             k += (uint64_t)gridDim.x * blockDim.x) {
+            if (geo && geo[k] != VF_GEO_FLUID) continue;
+            cell_nodes(a, (uint32_t)k, n);
+            add(n);
         }
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -221,7 +279,8 @@ __global__ __launch_bounds__(256) void moments_reduce_kernel(const S* __restrict
     }
     __syncthreads();
     if (threadIdx.x < NV) {
-        const double s = part[0][threadIdx.x] + part[1][threadIdx.x] + part[2][threadIdx.x] + part[3][threadIdx.x];
+        double s = 0.0;
+        for (int w = 0; w < kReduceThreads / 64; ++w) s += part[w][threadIdx.x];
         atomicAdd(out + threadIdx.x, s);
     }
 }
@@ -253,26 +312,46 @@ template <class S> struct InitNeqL {
                            p.isEvenTimestep);
     }
 };
+// whether the plane-numbered forms serve a lattice: a dense box whose planes fit grid.y
+static bool plane_box(const vf_lbm_parameter& p) { return !p.neighborX && p.nz <= 65535; }
+
 template <class S> struct MacroL {
+    template <bool BOX, bool BUF> static void go(const vf_lbm_parameter& p, hipStream_t s)
+    {
+        const dim3 grid = BOX ? dim3(plane_blocks(p.nx, p.ny), p.nz) : dim3((unsigned)((p.numberOfNodes + 255) / 256));
+        // FP32 beyond the cache: four resident workgroups per CU (415 -> 402 us at 256^3); a 16-bit
+        // lattice needs every wave (234 -> 253 us at four)
+        const bool cap = BOX && sizeof(S) == 4 && 27 * p.numberOfNodes * sizeof(S) > (256ull << 20);
+        hipLaunchKernelGGL((macroscopic_kernel<S, BOX, BUF>), grid, dim3(256), lds_reserve_for(cap ? 4 : 0), s, (const S*)p.distributions,
+                           make_addr(p), BOX ? make_plane_div(p.nx, p.ny) : PlaneDiv{}, p.typeOfGridNode, p.rho,
+                           p.velocityX, p.velocityY, p.velocityZ, p.pressure, p.isEvenTimestep);
+    }
     static void run(const vf_lbm_parameter& p, hipStream_t s)
     {
-        const dim3 grid((unsigned)((p.numberOfNodes + 255) / 256));
-        hipLaunchKernelGGL(macroscopic_kernel<S>, grid, dim3(256), 0, s, (const S*)p.distributions, make_addr(p),
-                           p.typeOfGridNode, p.rho, p.velocityX, p.velocityY, p.velocityZ, p.pressure, p.isEvenTimestep);
+        if (!plane_box(p)) go<false, false>(p, s);
+        else if (slots_fit_buffers(p.numberOfNodes, sizeof(S))) go<true, true>(p, s);
+        else go<true, false>(p, s);
     }
 };
 template <class S> struct ReduceL {
+    template <bool KE, bool BOX, bool BUF> static void go(const vf_lbm_parameter& p, double* out, hipStream_t s)
+    {
+        const dim3 grid = BOX ? plane_sum_grid(p.nx, p.ny, p.nz) : flat_sum_grid(p.numberOfNodes);
+        hipLaunchKernelGGL((moments_reduce_kernel<S, KE, BOX, BUF>), grid, dim3(kReduceThreads), 0, s, (const S*)p.distributions,
+                           make_addr(p), BOX ? make_plane_div(p.nx, p.ny) : PlaneDiv{}, p.typeOfGridNode,
+                           p.isEvenTimestep, out);
+    }
+    template <bool KE> static void pick(const vf_lbm_parameter& p, double* out, hipStream_t s)
+    {
+        if (!plane_box(p)) go<KE, false, false>(p, out, s);
+        else if (slots_fit_buffers(p.numberOfNodes, sizeof(S))) go<KE, true, true>(p, out, s);
+        else go<KE, true, false>(p, out, s);
+    }
     static void run(const vf_lbm_parameter& p, double* out, bool ke, hipStream_t s)
     {
-        const uint64_t blocks = (p.numberOfNodes + 255) / 256;
-        const dim3 grid((unsigned)(blocks < 2048 ? blocks : 2048));
         hipLaunchKernelGGL(zero_doubles_kernel, dim3(1), dim3(64), 0, s, out, ke ? 5 : 4);
-        if (ke)
-            hipLaunchKernelGGL((moments_reduce_kernel<S, true>), grid, dim3(256), 0, s, (const S*)p.distributions,
-                               make_addr(p), p.typeOfGridNode, p.isEvenTimestep, out);
-        else
-            hipLaunchKernelGGL((moments_reduce_kernel<S, false>), grid, dim3(256), 0, s, (const S*)p.distributions,
-                               make_addr(p), p.typeOfGridNode, p.isEvenTimestep, out);
+        if (ke) pick<true>(p, out, s);
+        else pick<false>(p, out, s);
     }
 };
 

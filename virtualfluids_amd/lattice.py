@@ -233,10 +233,17 @@ class Lattice:
         for dst, src in ((self.rho, rho), (self.vx, ux), (self.vy, uy), (self.vz, uz)):
             dst.copy_(torch.as_tensor(np.asarray(src, dtype=np.float32) if not torch.is_tensor(src) else src,
                                       dtype=torch.float32))
+        capi.call("vf_InitNavierStokesCompressibleNonEquilibrium", self.pref(), self._neighbor_inverse(),
+                  stream_handle(stream))
+
+    def _neighbor_inverse(self):
+        """The (-1,-1,-1) neighbours on the device, built on first use; None on a box lattice, whose
+        kernels step by coordinates."""
+        if self.box:
+            return None
         if not hasattr(self, "nbinv"):
             self.nbinv = _u32(self.grid.neighbor_inverse(), self.device)
-        capi.call("vf_InitNavierStokesCompressibleNonEquilibrium", self.pref(), _ptr(self.nbinv),
-                  stream_handle(stream))
+        return _ptr(self.nbinv)
 
     def macroscopic(self, stream=None):
         """drho, vx, vy, vz, p from the pre-collision state (host numpy arrays)."""
@@ -275,10 +282,8 @@ class Lattice:
         six face neighbours and (-1,-1,-1) neighbour are fluid, from the macroscopic fields of the
         current state."""
         capi.call("vf_CalculateMacroscopicQuantitiesCompressible", self.pref(), stream_handle(stream))
-        if not hasattr(self, "nbinv"):
-            self.nbinv = _u32(self.grid.neighbor_inverse(), self.device)
         out = torch.zeros(2, dtype=torch.float64, device=self.device)
-        capi.call("vf_KineticEnergy", self.pref(), _ptr(self.nbinv), _ptr(out), stream_handle(stream))
+        capi.call("vf_KineticEnergy", self.pref(), self._neighbor_inverse(), _ptr(out), stream_handle(stream))
         torch.cuda.synchronize(self.device)
         e, c = out.cpu().numpy()
         return float(e), int(round(c))
