@@ -66,9 +66,11 @@ enum vf_box_kernel {
     VF_BOX_KERNEL_NODE = 2  /* one node per thread (cache-resident form) */
 };
 enum vf_row_addressing {
-    VF_ROW_ADDRESSING_AUTO = 0,   /* buffer descriptors where 14 direction slots fit in 4 GiB */
-    VF_ROW_ADDRESSING_BUFFER = 1, /* buffer descriptors (only where they fit; else 64-bit) */
-    VF_ROW_ADDRESSING_GLOBAL = 2  /* 64-bit global addresses */
+    VF_ROW_ADDRESSING_AUTO = 0,   /* buffer descriptors: two where 14 direction slots fit in 4 GiB, else
+                                     (collision) four where 7 do, else 64-bit addresses */
+    VF_ROW_ADDRESSING_BUFFER = 1, /* as AUTO */
+    VF_ROW_ADDRESSING_GLOBAL = 2, /* 64-bit global addresses */
+    VF_ROW_ADDRESSING_BUFFER_WIDE = 3 /* four descriptors (collision; only where 7 slots fit) */
 };
 enum vf_adjoint_kernel {
     VF_ADJOINT_KERNEL_AUTO = 0,

@@ -35,7 +35,7 @@ _vp = ctypes.c_void_p
 
 # vf_box_kernel, vf_row_addressing, vf_adjoint_kernel
 BOX_KERNEL_AUTO, BOX_KERNEL_ROW, BOX_KERNEL_NODE = 0, 1, 2
-ROW_ADDRESSING_AUTO, ROW_ADDRESSING_BUFFER, ROW_ADDRESSING_GLOBAL = 0, 1, 2
+ROW_ADDRESSING_AUTO, ROW_ADDRESSING_BUFFER, ROW_ADDRESSING_GLOBAL, ROW_ADDRESSING_BUFFER_WIDE = 0, 1, 2, 3
 ADJOINT_KERNEL_AUTO, ADJOINT_KERNEL_ROW_WHOLE, ADJOINT_KERNEL_NODE, ADJOINT_KERNEL_ROW = 0, 1, 2, 3
 
 

@@ -219,17 +219,17 @@ __global__ __launch_bounds__(kBoxBlock) void k17_box_into_kernel(const S* __rest
 // the row, and around the periodic wrap, the boundary lanes trade those values through LDS.
 // A row need not fill its last wave (the lanes beyond it idle), and a Brinkman porosity field
 // scales each node's collision velocity.
-constexpr int kRowMaxThreads = 256;
+constexpr int kRowMaxThreads = 512;
 
-// BUF: the direction arrays are addressed through two buffer descriptors (kRowSplit), which
-// needs kRowSplit slots to span less than 4 GiB; otherwise each direction takes a 64-bit base
-// and a global access.
+// SPLIT: the direction arrays are addressed through buffer descriptors of SPLIT slots each, which
+// must span less than 4 GiB (kRowSplit slots: two descriptors; kRowSplitWide: four, lattices up to
+// 153 M nodes in FP32); 0: each direction takes a 64-bit base and a global access.
 
 // INTO: the stepped state goes to `fout` (same addresses, another buffer) and `f` is only read;
 // solid nodes then copy their cells, so `fout` is the complete state the in-place step leaves.
 // XCD: the rows are taken in the XCD block ranges of xcd_block (rows that do not fill whole
 // cache lines)
-template <class S, int V, bool EVEN, bool MASK, bool MACRO, bool BUF, bool INTO = false, bool XCD = false>
+template <class S, int V, bool EVEN, bool MASK, bool MACRO, int SPLIT, bool INTO = false, bool XCD = false>
 __global__ __launch_bounds__(kRowMaxThreads) void k17_row_kernel(S* f, S* fout, BoxArgs a, K17Rates r)
 {
     using IO = RowIO<S, V>;
@@ -261,34 +261,30 @@ __global__ __launch_bounds__(kRowMaxThreads) void k17_row_kernel(S* f, S* fout, 
                               rows[2] * (uint32_t)sizeof(S), rows[3] * (uint32_t)sizeof(S)};
     const uint64_t slotBytes = a.N * sizeof(S);
     S* const dst = INTO ? fout : f;
-    __amdgpu_buffer_rsrc_t rsLo, rsHi, wsLo, wsHi;
+    constexpr bool BUF = SPLIT > 0;
+    constexpr int GROUP = BUF ? SPLIT : 27, GROUPS = (27 + GROUP - 1) / GROUP;
+    __amdgpu_buffer_rsrc_t rs[GROUPS], ws[GROUPS]; // read and written descriptors
     if constexpr (BUF) {
-        rsLo = __builtin_amdgcn_make_buffer_rsrc(f, (short)0, (int)0xffffffff, 0x00020000);
-        rsHi = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<char*>(f) + kRowSplit * slotBytes, (short)0,
-                                                 (int)0xffffffff, 0x00020000);
-        if constexpr (INTO) {
-            wsLo = __builtin_amdgcn_make_buffer_rsrc(dst, (short)0, (int)0xffffffff, 0x00020000);
-            wsHi = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<char*>(dst) + kRowSplit * slotBytes, (short)0,
-                                                     (int)0xffffffff, 0x00020000);
-        } else {
-            wsLo = rsLo;
-            wsHi = rsHi;
+#pragma unroll
+        for (int i = 0; i < GROUPS; ++i) {
+            const uint64_t at = (uint64_t)(i * GROUP) * slotBytes;
+            rs[i] = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<char*>(f) + at, (short)0, (int)0xffffffff, 0x00020000);
+            ws[i] = INTO ? __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<char*>(dst) + at, (short)0, (int)0xffffffff,
+                                                             0x00020000)
+                         : rs[i];
         }
     }
     // byte offset of direction d's slot from its descriptor's base
-    auto soff = [&](int d) -> uint32_t {
-        const int sl = slot<EVEN>(d);
-        return (uint32_t)(sl >= kRowSplit ? sl - kRowSplit : sl) * (uint32_t)slotBytes;
-    };
+    auto soff = [&](int d) -> uint32_t { return (uint32_t)(slot<EVEN>(d) % GROUP) * (uint32_t)slotBytes; };
     auto load = [&](int d) {
-        if constexpr (BUF) return IO::load(slot<EVEN>(d) >= kRowSplit ? rsHi : rsLo, boff[node_sel(d) >> 1], soff(d));
+        if constexpr (BUF) return IO::load(rs[slot<EVEN>(d) / GROUP], boff[node_sel(d) >> 1], soff(d));
         else {
             const char* base = reinterpret_cast<const char*>(f) + (uint64_t)slot<EVEN>(d) * slotBytes;
             return IO::load(reinterpret_cast<const S*>(base + boff[node_sel(d) >> 1]));
         }
     };
     auto store = [&](int d, const float (&vals)[V]) {
-        if constexpr (BUF) IO::store(slot<EVEN>(d) >= kRowSplit ? wsHi : wsLo, boff[node_sel(d) >> 1], soff(d), vals);
+        if constexpr (BUF) IO::store(ws[slot<EVEN>(d) / GROUP], boff[node_sel(d) >> 1], soff(d), vals);
         else {
             char* base = reinterpret_cast<char*>(dst) + (uint64_t)slot<EVEN>(d) * slotBytes;
             IO::store(reinterpret_cast<S*>(base + boff[node_sel(d) >> 1]), vals);
@@ -459,7 +455,9 @@ __global__ __launch_bounds__(kIndexedBlock) void k17_indexed_kernel(S* __restric
 
 // ---- host launchers ----------------------------------------------------------------------
 // Width (nodes per lane) of the row kernel per storage type; 0 selects the scalar kernel.
-// Measured on MI355X at 256^3: FP32 1 node/lane (5.9 TB/s; 2 nodes/lane 5.8, scalar 4.9);
+// Measured on MI355X at 256^3: FP32 1 node/lane (5.9 TB/s; 2 nodes/lane 5.8, scalar 4.9), and at 512^3
+// 1 node/lane in workgroups of 512 lanes like 2 nodes/lane in 256 at the same cap (5.02 ms; without
+// a cap 5.6-5.9);
 // FP16 and BF16 4 nodes/lane where rows are whole waves of it (1-2 % above 2 nodes/lane; both
 // near the VALU issue limit), else 2. Rows longer than one workgroup's lanes take the next width
 // that fits; rows no width fits take the scalar kernel. kernelChoice.rowWidth pins a width.
@@ -487,45 +485,48 @@ template <class S> static int row_width(int nx, const vf_kernel_choice& kc)
 // and takes every wave. The 16-bit kernels are bound by VALU issue and need every wave they can
 // get. The cap is imposed by reserving LDS at launch; kernelChoice.rowWorkgroupsPerCU pins it.
 constexpr uint64_t kCacheResidentBytes = 256ull << 20;
-template <class S, int V, bool BUF> static int row_wgs_per_cu(uint64_t workingSet, const vf_kernel_choice& kc)
+template <class S, int V, int SPLIT> static int row_wgs_per_cu(uint64_t workingSet, const vf_kernel_choice& kc)
 {
     if (kc.rowWorkgroupsPerCU != 0) return kc.rowWorkgroupsPerCU < 0 ? 0 : kc.rowWorkgroupsPerCU;
     const bool streams = workingSet > kCacheResidentBytes;
-    return (Codec<S>::storage == VF_STORAGE_FP32 && V == 1 && BUF && streams) ? 2 : 0;
+    return (Codec<S>::storage == VF_STORAGE_FP32 && V == 1 && SPLIT > 0 && streams) ? 2 : 0;
 }
 
 // out: null for the in-place step, else the buffer the out-of-place step writes
-template <class S, int V, bool EVEN, bool BUF>
+template <class S, int V, bool EVEN, int SPLIT>
 static void launch_row_b(const BoxArgs& a, const K17Rates& r, bool mask, bool macro, S* f, S* out, uint64_t ws,
                          const vf_kernel_choice& kc, hipStream_t s)
 {
     dim3 grid(a.ny, a.nz);
     dim3 block(((a.nx / V + 63) / 64) * 64); // whole waves; lanes beyond the row idle
-    const size_t lds = lds_reserve_for(row_wgs_per_cu<S, V, BUF>(ws, kc));
+    const size_t lds = lds_reserve_for(row_wgs_per_cu<S, V, SPLIT>(ws, kc));
     if (out) {
-        if (mask) hipLaunchKernelGGL((k17_row_kernel<S, V, EVEN, true, false, BUF, true>), grid, block, lds, s, f, out, a, r);
-        else hipLaunchKernelGGL((k17_row_kernel<S, V, EVEN, false, false, BUF, true>), grid, block, lds, s, f, out, a, r);
+        if (mask) hipLaunchKernelGGL((k17_row_kernel<S, V, EVEN, true, false, SPLIT, true>), grid, block, lds, s, f, out, a, r);
+        else hipLaunchKernelGGL((k17_row_kernel<S, V, EVEN, false, false, SPLIT, true>), grid, block, lds, s, f, out, a, r);
         return;
     }
-    if (mask && macro) hipLaunchKernelGGL((k17_row_kernel<S, V, EVEN, true, true, BUF>), grid, block, lds, s, f, f, a, r);
-    else if (macro) hipLaunchKernelGGL((k17_row_kernel<S, V, EVEN, false, true, BUF>), grid, block, lds, s, f, f, a, r);
-    else if (BUF && xcd_rows(a.nx, sizeof(S), kc.rowXcdRanges)) {
-        if (mask) hipLaunchKernelGGL((k17_row_kernel<S, V, EVEN, true, false, BUF, false, true>), grid, block, lds, s, f, f, a, r);
-        else hipLaunchKernelGGL((k17_row_kernel<S, V, EVEN, false, false, BUF, false, true>), grid, block, lds, s, f, f, a, r);
+    if (mask && macro) hipLaunchKernelGGL((k17_row_kernel<S, V, EVEN, true, true, SPLIT>), grid, block, lds, s, f, f, a, r);
+    else if (macro) hipLaunchKernelGGL((k17_row_kernel<S, V, EVEN, false, true, SPLIT>), grid, block, lds, s, f, f, a, r);
+    else if (SPLIT && xcd_rows(a.nx, sizeof(S), kc.rowXcdRanges)) {
+        if (mask) hipLaunchKernelGGL((k17_row_kernel<S, V, EVEN, true, false, SPLIT, false, true>), grid, block, lds, s, f, f, a, r);
+        else hipLaunchKernelGGL((k17_row_kernel<S, V, EVEN, false, false, SPLIT, false, true>), grid, block, lds, s, f, f, a, r);
     }
-    else if (mask) hipLaunchKernelGGL((k17_row_kernel<S, V, EVEN, true, false, BUF>), grid, block, lds, s, f, f, a, r);
-    else hipLaunchKernelGGL((k17_row_kernel<S, V, EVEN, false, false, BUF>), grid, block, lds, s, f, f, a, r);
+    else if (mask) hipLaunchKernelGGL((k17_row_kernel<S, V, EVEN, true, false, SPLIT>), grid, block, lds, s, f, f, a, r);
+    else hipLaunchKernelGGL((k17_row_kernel<S, V, EVEN, false, false, SPLIT>), grid, block, lds, s, f, f, a, r);
 }
 
 template <class S, int V, bool EVEN>
 static void launch_row_t(const BoxArgs& a, const K17Rates& r, bool mask, bool macro, S* f, S* out, uint64_t ws,
                          const vf_kernel_choice& kc, hipStream_t s)
 {
-    // the larger descriptor spans kRowSplit slots; buffer offsets are 32-bit
-    if (slots_fit_buffers(a.N, sizeof(S)) && kc.rowAddressing != VF_ROW_ADDRESSING_GLOBAL)
-        launch_row_b<S, V, EVEN, true>(a, r, mask, macro, f, out, ws, kc, s);
-    else
-        launch_row_b<S, V, EVEN, false>(a, r, mask, macro, f, out, ws, kc, s);
+    // a descriptor's slots lie within 32-bit buffer offsets. Four descriptors against the 64-bit form,
+    // FP32 512^3: 5.02 against 5.58 ms
+    const bool global = kc.rowAddressing == VF_ROW_ADDRESSING_GLOBAL;
+    const bool wide = kc.rowAddressing == VF_ROW_ADDRESSING_BUFFER_WIDE;
+    if (!global && !wide && slots_fit_buffers(a.N, sizeof(S))) launch_row_b<S, V, EVEN, kRowSplit>(a, r, mask, macro, f, out, ws, kc, s);
+    else if (!global && (uint64_t)kRowSplitWide * a.N * sizeof(S) <= 0xffffffffull)
+        launch_row_b<S, V, EVEN, kRowSplitWide>(a, r, mask, macro, f, out, ws, kc, s);
+    else launch_row_b<S, V, EVEN, 0>(a, r, mask, macro, f, out, ws, kc, s);
 }
 
 // Nodes per lane of the row kernel the dense-box collision takes for this box, or 0 when it

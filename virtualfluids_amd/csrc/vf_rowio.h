@@ -27,6 +27,7 @@ __host__ __device__ constexpr int shifted_index(int d)
 // the rest from base + kRowSplit slots, so 32-bit offsets reach every slot while kRowSplit
 // slots span less than 4 GiB.
 constexpr int kRowSplit = 14;
+constexpr int kRowSplitWide = 7; // four descriptors, for lattices whose 14 slots reach beyond 4 GiB
 
 // host: whether kRowSplit slots of N elements of elemBytes lie within 32-bit buffer offsets
 inline bool slots_fit_buffers(uint64_t N, size_t elemBytes) { return kRowSplit * N * elemBytes <= 0xffffffffull; }
