@@ -479,17 +479,21 @@ template <class S> static int row_width(int nx, const vf_kernel_choice& kc)
 
 // Resident workgroups per CU for the row kernel (0: as many as registers allow). The FP32
 // kernel moves the most bytes per instruction and runs best with few resident rows when it
-// streams from HBM: at 256^3 on MI355X, 8 resident 4-wave workgroups per CU give 5.72 TB/s, 3-4
-// give 5.84-5.86 and 2 give 5.92-5.93 (fewer concurrent direction streams per memory channel);
-// one gives 3.8. A working set that fits the 256 MB infinity cache is latency-bound instead
-// and takes every wave. The 16-bit kernels are bound by VALU issue and need every wave they can
-// get. The cap is imposed by reserving LDS at launch; kernelChoice.rowWorkgroupsPerCU pins it.
+// streams from HBM (fewer concurrent direction streams per memory channel), as long as at least
+// eight waves are resident: measured on MI355X, us per step, rows of one wave (64 x 300 x 300) 532
+// at 2, 311 at 4, 232 at 8, 238 without a cap; of two (128 x 300 x 300) 588 at 2, 438 at 4, 457
+// without; of four (256 x 200 x 200) 396 at 2, 389 at 4, 404 without; of eight (512^3) 6394 at 1, 5021
+// at 2, 5901 at 4, 5857 without. A working set that fits the 256 MB infinity cache is
+// latency-bound instead and takes every wave. The 16-bit kernels are bound by VALU issue and need
+// every wave they can get. The cap is imposed by reserving LDS at launch;
+// kernelChoice.rowWorkgroupsPerCU pins it.
 constexpr uint64_t kCacheResidentBytes = 256ull << 20;
-template <class S, int V, int SPLIT> static int row_wgs_per_cu(uint64_t workingSet, const vf_kernel_choice& kc)
+template <class S, int V, int SPLIT> static int row_wgs_per_cu(uint64_t workingSet, int waves, const vf_kernel_choice& kc)
 {
     if (kc.rowWorkgroupsPerCU != 0) return kc.rowWorkgroupsPerCU < 0 ? 0 : kc.rowWorkgroupsPerCU;
     const bool streams = workingSet > kCacheResidentBytes;
-    return (Codec<S>::storage == VF_STORAGE_FP32 && V == 1 && SPLIT > 0 && streams) ? 2 : 0;
+    if (Codec<S>::storage != VF_STORAGE_FP32 || V > 2 || SPLIT == 0 || !streams) return 0;
+    return waves == 1 ? 8 : waves <= 4 ? 4 : 2;
 }
 
 // out: null for the in-place step, else the buffer the out-of-place step writes
@@ -499,7 +503,7 @@ static void launch_row_b(const BoxArgs& a, const K17Rates& r, bool mask, bool ma
 {
     dim3 grid(a.ny, a.nz);
     dim3 block(((a.nx / V + 63) / 64) * 64); // whole waves; lanes beyond the row idle
-    const size_t lds = lds_reserve_for(row_wgs_per_cu<S, V, SPLIT>(ws, kc));
+    const size_t lds = lds_reserve_for(row_wgs_per_cu<S, V, SPLIT>(ws, (int)block.x / 64, kc));
     if (out) {
         if (mask) hipLaunchKernelGGL((k17_row_kernel<S, V, EVEN, true, false, SPLIT, true>), grid, block, lds, s, f, out, a, r);
         else hipLaunchKernelGGL((k17_row_kernel<S, V, EVEN, false, false, SPLIT, true>), grid, block, lds, s, f, out, a, r);
@@ -537,6 +541,8 @@ static void launch_row_t(const BoxArgs& a, const K17Rates& r, bool mask, bool ma
 // step); rows of other lengths leave lanes idle and start inside cache lines, and there the
 // node kernel, whose workgroups take consecutive nodes of a plane, leads (258 x 130 x 130 FP16
 // 87 against 153 us, FP32 203 against 264 us; measured on MI355X, one lattice stepped alone).
+// FP32 rows of a single wave are the exception: a workgroup of one wave shares nothing, and the
+// node kernel leads (64 x 300 x 300 225 against 232 us).
 // A pinned row kernel or row width keeps the row kernel.
 template <class S> static int box_row_width(const vf_lbm_parameter& p)
 {
@@ -549,7 +555,9 @@ template <class S> static int box_row_width(const vf_lbm_parameter& p)
     const uint64_t ws = p.workingSetBytes ? p.workingSetBytes : 27 * p.numberOfNodes * sizeof(S);
     const bool pinned = kc.boxKernel == VF_BOX_KERNEL_ROW || kc.rowWidth != 0;
     if (pinned) return V;
-    return (ws <= kCacheResidentBytes || (p.nx / V) % 64 != 0) ? 0 : V;
+    if (ws <= kCacheResidentBytes || (p.nx / V) % 64 != 0) return 0;
+    if (sizeof(S) == 4 && p.nx / V == 64) return 0;
+    return V;
 }
 
 // The row kernel when box_row_width selects it. Returns false when it does not apply.
