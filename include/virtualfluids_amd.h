@@ -277,6 +277,19 @@ int vf_VelocityInterpolatedCompressible(const vf_lbm_parameter* para, const vf_q
 /* VelocityWithPressureInterpolatedCompressible (Velocity.cu:109-129) */
 int vf_VelocityWithPressureInterpolatedCompressible(const vf_lbm_parameter* para, const vf_q_boundary_conditions* bc,
                                                     void* stream);
+/* One of the two above followed by vf_NoSlipInterpolatedCompressible, in one launch with the same
+ * values, for lists of which neither writes a cell that the other reads or writes: no link both
+ * have in common, and no link of one that leads to a node of the other. */
+int vf_VelocityAndNoSlipInterpolatedCompressible(const vf_lbm_parameter* para, const vf_q_boundary_conditions* velocity,
+                                                 const vf_q_boundary_conditions* noslip, void* stream);
+int vf_VelocityWithPressureAndNoSlipInterpolatedCompressible(const vf_lbm_parameter* para,
+                                                             const vf_q_boundary_conditions* velocity,
+                                                             const vf_q_boundary_conditions* noslip, void* stream);
+/* *independent: whether that holds for two lists of a dense box (host arrays: k[n], q27 [27 n],
+ * direction-major; a link is one with 0 <= q <= 1, the box wraps around). VF_ERR_INVALID_ARGUMENT for
+ * a node outside the box or missing arrays. */
+int vf_bc_lists_independent(int32_t nx, int32_t ny, int32_t nz, uint32_t na, const int32_t* ka, const double* qa,
+                            uint32_t nb, const int32_t* kb, const double* qb, int32_t* independent);
 /* PressureNonEquilibriumCompressible, pre-collision, after the parity swap
  * (src/gpu/core/BoundaryConditions/Pressure/Pressure.cu:63-81) */
 int vf_PressureNonEquilibriumCompressible(const vf_lbm_parameter* para, const vf_q_boundary_conditions* bc,
@@ -492,13 +505,15 @@ enum vf_launch_kind {
     VF_LAUNCH_BOX = 0,             /* vf_k17_run_box(level, collisionTemplate) */
     VF_LAUNCH_BOX_BOUNCE_BACK = 1, /* vf_k17_run_box_bounce_back(level, collisionTemplate, bounceBack) */
     VF_LAUNCH_INDICES = 2,         /* vf_k17_run_on_indices over the level's fluid nodes, collisionTemplate */
-    VF_LAUNCH_BC = 3,              /* bc(level, list) */
+    VF_LAUNCH_BC = 3,              /* bc(level, list), or pair(level, list, list2) where pair is set */
     VF_LAUNCH_SWAP = 4,            /* flips level->isEvenTimestep (no launch) */
     VF_LAUNCH_COARSE_TO_FINE = 5,  /* vf_ScaleCoarseToFineCompressible(level, fine, cells, offsets) */
     VF_LAUNCH_FINE_TO_COARSE = 6   /* vf_ScaleFineToCoarseCompressible(level, fine, cells, offsets) */
 };
 /* The launchers of one boundary-condition list */
 typedef int (*vf_bc_launcher)(const vf_lbm_parameter* para, const vf_q_boundary_conditions* bc, void* stream);
+typedef int (*vf_bc_pair_launcher)(const vf_lbm_parameter* para, const vf_q_boundary_conditions* velocity,
+                                   const vf_q_boundary_conditions* noslip, void* stream);
 /* All pointers are host pointers, read when the sequence runs; fields a kind does not use are
  * ignored. */
 typedef struct vf_launch {
@@ -511,6 +526,8 @@ typedef struct vf_launch {
     const vf_post_bounce_back* bounceBack;
     const vf_interpolation_cells* cells;
     const vf_interpolation_cell_neighbor* offsets; /* or NULL */
+    vf_bc_pair_launcher pair;                      /* VF_LAUNCH_BC of two lists: pair(level, list, list2) */
+    const vf_q_boundary_conditions* list2;
 } vf_launch;
 
 int vf_run_launches(const vf_launch* list, uint32_t n, uint32_t repeats, void* stream);

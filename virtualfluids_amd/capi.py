@@ -151,6 +151,8 @@ class Launch(ctypes.Structure):
         ("bounceBack", ctypes.POINTER(PostBounceBack)),
         ("cells", ctypes.POINTER(InterpolationCells)),
         ("offsets", ctypes.POINTER(InterpolationCellNeighbor)),
+        ("pair", _vp),
+        ("list2", ctypes.POINTER(QBoundaryConditions)),
     ]
 
 
@@ -171,6 +173,9 @@ SIGNATURES = {
     "vf_k17_run_box_into": [_P, _vp, _vp],
     "vf_k17_run_box_bounce_back": [_P, ctypes.c_int32, ctypes.POINTER(PostBounceBack), _vp],
     "vf_NoSlipBounceBack": [_P, _Q, _vp],
+    "vf_bc_lists_independent": [ctypes.c_int32] * 3 + [ctypes.c_uint32, _vp, _vp] * 2 + [ctypes.POINTER(ctypes.c_int32)],
+    "vf_VelocityAndNoSlipInterpolatedCompressible": [_P, _Q, _Q, _vp],
+    "vf_VelocityWithPressureAndNoSlipInterpolatedCompressible": [_P, _Q, _Q, _vp],
     "vf_NoSlipInterpolatedCompressible": [_P, _Q, _vp],
     "vf_VelocityBounceBack": [_P, _Q, _vp],
     "vf_VelocityInterpolatedCompressible": [_P, _Q, _vp],

@@ -47,6 +47,18 @@ class LaunchList:
         self._add(capi.LAUNCH_BC, level, bc=ctypes.cast(getattr(capi.load(), fn_name), ctypes.c_void_p),
                   list=ctypes.pointer(bc_struct))
 
+    def bc_pair(self, level, fn_name: str, velocity_struct, noslip_struct):
+        self._add(capi.LAUNCH_BC, level, pair=ctypes.cast(getattr(capi.load(), fn_name), ctypes.c_void_p),
+                  list=ctypes.pointer(velocity_struct), list2=ctypes.pointer(noslip_struct))
+
+    def post_groups(self, level, groups):
+        """The post-collision launches (simulation.paired_launches)."""
+        for fn, bcs in groups:
+            if len(bcs) == 2:
+                self.bc_pair(level, fn, *(bc.struct for _, bc in bcs))
+            else:
+                self.bc(level, fn, bcs[0][1].struct)
+
     def swap(self, level):
         self._add(capi.LAUNCH_SWAP, level)
 
