@@ -155,21 +155,20 @@ class DeviceInterfaceCells:
         """vf_interpolation_sources of the coarse cells (corner q of cell i: q's bits step +x, +y,
         +z through the grid's neighbour arrays), built once: (struct, workspace floats)."""
         if self._sources is None:
-            base = np.asarray(self.host.coarse, dtype=np.int64)
             corners = np.empty((self.n, 8), dtype=np.int64)
-            for q in range(8):
-                k = base.copy()
-                if q & 1:
-                    k = grid.nbx[k].astype(np.int64)
-                if q & 2:
-                    k = grid.nby[k].astype(np.int64)
-                if q & 4:
-                    k = grid.nbz[k].astype(np.int64)
-                corners[:, q] = k
-            lanes_flat = corners.reshape(-1)  # entry 8 i + q
-            order = np.argsort(lanes_flat, kind="stable")
-            nodes, first_idx = np.unique(lanes_flat[order], return_index=True)
-            first = np.append(first_idx, order.size).astype(np.uint32)
+            corners[:, 0] = np.asarray(self.host.coarse, dtype=np.int64)
+            for q in range(1, 8):  # the corner without q's highest bit, one step further
+                step = grid.nbx if q == 1 else grid.nby if q < 4 else grid.nbz
+                corners[:, q] = step[corners[:, q - (1 if q == 1 else 2 if q < 4 else 4)]]
+            # sorted by node, then by entry 8 i + q: one sort of the pairs (190 000 of
+            # them 3 ms, an index sort 25 ms on the same core)
+            entries = 8 * self.n
+            bits = entries.bit_length()
+            key = np.sort(corners.reshape(-1) << bits | np.arange(entries))
+            node, order = key >> bits, key & ((1 << bits) - 1)
+            starts = np.flatnonzero(np.diff(node, prepend=-1))
+            nodes = node[starts]
+            first = np.append(starts, order.size).astype(np.uint32)
 
             def u32(a):
                 return torch.from_numpy(np.ascontiguousarray(a, dtype=np.uint32).view(np.int32)).to(self.device)
