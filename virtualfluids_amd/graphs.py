@@ -2,7 +2,9 @@
 
 A long run of short kernels is bound by the host launching them; capturing the steps in HIP
 graphs and replaying them takes the host out of the loop. No counterpart in the reference (its
-time loop launches every kernel from the host).
+time loop launches every kernel from the host). The package's own runs enqueue their launches from a
+native loop instead (launches.py), which has nothing to capture; this is for programs with steps of
+their own.
 """
 from __future__ import annotations
 
