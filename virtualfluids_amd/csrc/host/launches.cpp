@@ -149,7 +149,7 @@ extern "C" int vf_bc_lists_independent(int32_t nx, int32_t ny, int32_t nz, uint3
     *independent = 1;
     if (na == 0 || nb == 0) return VF_OK;
     try {
-        *independent = lists_independent({nx, ny, nz}, {na, ka, qa, {}}, {nb, kb, qb, {}}) ? 1 : 0;
+        *independent = lists_independent({nx, ny, nz}, {na, ka, qa}, {nb, kb, qb}) ? 1 : 0;
         return VF_OK;
     } catch (const std::bad_alloc&) {
         set_last_error("bc_lists_independent: out of memory");
