@@ -406,10 +406,11 @@ void launch_scalar_b(const AdjBoxArgs& a, const K17Rates& r, const S* f, float* 
 }
 template <class S, bool EVEN>
 void launch_scalar(const AdjBoxArgs& a, const K17Rates& r, const S* f, float* lam, bool mask, bool shift, dim3 grid,
-                   hipStream_t s, bool xcd = false)
+                   hipStream_t s, const vf_kernel_choice& kc, bool xcd = false)
 {
     // the buffer form needs kRowSplit slots of the adjoint (the larger element) within 32-bit offsets
-    if (slots_fit_buffers(a.N, sizeof(float))) launch_scalar_b<S, EVEN, true>(a, r, f, lam, mask, shift, grid, s, xcd);
+    if (slots_fit_buffers(a.N, sizeof(float)) && kc.rowAddressing != VF_ROW_ADDRESSING_GLOBAL)
+        launch_scalar_b<S, EVEN, true>(a, r, f, lam, mask, shift, grid, s, xcd);
     else launch_scalar_b<S, EVEN, false>(a, r, f, lam, mask, shift, grid, s, xcd);
 }
 
@@ -452,14 +453,15 @@ void launch_box(const vf_lbm_parameter& p, float* lam, float* shift, float* padj
         AdjBoxArgs at = a;
         at.x0 = rowEnd;
         const uint64_t n = (uint64_t)(p.nx - rowEnd) * p.ny * p.nz;
-        launch_scalar<S, EVEN>(at, r, f, lam, mask, shift != nullptr, dim3((unsigned)((n + kAdjBlock - 1) / kAdjBlock)), s);
+        launch_scalar<S, EVEN>(at, r, f, lam, mask, shift != nullptr, dim3((unsigned)((n + kAdjBlock - 1) / kAdjBlock)), s,
+                               kc);
         return;
     }
     static_assert(kAdjBlock == kPlaneBlock, "the scalar adjoint kernel takes plane-flat workgroups");
     // XCD block ranges only where pinned: the adjoint's three streams per direction ran slower
     // with them (sphere channel 125 -> 151 us, 258 x 130 x 130 FP16 227 -> 284 us)
     launch_scalar<S, EVEN>(a, r, f, lam, mask, shift != nullptr, dim3(plane_blocks(p.nx, p.ny), p.nz), s,
-                           kc.rowXcdRanges == 1);
+                           kc, kc.rowXcdRanges == 1);
 }
 
 template <class S, bool EVEN>

@@ -617,6 +617,12 @@ template <class S> static NodeLaunch node_launch(const vf_lbm_parameter& p, bool
     return {xcd, lds_reserve_for(cap)};
 }
 
+// Buffer descriptors where 14 slots lie within 4 GiB, unless 64-bit addresses are pinned
+template <class S> static bool node_buffers(const vf_lbm_parameter& p)
+{
+    return slots_fit_buffers(p.numberOfNodes, sizeof(S)) && p.kernelChoice.rowAddressing != VF_ROW_ADDRESSING_GLOBAL;
+}
+
 template <class S, bool EVEN, bool BUF>
 static void launch_node_b(const vf_lbm_parameter& p, const BoxArgs& a, const K17Rates& r, bool macro, hipStream_t s)
 {
@@ -640,7 +646,7 @@ static void launch_box_t(const vf_lbm_parameter& p, bool macro, hipStream_t s)
               p.porosity, make_plane_div(p.nx, p.ny)};
     const K17Rates r = make_k17_rates(p);
     if (try_launch_row<S, EVEN>(p, a, r, macro, nullptr, s)) return;
-    if (slots_fit_buffers(a.N, sizeof(S))) launch_node_b<S, EVEN, true>(p, a, r, macro, s);
+    if (node_buffers<S>(p)) launch_node_b<S, EVEN, true>(p, a, r, macro, s);
     else launch_node_b<S, EVEN, false>(p, a, r, macro, s);
 }
 
@@ -668,7 +674,7 @@ static bool launch_box_bb_t(const vf_lbm_parameter& p, bool macro, const FusedBB
     BoxArgs a{p.numberOfNodes, p.nx, p.ny, p.nz, p.fluidMask, p.rho, p.velocityX, p.velocityY, p.velocityZ,
               p.porosity, make_plane_div(p.nx, p.ny)};
     const K17Rates r = make_k17_rates(p);
-    if (slots_fit_buffers(a.N, sizeof(S))) launch_node_bb_b<S, EVEN, true>(p, a, r, macro, bb, s);
+    if (node_buffers<S>(p)) launch_node_bb_b<S, EVEN, true>(p, a, r, macro, bb, s);
     else launch_node_bb_b<S, EVEN, false>(p, a, r, macro, bb, s);
     return true;
 }
@@ -692,7 +698,7 @@ template <class S, bool EVEN>
 static void launch_indexed_t(const vf_lbm_parameter& p, const uint32_t* idx, uint32_t n, bool macro, bool force,
                              hipStream_t s)
 {
-    if (slots_fit_buffers(p.numberOfNodes, sizeof(S))) launch_indexed_b<S, EVEN, true>(p, idx, n, macro, force, s);
+    if (node_buffers<S>(p)) launch_indexed_b<S, EVEN, true>(p, idx, n, macro, force, s);
     else launch_indexed_b<S, EVEN, false>(p, idx, n, macro, force, s);
 }
 
@@ -741,7 +747,7 @@ template <class S, bool EVEN> struct BoxIntoL {
                   make_plane_div(p.nx, p.ny)};
         const K17Rates r = make_k17_rates(p);
         if (try_launch_row<S, EVEN>(p, a, r, false, static_cast<S*>(out), s)) return;
-        if (slots_fit_buffers(a.N, sizeof(S))) launch_into_b<S, EVEN, true>(p, a, r, static_cast<S*>(out), s);
+        if (node_buffers<S>(p)) launch_into_b<S, EVEN, true>(p, a, r, static_cast<S*>(out), s);
         else launch_into_b<S, EVEN, false>(p, a, r, static_cast<S*>(out), s);
     }
 };

@@ -346,7 +346,7 @@ class Simulation:
     def _post_launches(self, steps: int = 1):
         """The launches of the groups for `steps` more steps: paired_launches once 512 steps have been
         asked for, until then a launch per group. A shared launch saves 2 to 4 us a step, and finding out
-        whether the lists allow it takes up to 1.5 ms of host time (85 000 nodes)."""
+        whether the lists allow it takes about 1 ms of host time (85 000 nodes)."""
         groups = self._post_groups()
         if self._paired is not None and self._paired[0] is groups:
             return self._paired[1]
