@@ -1,0 +1,41 @@
+"""When a velocity and a no-slip list may share a launch (bc_post_pair_kernel): judged on the values
+that the kernels see, at a cost that follows the lists."""
+from types import SimpleNamespace
+
+import numpy as np
+import pytest
+
+from virtualfluids_amd.grid import CX, CY, CZ
+from virtualfluids_amd.simulation import _independent
+
+
+def _grid(size, lists):
+    nx, ny, nz = size
+    return SimpleNamespace(nx=nx, ny=ny, nz=nz, N=nx * ny * nz, bcs=lists)
+
+
+def _list(k, links):
+    """Nodes k; links: [(direction, entry, distance)]."""
+    q = np.full((27, len(k)), -1.0)
+    for d, i, value in links:
+        q[d, i] = value
+    return SimpleNamespace(k=np.asarray(k, dtype=np.int32), n=len(k), q27=q.ravel())
+
+
+# the kernels read FP32: 1 + 1e-9 rounds to 1 and -1e-60 to -0, links both; 1 + 1e-6 and -1e-30 stay outside
+@pytest.mark.parametrize("q,link", [(1.0, True), (1.0 + 1e-9, True), (-1e-60, True), (1.0 + 1e-6, False),
+                                    (-1e-30, False), (float("nan"), False), (-1.0, False)])
+@pytest.mark.parametrize("swap", [False, True])
+def test_links_are_those_of_the_fp32_distances(q, link, swap):
+    size = (8, 8, 8)
+    at = 3 + 8 * (3 + 8 * 3)
+    for d in (1, 7, 26):
+        to = at + CX[d] + 8 * (CY[d] + 8 * CZ[d])
+        lists = [_list([at], [(d, 0, q)]), _list([to, 0], [])]
+        if swap:
+            lists.reverse()
+        assert _independent(_grid(size, {"a": lists[0], "b": lists[1]}), "a", "b") == (not link)
+        shared = [_list([at], [(d, 0, q)]), _list([at], [(d, 0, 0.5)])]
+        if swap:
+            shared.reverse()
+        assert _independent(_grid(size, {"a": shared[0], "b": shared[1]}), "a", "b") == (not link)

@@ -56,7 +56,8 @@ struct HostList {
     const int32_t* k;
     const double* q;
     const double* at(int d, uint32_t i) const { return q + (uint64_t)d * n + i; }
-    static bool link(const double* v) { return *v >= 0.0 && *v <= 1.0; }
+    // as the kernels see it, which read the distances in FP32 (1 + 1e-9 is a link there)
+    static bool link(const double* v) { const float q = (float)*v; return q >= 0.0f && q <= 1.0f; }
 };
 
 // The shorter list's nodes (a) in a table over their extent; only nodes of the other within a node
