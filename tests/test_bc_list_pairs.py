@@ -39,3 +39,17 @@ def test_links_are_those_of_the_fp32_distances(q, link, swap):
         if swap:
             shared.reverse()
         assert _independent(_grid(size, {"a": shared[0], "b": shared[1]}), "a", "b") == (not link)
+
+
+def test_memory_follows_the_lists():
+    """A few nodes in opposite corners of a box of 10^9 nodes: nothing of the box's size is held."""
+    import resource
+
+    size = (1000, 1000, 1000)
+    N = 10 ** 9
+    a, b = _list([0, N - 1], [(1, 0, 0.5)]), _list([5, N // 2, N - 7], [(2, 1, 0.5)])
+    before = resource.getrusage(resource.RUSAGE_SELF).ru_maxrss
+    assert _independent(_grid(size, {"a": a, "b": b}), "a", "b")
+    assert resource.getrusage(resource.RUSAGE_SELF).ru_maxrss - before < 64 * 1024  # KiB
+    b.k[0] = 1  # where a's first node has its link
+    assert not _independent(_grid(size, {"a": a, "b": b}), "a", "b")

@@ -55,13 +55,23 @@ struct HostList {
     uint32_t n;
     const int32_t* k;
     const double* q;
-    const double* at(int d, uint32_t i) const { return q + (uint64_t)d * n + i; }
-    // as the kernels see it, which read the distances in FP32 (1 + 1e-9 is a link there)
-    static bool link(const double* v) { const float q = (float)*v; return q >= 0.0f && q <= 1.0f; }
+    // bit d: a link along d, as the kernels see it, which read the distances in FP32 (1 + 1e-9 is a
+    // link there)
+    uint32_t links(uint32_t i) const
+    {
+        uint32_t m = 0;
+        for (int d = 1; d < 27; ++d) {
+            const float v = (float)q[(uint64_t)d * n + i];
+            m |= (v >= 0.0f && v <= 1.0f ? 1u : 0u) << d;
+        }
+        return m;
+    }
 };
 
-// The shorter list's nodes (a) in a table over their extent; only nodes of the other within a node
-// of that extent (an inflow face: the walls' rim) look their neighbourhood up.
+// The shorter list's nodes (a) in a hash table, and the x, y and z planes that hold any of them; only
+// nodes of the other list beside such planes (an inflow face: the walls' rim) look their
+// neighbourhood up. Memory and time follow the lists, not the box: two opposite faces of 384^3 and its
+// walls (874 000 nodes) 231 -> 14 ms and no 230 MB table.
 bool lists_independent(const int32_t (&size)[3], HostList a, HostList b)
 {
     if (a.n > b.n) std::swap(a, b);
@@ -78,57 +88,44 @@ bool lists_independent(const int32_t (&size)[3], HostList a, HostList b)
         }
         last = k;
     };
-    int32_t c[3] = {}, lo[3] = {INT32_MAX, INT32_MAX, INT32_MAX}, hi[3] = {-1, -1, -1};
+    int bits = 4;
+    while ((1ull << bits) < 2ull * a.n) ++bits;
+    const uint32_t mask = (uint32_t)((1ull << bits) - 1);
+    const auto hash = [bits](int32_t k) { return (uint32_t)(((uint64_t)(uint32_t)k * 0x9e3779b97f4a7c15ull) >> (64 - bits)); };
+    std::vector<uint32_t> table((size_t)mask + 1, 0); // index + 1 in a
+    std::vector<uint8_t> held[3], beside[3];          // planes that hold nodes of a; those and the ones beside
+    for (int x = 0; x < 3; ++x) held[x].assign(size[x], 0);
+    int32_t c[3] = {};
     for (uint32_t i = 0; i < a.n; ++i) {
         coordinates(a.k[i], c);
-        for (int x = 0; x < 3; ++x) {
-            lo[x] = std::min(lo[x], c[x]);
-            hi[x] = std::max(hi[x], c[x]);
-        }
+        for (int x = 0; x < 3; ++x) held[x][c[x]] = 1;
+        uint32_t h = hash(a.k[i]);
+        while (table[h]) h = (h + 1) & mask;
+        table[h] = i + 1;
     }
-    const int64_t ex = hi[0] - lo[0] + 1, ey = hi[1] - lo[1] + 1, ez = hi[2] - lo[2] + 1;
-    std::vector<uint32_t> table((size_t)(ex * ey * ez), 0); // index + 1 in a
-    const auto place = [&](const int32_t (&v)[3]) {
-        return (size_t)(v[0] - lo[0] + ex * (v[1] - lo[1] + ey * (v[2] - lo[2])));
-    };
-    for (uint32_t i = 0; i < a.n; ++i) {
-        coordinates(a.k[i], c);
-        table[place(c)] = i + 1;
+    const auto wrapped = [&size](int x, int32_t v) { return v < 0 ? size[x] - 1 : v >= size[x] ? 0 : v; };
+    for (int x = 0; x < 3; ++x) {
+        beside[x] = held[x];
+        for (int32_t v = 0; v < size[x]; ++v)
+            if (held[x][wrapped(x, v - 1)] || held[x][wrapped(x, v + 1)]) beside[x][v] = 1;
     }
-    // lowest and highest coordinate beside the extent; a box that wraps around has others as well
-    const auto beside = [&](int x, int32_t v) {
-        return (v >= lo[x] - 1 && v <= hi[x] + 1) || (lo[x] == 0 && v == size[x] - 1) || (hi[x] == size[x] - 1 && v == 0);
-    };
-    // the distances to look at lie a cache line apart each: fetched ahead, tested afterwards
-    std::vector<const double*> alone;                          // no link may be here
-    std::vector<std::pair<const double*, const double*>> both; // not both may be links
-    const auto fetch = [](const double* v) {
-        __builtin_prefetch(v);
-        return v;
-    };
     for (uint32_t i = 0; i < b.n; ++i) {
         coordinates(b.k[i], c);
-        if (!beside(0, c[0]) || !beside(1, c[1]) || !beside(2, c[2])) continue;
+        if (!beside[0][c[0]] || !beside[1][c[1]] || !beside[2][c[2]]) continue;
+        const uint32_t links = b.links(i);
         for (int d = 0; d < 27; ++d) {
-            int32_t v[3] = {c[0] + vfa::cx(d), c[1] + vfa::cy(d), c[2] + vfa::cz(d)};
-            bool in = true;
-            for (int x = 0; x < 3; ++x) {
-                v[x] = v[x] < 0 ? size[x] - 1 : v[x] >= size[x] ? 0 : v[x];
-                in = in && v[x] >= lo[x] && v[x] <= hi[x];
-            }
-            const uint32_t j = in ? table[place(v)] : 0;
-            if (j == 0) continue;
-            if (d == 0) {
-                for (int e = 1; e < 27; ++e) both.emplace_back(fetch(a.at(e, j - 1)), fetch(b.at(e, i)));
-            } else {
-                alone.push_back(fetch(b.at(d, i)));
-                alone.push_back(fetch(a.at(vfa::inv(d), j - 1)));
+            const int32_t v[3] = {wrapped(0, c[0] + vfa::cx(d)), wrapped(1, c[1] + vfa::cy(d)), wrapped(2, c[2] + vfa::cz(d))};
+            if (!held[0][v[0]] || !held[1][v[1]] || !held[2][v[2]]) continue;
+            const int32_t k = v[0] + size[0] * (v[1] + size[1] * v[2]);
+            for (uint32_t h = hash(k); table[h]; h = (h + 1) & mask) {
+                const uint32_t j = table[h] - 1;
+                if (a.k[j] != k) continue;
+                // a link in common, or one of either that leads to the other's node
+                if (d == 0 ? (links & a.links(j)) != 0 : (links >> d & 1u) || (a.links(j) >> vfa::inv(d) & 1u)) return false;
             }
         }
     }
-    return std::none_of(alone.begin(), alone.end(), HostList::link) &&
-           std::none_of(both.begin(), both.end(),
-                        [](const auto& p) { return HostList::link(p.first) && HostList::link(p.second); });
+    return true;
 }
 
 } // namespace
