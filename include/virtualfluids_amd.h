@@ -287,8 +287,9 @@ int vf_VelocityWithPressureAndNoSlipInterpolatedCompressible(const vf_lbm_parame
                                                              const vf_q_boundary_conditions* velocity,
                                                              const vf_q_boundary_conditions* noslip, void* stream);
 /* *independent: whether that holds for two lists of a dense box (host arrays: k[n], q27 [27 n],
- * direction-major; a link is one with 0 <= q <= 1 in FP32, the box wraps around). VF_ERR_INVALID_ARGUMENT for
- * a node outside the box or missing arrays. */
+ * direction-major; a link is one with 0 <= q <= 1 in FP32, the box wraps around); 0 where
+ * there is no memory for the search (8 to 16 bytes per node of the shorter list).
+ * VF_ERR_INVALID_ARGUMENT for a node outside the box or missing arrays. */
 int vf_bc_lists_independent(int32_t nx, int32_t ny, int32_t nz, uint32_t na, const int32_t* ka, const double* qa,
                             uint32_t nb, const int32_t* kb, const double* qb, int32_t* independent);
 /* PressureNonEquilibriumCompressible, pre-collision, after the parity swap

@@ -53,3 +53,29 @@ def test_memory_follows_the_lists():
     assert resource.getrusage(resource.RUSAGE_SELF).ru_maxrss - before < 64 * 1024  # KiB
     b.k[0] = 1  # where a's first node has its link
     assert not _independent(_grid(size, {"a": a, "b": b}), "a", "b")
+
+
+def test_no_memory_for_the_search_keeps_the_launches(tmp_path):
+    """Without memory for the search the lists count as dependent: two launches, and no error that a
+    run of steps would raise. In a process of its own, whose address space ends before the search's."""
+    import subprocess
+    import sys
+
+    code = """
+import ctypes, resource
+import numpy as np
+from virtualfluids_amd import capi
+lib = capi.load()
+n = 6_000_000
+k = np.arange(n, dtype=np.int32)
+q = np.zeros(27, dtype=np.float64)  # read for nodes beside the other list only: none here
+far = k + np.int32(450 * 900 ** 2)
+out = ctypes.c_int32(7)
+p = lambda a: a.ctypes.data_as(ctypes.c_void_p)
+used = int(open("/proc/self/statm").read().split()[0]) * resource.getpagesize()
+resource.setrlimit(resource.RLIMIT_AS, (used + (16 << 20), resource.RLIM_INFINITY))
+rc = lib.vf_bc_lists_independent(900, 900, 900, n, p(k), p(q), n, p(far), p(q), ctypes.byref(out))
+print(rc, out.value)
+"""
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120)
+    assert r.stdout.split() == ["0", "0"], (r.stdout, r.stderr)

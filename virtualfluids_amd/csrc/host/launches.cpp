@@ -148,9 +148,8 @@ extern "C" int vf_bc_lists_independent(int32_t nx, int32_t ny, int32_t nz, uint3
     if (na == 0 || nb == 0) return VF_OK;
     try {
         *independent = lists_independent({nx, ny, nz}, {na, ka, qa}, {nb, kb, qb}) ? 1 : 0;
-        return VF_OK;
     } catch (const std::bad_alloc&) {
-        set_last_error("bc_lists_independent: out of memory");
-        return VF_ERR_INVALID_ARGUMENT;
+        *independent = 0; // not found out: the lists keep their launches
     }
+    return VF_OK;
 }
