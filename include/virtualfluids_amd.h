@@ -292,6 +292,9 @@ int vf_VelocityWithPressureAndNoSlipInterpolatedCompressible(const vf_lbm_parame
  * VF_ERR_INVALID_ARGUMENT for a node outside the box or missing arrays. */
 int vf_bc_lists_independent(int32_t nx, int32_t ny, int32_t nz, uint32_t na, const int32_t* ka, const double* qa,
                             uint32_t nb, const int32_t* kb, const double* qb, int32_t* independent);
+/* The same from the links themselves: bit d of a node's word is set where 0 <= q_d <= 1 in FP32. */
+int vf_bc_links_independent(int32_t nx, int32_t ny, int32_t nz, uint32_t na, const int32_t* ka, const uint32_t* linksA,
+                            uint32_t nb, const int32_t* kb, const uint32_t* linksB, int32_t* independent);
 /* PressureNonEquilibriumCompressible, pre-collision, after the parity swap
  * (src/gpu/core/BoundaryConditions/Pressure/Pressure.cu:63-81) */
 int vf_PressureNonEquilibriumCompressible(const vf_lbm_parameter* para, const vf_q_boundary_conditions* bc,

@@ -79,3 +79,58 @@ print(rc, out.value)
 """
     r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120)
     assert r.stdout.split() == ["0", "0"], (r.stdout, r.stderr)
+
+
+def _channel():
+    from virtualfluids_amd.grid import sphere_channel
+    from virtualfluids_amd.lattice import Lattice
+    from virtualfluids_amd.simulation import BoundaryConditionFactory as F, Simulation
+
+    f = F()
+    f.set_velocity_boundary_condition(F.VelocityBC.VelocityInterpolatedCompressible)
+    f.set_no_slip_boundary_condition(F.NoSlipBC.NoSlipInterpolatedCompressible)
+    f.set_geometry_boundary_condition(F.NoSlipBC.NoSlipInterpolatedCompressible)
+    f.set_pressure_boundary_condition(F.PressureBC.PressureNonEquilibriumCompressible)
+    L = Lattice(sphere_channel((16, 10, 10), (6, 5, 5), 2.4, 0.04), 1.7, device="cpu")
+    return Simulation(L, f)
+
+
+def _shared_link(velocity, walls):
+    """(direction, entry of the walls) of a node in both lists, along a link of the velocity list."""
+    kv, kw = velocity.k.numpy(), walls.k.numpy()
+    node = np.intersect1d(kv, kw)[0]
+    qv = velocity.q27.numpy().reshape(27, -1)[:, np.flatnonzero(kv == node)[0]]
+    return next(d for d in range(1, 27) if 0 <= qv[d] <= 1), int(np.flatnonzero(kw == node)[0])
+
+
+@pytest.mark.parametrize("change", ["q27", "k", "pointer", "before"])
+def test_lists_changed_on_the_device_are_judged_as_they_are(change):
+    """The launch reads the device lists: what they hold decides, and a pair whose lists changed since
+    goes back to two launches (also where the lists would pass again)."""
+    sim = _channel()
+    if change == "before":
+        groups = sim._post_groups()
+    else:
+        assert [len(bcs) for _, bcs in sim._post_launches(10 ** 6)] == [2]
+        assert [len(bcs) for _, bcs in sim._post_launches(1)] == [2]
+        groups = sim.groups
+    (_, _, velocity), (_, _, walls) = groups
+    d, i = _shared_link(velocity, walls)
+    if change in ("q27", "before"):
+        walls.q27.view(27, -1)[d, i] = 0.5
+    elif change == "k":
+        walls.k.copy_(walls.k.flip(0))
+    else:
+        walls.kept = walls.q27.clone()
+        walls.struct.q27 = walls.kept.data_ptr()
+    assert [len(bcs) for _, bcs in sim._post_launches(1)] == [1, 1]
+    if change in ("q27", "before"):
+        assert [len(bcs) for _, bcs in sim._post_launches(10 ** 6)] == [1, 1]
+
+
+def test_a_given_stream_is_not_waited_for():
+    """Judging reads the lists back, which waits for the current stream's work: not in a call whose
+    caller asked for another one."""
+    sim = _channel()
+    assert [len(bcs) for _, bcs in sim._post_launches(10 ** 6, stream=object())] == [1, 1]
+    assert [len(bcs) for _, bcs in sim._post_launches(1)] == [2]

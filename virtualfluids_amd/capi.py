@@ -174,6 +174,7 @@ SIGNATURES = {
     "vf_k17_run_box_bounce_back": [_P, ctypes.c_int32, ctypes.POINTER(PostBounceBack), _vp],
     "vf_NoSlipBounceBack": [_P, _Q, _vp],
     "vf_bc_lists_independent": [ctypes.c_int32] * 3 + [ctypes.c_uint32, _vp, _vp] * 2 + [ctypes.POINTER(ctypes.c_int32)],
+    "vf_bc_links_independent": [ctypes.c_int32] * 3 + [ctypes.c_uint32, _vp, _vp] * 2 + [ctypes.POINTER(ctypes.c_int32)],
     "vf_VelocityAndNoSlipInterpolatedCompressible": [_P, _Q, _Q, _vp],
     "vf_VelocityWithPressureAndNoSlipInterpolatedCompressible": [_P, _Q, _Q, _vp],
     "vf_NoSlipInterpolatedCompressible": [_P, _Q, _vp],

@@ -51,12 +51,12 @@ extern "C" int vf_run_launches(const vf_launch* list, uint32_t n, uint32_t repea
 
 namespace {
 
-struct HostList {
+// bit d of links: a link along d, as the kernels see it, which read the distances in FP32 (1 + 1e-9 is a
+// link there)
+struct DistanceList {
     uint32_t n;
     const int32_t* k;
     const double* q;
-    // bit d: a link along d, as the kernels see it, which read the distances in FP32 (1 + 1e-9 is a
-    // link there)
     uint32_t links(uint32_t i) const
     {
         uint32_t m = 0;
@@ -67,12 +67,18 @@ struct HostList {
         return m;
     }
 };
+struct LinkList {
+    uint32_t n;
+    const int32_t* k;
+    const uint32_t* q;
+    uint32_t links(uint32_t i) const { return q[i] & ~1u; }
+};
 
 // The shorter list's nodes (a) in a hash table, and the x, y and z planes that hold any of them; only
 // nodes of the other list beside such planes (an inflow face: the walls' rim) look their
 // neighbourhood up. Memory and time follow the lists, not the box: two opposite faces of 384^3 and its
 // walls (874 000 nodes) 231 -> 14 ms and no 230 MB table.
-bool lists_independent(const int32_t (&size)[3], HostList a, HostList b)
+template <class List> bool lists_independent(const int32_t (&size)[3], List a, List b)
 {
     if (a.n > b.n) std::swap(a, b);
     // the coordinates of node k; c holds those of node `last` (lists run along x for the most part)
@@ -128,28 +134,40 @@ bool lists_independent(const int32_t (&size)[3], HostList a, HostList b)
     return true;
 }
 
+template <class List>
+int independent_in_box(int32_t nx, int32_t ny, int32_t nz, const List& a, const List& b, int32_t* independent)
+{
+    using namespace vfa;
+    const int64_t nodes = nx > 0 && ny > 0 && nz > 0 ? (int64_t)nx * ny * nz : 0;
+    const auto valid = [&](const List& l) {
+        return l.n == 0 || (l.k && l.q && std::all_of(l.k, l.k + l.n, [&](int32_t v) { return v >= 0 && v < nodes; }));
+    };
+    if (nodes == 0 || nodes > INT32_MAX || !independent || !valid(a) || !valid(b)) {
+        set_last_error("bc lists independent: missing arrays or a node outside the box");
+        return VF_ERR_INVALID_ARGUMENT;
+    }
+    *independent = 1;
+    if (a.n == 0 || b.n == 0) return VF_OK;
+    try {
+        *independent = lists_independent({nx, ny, nz}, a, b) ? 1 : 0;
+    } catch (const std::bad_alloc&) {
+        *independent = 0; // not found out: the lists keep their launches
+    }
+    return VF_OK;
+}
+
 } // namespace
 
 extern "C" int vf_bc_lists_independent(int32_t nx, int32_t ny, int32_t nz, uint32_t na, const int32_t* ka,
                                        const double* qa, uint32_t nb, const int32_t* kb, const double* qb,
                                        int32_t* independent)
 {
-    using namespace vfa;
-    const int64_t nodes = nx > 0 && ny > 0 && nz > 0 ? (int64_t)nx * ny * nz : 0;
-    const auto inside = [&](uint32_t n, const int32_t* k) {
-        return std::all_of(k, k + n, [&](int32_t v) { return v >= 0 && v < nodes; });
-    };
-    if (nodes == 0 || nodes > INT32_MAX || !independent || (na && (!ka || !qa)) || (nb && (!kb || !qb)) || !inside(na, ka) ||
-        !inside(nb, kb)) {
-        set_last_error("bc_lists_independent: missing arrays or a node outside the box");
-        return VF_ERR_INVALID_ARGUMENT;
-    }
-    *independent = 1;
-    if (na == 0 || nb == 0) return VF_OK;
-    try {
-        *independent = lists_independent({nx, ny, nz}, {na, ka, qa}, {nb, kb, qb}) ? 1 : 0;
-    } catch (const std::bad_alloc&) {
-        *independent = 0; // not found out: the lists keep their launches
-    }
-    return VF_OK;
+    return independent_in_box(nx, ny, nz, DistanceList{na, ka, qa}, DistanceList{nb, kb, qb}, independent);
+}
+
+extern "C" int vf_bc_links_independent(int32_t nx, int32_t ny, int32_t nz, uint32_t na, const int32_t* ka,
+                                       const uint32_t* linksA, uint32_t nb, const int32_t* kb, const uint32_t* linksB,
+                                       int32_t* independent)
+{
+    return independent_in_box(nx, ny, nz, LinkList{na, ka, linksA}, LinkList{nb, kb, linksB}, independent);
 }

@@ -81,6 +81,26 @@ class DeviceBC:
         s.direction = self.direction
         s.nodesAlongRows = int(nodes_along_rows(k))
 
+    def links(self):
+        """The list as the kernels read it, on the host: nodes k and per node the bitmask of its
+        links d (0 <= q_d <= 1). Waits for the current stream. None where the struct points at other
+        arrays than this list's own."""
+        s = self.struct
+        if (s.k, s.q27, s.numberOfBCnodes) != (self.k.data_ptr(), self.q27.data_ptr(), self.n):
+            return None
+        q = self.q27.reshape(27, self.n)
+        bits = torch.arange(27, dtype=torch.int32, device=q.device)[:, None]
+        links = (((q >= 0) & (q <= 1)).to(torch.int32) << bits).sum(0, dtype=torch.int32)
+        return self.k.cpu().numpy(), links.cpu().numpy().view(np.uint32)
+
+    def version(self):
+        """Changes with the nodes and link distances that the struct points at (torch's counters of
+        writes to a tensor); None where the tensors have none."""
+        if self.k.is_inference() or self.q27.is_inference():
+            return None
+        s = self.struct
+        return s.k, s.q27, s.numberOfBCnodes, self.k._version, self.q27._version
+
 
 class Lattice:
     """One grid level on the GPU."""

@@ -141,44 +141,50 @@ _PAIRED = {"vf_VelocityInterpolatedCompressible": "vf_VelocityAndNoSlipInterpola
 def paired_launches(lattice: Lattice, groups):
     """The launches of post_launch_groups as [(launcher, [(name, DeviceBC), ...])]: an interpolated
     velocity list and the no-slip list after it share a launch (two lists, the same values) where the
-    order of the two cannot matter."""
+    order of the two cannot matter. Judged on the lists that the launch will read; without device
+    lists (planning ahead of a lattice), on the grid's."""
     out = [(fn, [(name, bc)]) for name, fn, bc in groups]
     for i in range(len(out) - 1):
         (fa, a), (fb, b) = out[i], out[i + 1]
-        if fa in _PAIRED and fb == "vf_NoSlipInterpolatedCompressible" and lattice.box and _independent(
-                lattice.grid, a[0][0], b[0][0]):
+        if fa not in _PAIRED or fb != "vf_NoSlipInterpolatedCompressible" or not lattice.box:
+            continue
+        (first, bc), (second, bc2) = a[0], b[0]
+        if (_independent(lattice.grid, first, second) if bc is None or bc2 is None
+                else _device_lists_independent(lattice.grid, bc, bc2)):
             return out[:i] + [(_PAIRED[fa], a + b)] + out[i + 2:]
     return out
 
 
-def _independent(grid, first: str, second: str) -> bool:
-    """Whether two BC lists (names as in post_launch_groups) have no link in common and no link of
-    either leads to a node of the other, whose populations that link's write would change
-    (vf_bc_lists_independent)."""
+def _call_independent(fn: str, grid, a, b) -> bool:
+    """vf_bc_lists_independent or vf_bc_links_independent for a, b = (nodes, their distances or links)."""
     import ctypes
-
-    import numpy as np
 
     from . import capi
 
+    ok = ctypes.c_int32(0)
+    args = [x for k, q in (a, b) for x in (len(k), k.ctypes.data_as(ctypes.c_void_p), q.ctypes.data_as(ctypes.c_void_p))]
+    capi.call(fn, grid.nx, grid.ny, grid.nz, *args, ctypes.byref(ok))
+    return bool(ok.value)
+
+
+def _device_lists_independent(grid, first, second) -> bool:
+    """Whether two DeviceBC lists have no link in common and no link of either leads to a node of the
+    other, whose populations that link's write would change."""
+    if first.version() is None or second.version() is None:
+        return False
+    a, b = first.links(), second.links()
+    return a is not None and b is not None and _call_independent("vf_bc_links_independent", grid, a, b)
+
+
+def _independent(grid, first: str, second: str) -> bool:
+    """The same for two of a grid's lists (names as in post_launch_groups)."""
+    import numpy as np
+
     def host(name):
-        out = []
-        for part in name.split("+"):
-            h = grid.bcs[part]
-            out.append((int(h.n), np.ascontiguousarray(h.k, dtype=np.int32),
-                        np.ascontiguousarray(h.q27, dtype=np.float64)))
-        return out
+        return [(np.ascontiguousarray(h.k, dtype=np.int32), np.ascontiguousarray(h.q27, dtype=np.float64))
+                for h in (grid.bcs[part] for part in name.split("+"))]
 
-    def args(n, k, q):
-        return n, k.ctypes.data_as(ctypes.c_void_p), q.ctypes.data_as(ctypes.c_void_p)
-
-    others, ok = host(second), ctypes.c_int32(0)
-    for a in host(first):
-        for b in others:
-            capi.call("vf_bc_lists_independent", grid.nx, grid.ny, grid.nz, *args(*a), *args(*b), ctypes.byref(ok))
-            if not ok.value:
-                return False
-    return True
+    return all(_call_independent("vf_bc_lists_independent", grid, a, b) for a in host(first) for b in host(second))
 
 
 class BCEntryTables:
@@ -303,6 +309,7 @@ class Simulation:
         self.fused = None
         self.groups = None
         self._paired = None
+        self._paired_versions = ()
         self._unpaired_steps = 0
         post = [("velocity", self.velocity_fn), ("noslip", self.noslip_fn), ("geometry", self.geometry_fn)]
         post = [(name, fn) for name, fn in post if fn and lattice.bcs.get(name) is not None and lattice.bcs[name].n]
@@ -332,7 +339,7 @@ class Simulation:
 
         L = self.lattice
         L.collide(stream=stream)
-        for fn, bcs in self._post_launches():
+        for fn, bcs in self._post_launches(stream=stream):
             capi.call(fn, L.pref(), *(ctypes.byref(bc.struct) for _, bc in bcs), stream_handle(stream))
 
     def _post_groups(self):
@@ -343,31 +350,48 @@ class Simulation:
                                                             ("geometry", self.geometry_fn)])
         return self.groups
 
-    def _post_launches(self, steps: int = 1):
-        """The launches of the groups for `steps` more steps: paired_launches once 512 steps have been
-        asked for, until then a launch per group. A shared launch saves 2 to 4 us a step, and finding out
-        whether the lists allow it takes about 1 ms of host time (85 000 nodes)."""
+    def _post_launches(self, steps: int = 1, stream=None):
+        """The launches of the groups for `steps` more steps on `stream` (None: the current one):
+        paired_launches once 512 steps have been asked for, until then a launch per group. A shared
+        launch saves 2 to 4 us a step, and finding out whether the lists allow it takes about 1 ms of
+        host time (85 000 nodes) and waits for the current stream's work, so calls with a stream of
+        their own or inside a capture do not ask. A pair whose lists are written to afterwards (as torch
+        counts; a program that writes them through raw pointers takes a new Simulation) is given up, and
+        asked for again after as many steps."""
+        import torch
+
         groups = self._post_groups()
         if self._paired is not None and self._paired[0] is groups:
-            return self._paired[1]
+            if self._paired_versions == self._pair_versions(groups):
+                return self._paired[1]
+            self._paired, self._unpaired_steps = None, 0
         self._unpaired_steps += steps
-        if self._unpaired_steps < 512:
+        if (self._unpaired_steps < 512 or stream is not None
+                or self.lattice.device.type == "cuda" and torch.cuda.is_current_stream_capturing()):
             return [(fn, [(name, bc)]) for name, fn, bc in groups]
         self._paired = (groups, paired_launches(self.lattice, groups))
+        self._paired_versions = self._pair_versions(groups)
         return self._paired[1]
+
+    def _pair_versions(self, groups):
+        """What paired lists held when they were judged (DeviceBC.version); () without a pair."""
+        if len(self._paired[1]) == len(groups):
+            return ()
+        return tuple(bc.version() for _, bcs in self._paired[1] if len(bcs) == 2 for _, bc in bcs)
 
     def step(self, stream=None):
         self._launch(stream)
         self.t += 1
 
-    def add_launches(self, out, steps: int = 1):
-        """Append the launches of one step (what _launch makes) to a LaunchList, for a run of `steps`."""
+    def add_launches(self, out, steps: int = 1, stream=None):
+        """Append the launches of one step (what _launch makes) to a LaunchList, for a run of `steps` on
+        `stream`."""
         L = self.lattice
         if self.fused is not None:
             out.collide_bounce_back(L.param, self.fused.struct)
         else:
             out.collide(L.param, L.box)
-            out.post_groups(L.param, self._post_launches(steps))
+            out.post_groups(L.param, self._post_launches(steps, stream))
         out.swap(L.param)
         bc = L.bcs.get("pressure")
         if self.pressure_fn and bc is not None and bc.n:
@@ -387,7 +411,7 @@ class Simulation:
         from .launches import LaunchList
 
         out = LaunchList()
-        self.add_launches(out, steps)
+        self.add_launches(out, steps, stream)
         out.run(steps, stream)
         self.t += max(steps, 0)
         if stream is None and steps >= 3:
@@ -443,13 +467,13 @@ class MultiLevelSimulation:
         self._update(0, stream)
         self.t += 1
 
-    def _add_launches(self, level: int, out, steps: int):
+    def _add_launches(self, level: int, out, steps: int, stream):
         """Append the launches of one step of `level` (what _update makes) to a LaunchList."""
         fine = len(self.lattices) - 1
         if level != fine:
-            self._add_launches(level + 1, out, steps)
-            self._add_launches(level + 1, out, steps)
-        self.levels[level].add_launches(out, steps)
+            self._add_launches(level + 1, out, steps, stream)
+            self._add_launches(level + 1, out, steps, stream)
+        self.levels[level].add_launches(out, steps, stream)
         if level != fine:
             cf, fc = self.cells[level]
             coarse_p, fine_p = self.lattices[level].param, self.lattices[level + 1].param
@@ -472,7 +496,7 @@ class MultiLevelSimulation:
         from .launches import LaunchList
 
         out = LaunchList()
-        self._add_launches(0, out, steps)
+        self._add_launches(0, out, steps, stream)
         out.run(steps, stream)
         for level, lv in enumerate(self.levels):
             lv.t += max(steps, 0) * 2 ** level
