@@ -352,9 +352,10 @@ class Simulation:
 
     def _post_launches(self, steps: int = 1, stream=None):
         """The launches of the groups for `steps` more steps on `stream` (None: the current one):
-        paired_launches once 512 steps have been asked for, until then a launch per group. A shared
-        launch saves 2 to 4 us a step, and finding out whether the lists allow it takes about 1 ms of
-        host time (85 000 nodes) and waits for the current stream's work, so calls with a stream of
+        paired_launches once enough steps have been asked for, until then a launch per group. A shared
+        launch saves 2 to 4 us a step. Finding out whether the lists allow it takes 0.2 ms of host time
+        and 1 to 5 ns a node (87 000 nodes 0.4 ms, 615 000 1.2 ms), so it waits for 512 steps and
+        for a step per 200 nodes; it also waits for the current stream's work, so calls with a stream of
         their own or inside a capture do not ask. A pair whose lists are written to afterwards (as torch
         counts; a program that writes them through raw pointers takes a new Simulation) is given up, and
         asked for again after as many steps."""
@@ -366,7 +367,7 @@ class Simulation:
                 return self._paired[1]
             self._paired, self._unpaired_steps = None, 0
         self._unpaired_steps += steps
-        if (self._unpaired_steps < 512 or stream is not None
+        if (self._unpaired_steps < max(512, sum(bc.n for _, _, bc in groups) // 200) or stream is not None
                 or self.lattice.device.type == "cuda" and torch.cuda.is_current_stream_capturing()):
             return [(fn, [(name, bc)]) for name, fn, bc in groups]
         self._paired = (groups, paired_launches(self.lattice, groups))
