@@ -48,3 +48,16 @@ def test_every_repeat_is_enqueued(n):
     p, out = _swaps(3)
     out.run(n, STREAM)
     assert p.isEvenTimestep == (1 + 3 * n) % 2
+
+
+@pytest.mark.parametrize("n", [4.0, 3.5, 300.0, "int64", "float64"])
+def test_step_counts_need_not_be_ints(n):
+    """A count of steps computed from times (T / dt) runs until it is used up."""
+    import math
+
+    import numpy as np
+
+    n = {"int64": np.int64(300), "float64": np.float64(299.5)}.get(n, n)
+    p, out = _swaps(1)
+    out.run(n, STREAM)
+    assert p.isEvenTimestep == (1 + math.ceil(n)) % 2

@@ -9,6 +9,7 @@ us per step over 100 steps, 16.9 with graphs captured in the run, 12.7 from the 
 from __future__ import annotations
 
 import ctypes
+import math
 
 import torch
 
@@ -82,7 +83,8 @@ class LaunchList:
             self._scale(capi.LAUNCH_COARSE_TO_FINE, coarse, fine, cells)
 
     def run(self, repeats: int, stream=None):
-        """Enqueue the list `repeats` times on `stream` (default: the current stream)."""
+        """Enqueue the list `repeats` times (a fraction counts as a whole one) on `stream` (default: the
+        current stream)."""
         from .lattice import stream_handle
 
         if repeats <= 0 or not self._entries:
@@ -90,7 +92,7 @@ class LaunchList:
         if self._array is None:
             self._array = (capi.Launch * len(self._entries))(*self._entries)
         while repeats > 0:
-            n = min(repeats, _REPEATS)
+            n = math.ceil(min(repeats, _REPEATS))
             capi.call("vf_run_launches", self._array, len(self._entries), n, stream_handle(stream))
             repeats -= n
 
