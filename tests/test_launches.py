@@ -106,3 +106,36 @@ def test_run_inside_a_captured_graph(gpu):
         assert torch.equal(a.lattice.f, b.lattice.f), f"replay {i}"
         _ = b.lattice.f.float().sum().item()
     torch.cuda.synchronize()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", ["one", "two", "three"])
+def test_gradient_forwards_return_when_their_steps_are_done(gpu, case):
+    """The forward sweeps of the gradients return once their steps are done, on whichever stream the
+    caller reads the result: milliseconds of steps, enqueued in a fraction of that."""
+    import torch
+
+    from virtualfluids_amd import adjoint
+    from virtualfluids_amd.grid import periodic_box
+    from virtualfluids_amd.lattice import Lattice
+    from virtualfluids_amd.refinement import nested_box
+
+    def lattice(g):
+        L = Lattice(g, 1.7)
+        z = np.zeros(g.N)
+        L.init_equilibrium(z, z, z, z)
+        return L
+
+    if case == "one":
+        L = lattice(periodic_box(160, 160, 160))
+        call = lambda: adjoint.k17_steps(L.f, L, 100, 1000)
+    else:
+        nb = nested_box((96, 96, 96), (24, 24, 24), (72, 72, 72))
+        Ls, cells = [lattice(nb.coarse), lattice(nb.fine)], (nb.cf, nb.fc)
+        call = ((lambda: adjoint.k17_two_level_steps(Ls[0].f, Ls[1].f, Ls[0], Ls[1], cells, 100, 1000)) if case == "two"
+                else (lambda: adjoint.k17_multilevel_steps([L.f for L in Ls], Ls, [cells], 100, 1000)))
+    call()
+    torch.cuda.synchronize()
+    for _ in range(3):
+        call()
+        assert torch.cuda.current_stream().query()

@@ -250,6 +250,7 @@ class _K17Steps(torch.autograd.Function):
                     (observe_from - i) if observe is not None else steps)
             even = run.run(n, even)
             i += n
+        run.close()
         ctx.stepper, ctx.steps, ctx.K = stepper, steps, checkpoint_every
         ctx.checkpoints = checkpoints
         ctx.kept = kept
@@ -433,6 +434,7 @@ class _TwoLevelSteps(torch.autograd.Function):
             n = min(K - i % K, steps - i, (observe_from - i) if observe is not None else steps)
             even = run.run(n, even)
             i += n
+        run.close()
         ctx.sc, ctx.sf, ctx.cells, ctx.steps, ctx.K = sc, sf, cells, steps, K
         ctx.in_place = in_place
         ctx.observe, ctx.observe_from = observe, observe_from
@@ -841,6 +843,7 @@ class _MultiLevelSteps(torch.autograd.Function):
             n_run = min(K - i % K, steps - i, (observe_from - i) if observe is not None else steps)
             even = run.run(n_run, even)
             i += n_run
+        run.close()
         ctx.meta = meta
         ctx.checkpoints = checkpoints
         ctx.flags = (velocity is not None, rho_bc is not None, [p is not None for p in pors])

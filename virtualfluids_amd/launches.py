@@ -101,17 +101,19 @@ class StepLaunches:
     """Time steps that work in place on fixed buffers: run(n, even) takes n steps from parity `even`
     and returns the parity after them; calling the object takes one. With `launches` (the step's
     LaunchList and the parameter struct whose isEvenTimestep is the step's parity) they are enqueued
-    natively; otherwise step(even, stream) launches each."""
+    natively; otherwise step(even, stream) launches each. close() ends them."""
 
     def __init__(self, step, launches=None):
         self.step = step
         self.launches = launches
+        self.enqueued = 0
 
     def run(self, n: int, even: bool) -> bool:
         if self.launches is not None:
             program, param = self.launches
             param.isEvenTimestep = 1 if even else 0
             program.run(n)
+            self.enqueued += n
             return bool(param.isEvenTimestep)
         for _ in range(n):
             self.step(even, torch.cuda.current_stream())
@@ -120,3 +122,9 @@ class StepLaunches:
 
     def __call__(self, even: bool):
         self.run(1, even)
+
+    def close(self):
+        """Wait for the steps, as Simulation.run does: a sweep of three or more native steps has
+        returned when they are done."""
+        if self.enqueued >= 3:
+            torch.cuda.current_stream().synchronize()
