@@ -459,12 +459,22 @@ __global__ __launch_bounds__(kIndexedBlock) void k17_indexed_kernel(S* __restric
 // 1 node/lane in workgroups of 512 lanes like 2 nodes/lane in 256 at the same cap (5.02 ms; without
 // a cap 5.6-5.9);
 // FP16 and BF16 4 nodes/lane where rows are whole waves of it (1-2 % above 2 nodes/lane; both
-// near the VALU issue limit), else 2. Rows longer than one workgroup's lanes take the next width
-// that fits; rows no width fits take the scalar kernel. kernelChoice.rowWidth pins a width.
+// near the VALU issue limit), else 2. Rows longer than a workgroup's lanes (row_max_lanes) take the next
+// width that fits; rows no width fits take the scalar kernel. kernelChoice.rowWidth pins a width.
+
+// Lanes of a row's workgroup: 512 at one or two nodes a lane. At four, more than 256 lanes are slower than
+// the scalar kernel (us per step, row against scalar: 1280 x 110 x 110 FP32 783 / 627, FP16 622 / 351,
+// BF16 573 / 348; 2048 x 90 x 90 744 / 673, 523 / 378, 492 / 377). FP16 keeps 256 for its results: the
+// two kernels round FP16 differently (a multiply-add folded into the conversion or not), and rows of
+// five waves and more are the scalar kernel's.
+template <class S> constexpr int row_max_lanes(int V)
+{
+    return V == 4 || Codec<S>::storage == VF_STORAGE_FP16 ? 256 : kRowMaxThreads;
+}
 template <class S> static int row_width(int nx, const vf_kernel_choice& kc)
 {
     if (kc.rowWidth != 0) return kc.rowWidth;
-    auto fits = [nx](int v) { return nx % v == 0 && nx / v <= kRowMaxThreads; };
+    auto fits = [nx](int v) { return nx % v == 0 && nx / v <= row_max_lanes<S>(v); };
     auto waves = [nx](int v) { return (nx / v + 63) / 64; };
     if (Codec<S>::storage == VF_STORAGE_FP32) {
         // two nodes per lane where one node per lane leaves a last wave of a few lanes (a row
@@ -549,7 +559,7 @@ template <class S> static int box_row_width(const vf_lbm_parameter& p)
     const vf_kernel_choice& kc = p.kernelChoice;
     if (kc.boxKernel == VF_BOX_KERNEL_NODE) return 0;
     const int V = row_width<S>(p.nx, kc);
-    if (V <= 0 || p.nx % V != 0 || p.nx / V > kRowMaxThreads) return 0;
+    if (V <= 0 || p.nx % V != 0 || p.nx / V > row_max_lanes<S>(V)) return 0;
     if (V == 1 && sizeof(S) != 4) return 0;
     if (V != 1 && V != 2 && V != 4) return 0;
     const uint64_t ws = p.workingSetBytes ? p.workingSetBytes : 27 * p.numberOfNodes * sizeof(S);
