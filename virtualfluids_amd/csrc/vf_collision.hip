@@ -498,6 +498,7 @@ template <class S> static int row_width(int nx, const vf_kernel_choice& kc)
 // every wave they can get. The cap is imposed by reserving LDS at launch;
 // kernelChoice.rowWorkgroupsPerCU pins it.
 constexpr uint64_t kCacheResidentBytes = 256ull << 20;
+constexpr uint64_t kNearCacheBytes = kCacheResidentBytes / 4 * 5; // the cache still serves a good part
 template <class S, int V, int SPLIT> static int row_wgs_per_cu(uint64_t workingSet, int waves, const vf_kernel_choice& kc)
 {
     if (kc.rowWorkgroupsPerCU != 0) return kc.rowWorkgroupsPerCU < 0 ? 0 : kc.rowWorkgroupsPerCU;
@@ -552,9 +553,12 @@ static void launch_row_t(const BoxArgs& a, const K17Rates& r, bool mask, bool ma
 // node kernel, whose workgroups take consecutive nodes of a plane, leads (258 x 130 x 130 FP16
 // 87 against 153 us, FP32 203 against 264 us; measured on MI355X, one lattice stepped alone).
 // FP32 rows of a single wave are the exception: a workgroup of one wave shares nothing, and the
-// node kernel leads (64 x 300 x 300 225 against 232 us).
+// node kernel leads (64 x 300 x 300 225 against 232 us). FP32 rows of five to seven waves
+// leave lattices that the cache still serves in good part, up to 5/4 of it, to the node kernel in place
+// (256 to 295 MiB: row 1.13 to 1.32 times the node kernel's time, 640 x 60 x 70 110 / 99 us; 349 to 430 MiB
+// 0.88 to 0.94; 320 x 200 x 256 667 / 733); out of place the row kernel leads at every size (0.82 to 0.96).
 // A pinned row kernel or row width keeps the row kernel.
-template <class S> static int box_row_width(const vf_lbm_parameter& p)
+template <class S> static int box_row_width(const vf_lbm_parameter& p, bool into)
 {
     const vf_kernel_choice& kc = p.kernelChoice;
     if (kc.boxKernel == VF_BOX_KERNEL_NODE) return 0;
@@ -566,7 +570,8 @@ template <class S> static int box_row_width(const vf_lbm_parameter& p)
     const bool pinned = kc.boxKernel == VF_BOX_KERNEL_ROW || kc.rowWidth != 0;
     if (pinned) return V;
     if (ws <= kCacheResidentBytes || (p.nx / V) % 64 != 0) return 0;
-    if (sizeof(S) == 4 && p.nx / V == 64) return 0;
+    const int waves = p.nx / V / 64;
+    if (sizeof(S) == 4 && (waves == 1 || (!into && waves > 4 && waves < 8 && ws <= kNearCacheBytes))) return 0;
     return V;
 }
 
@@ -575,7 +580,7 @@ template <class S, bool EVEN>
 static bool try_launch_row(const vf_lbm_parameter& p, const BoxArgs& a, const K17Rates& r, bool macro, S* out,
                            hipStream_t s)
 {
-    const int V = box_row_width<S>(p);
+    const int V = box_row_width<S>(p, out != nullptr);
     if (V == 0) return false;
     const vf_kernel_choice& kc = p.kernelChoice;
     S* f = static_cast<S*>(p.distributions);
@@ -609,7 +614,9 @@ static bool try_launch_row(const vf_lbm_parameter& p, const BoxArgs& a, const K1
 // stream serve HBM better, until the loads in flight no longer cover its latency. Eight against
 // the cap here: FP32 in place 258 x 130 x 130 192 -> 188 (4), 333 x 200 x 290 1006 -> 805 (2); out of
 // place 255 -> 198 (3, masked), 333 x 200 x 290 945 -> 900 (3); 16-bit in place 333 x 200 x 290 500 ->
-// 462 (4), out of place 542 -> 498 (4). Lattices of less than half the cache are latency-bound
+// 462 (4), out of place 542 -> 498 (4). Up to 5/4 of the cache four lead in FP32 in place as within it
+// (256 to 295 MiB, whole planes: two 1.06 to 1.19 times, four 0.97 to 1.00 times the time of eight; from
+// 349 MiB two 0.93 to 1.01). Lattices of less than half the cache are latency-bound
 // (26 MB: 9.7 -> 10.7 at 4) and take every wave.
 struct NodeLaunch {
     bool xcd;
@@ -623,7 +630,7 @@ template <class S> static NodeLaunch node_launch(const vf_lbm_parameter& p, bool
     const bool xcd = choice == 1 || choice == 2 ? choice == 1
                                                 : xcd_planes(p.nx, p.ny, sizeof(S), 0) && !ordered;
     int cap = 0;
-    if (own > kCacheResidentBytes / 2) cap = sizeof(S) == 2 ? 4 : into ? 3 : xcd || own <= kCacheResidentBytes ? 4 : 2;
+    if (own > kCacheResidentBytes / 2) cap = sizeof(S) == 2 ? 4 : into ? 3 : xcd || own <= kNearCacheBytes ? 4 : 2;
     return {xcd, lds_reserve_for(cap)};
 }
 
@@ -680,7 +687,7 @@ static void launch_node_bb_b(const vf_lbm_parameter& p, const BoxArgs& a, const 
 template <class S, bool EVEN>
 static bool launch_box_bb_t(const vf_lbm_parameter& p, bool macro, const FusedBB& bb, hipStream_t s)
 {
-    if (box_row_width<S>(p) != 0) return false;
+    if (box_row_width<S>(p, false) != 0) return false;
     BoxArgs a{p.numberOfNodes, p.nx, p.ny, p.nz, p.fluidMask, p.rho, p.velocityX, p.velocityY, p.velocityZ,
               p.porosity, make_plane_div(p.nx, p.ny)};
     const K17Rates r = make_k17_rates(p);
