@@ -622,13 +622,14 @@ struct NodeLaunch {
     bool xcd;
     size_t lds; // reserved at launch to impose the cap
 };
-template <class S> static NodeLaunch node_launch(const vf_lbm_parameter& p, bool into)
+// ranges: whether the launch has a variant in XCD block ranges; the cap goes with the order launched
+template <class S> static NodeLaunch node_launch(const vf_lbm_parameter& p, bool into, bool ranges)
 {
     const uint64_t own = 27 * p.numberOfNodes * sizeof(S);
     const int choice = p.kernelChoice.rowXcdRanges;
     const bool ordered = !into && own > (sizeof(S) == 4 ? 2 * kCacheResidentBytes : kCacheResidentBytes);
-    const bool xcd = choice == 1 || choice == 2 ? choice == 1
-                                                : xcd_planes(p.nx, p.ny, sizeof(S), 0) && !ordered;
+    const bool xcd = ranges && (choice == 1 || choice == 2 ? choice == 1
+                                                           : xcd_planes(p.nx, p.ny, sizeof(S), 0) && !ordered);
     int cap = 0;
     if (own > kCacheResidentBytes / 2) cap = sizeof(S) == 2 ? 4 : into ? 3 : xcd || own <= kNearCacheBytes ? 4 : 2;
     return {xcd, lds_reserve_for(cap)};
@@ -647,7 +648,7 @@ static void launch_node_b(const vf_lbm_parameter& p, const BoxArgs& a, const K17
     const bool mask = p.fluidMask != nullptr;
     const dim3 grid(plane_blocks(p.nx, p.ny), p.nz), bx(kBoxBlock);
     const FusedBB none{};
-    const auto [xcd, lds] = node_launch<S>(p, false);
+    const auto [xcd, lds] = node_launch<S>(p, false, !macro);
     if (mask && macro) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, BUF, true, true>), grid, dim3(bx), lds, s, f, a, r, none);
     else if (mask && xcd) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, BUF, true, false, false, true>), grid, dim3(bx), lds, s, f, a, r, none);
     else if (mask) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, BUF, true, false>), grid, dim3(bx), lds, s, f, a, r, none);
@@ -674,7 +675,7 @@ static void launch_node_bb_b(const vf_lbm_parameter& p, const BoxArgs& a, const 
     S* f = static_cast<S*>(p.distributions);
     const bool mask = p.fluidMask != nullptr;
     const dim3 grid(plane_blocks(p.nx, p.ny), p.nz), bx(kBoxBlock);
-    const auto [xcd, lds] = node_launch<S>(p, false);
+    const auto [xcd, lds] = node_launch<S>(p, false, mask && !macro);
     if (mask && macro) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, BUF, true, true, true>), grid, dim3(bx), lds, s, f, a, r, bb);
     else if (mask && xcd) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, BUF, true, false, true, true>), grid, dim3(bx), lds, s, f, a, r, bb);
     else if (mask) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, BUF, true, false, true>), grid, dim3(bx), lds, s, f, a, r, bb);
@@ -747,7 +748,7 @@ static void launch_into_b(const vf_lbm_parameter& p, const BoxArgs& a, const K17
 {
     const dim3 grid(plane_blocks(p.nx, p.ny), p.nz), bx(kBoxBlock);
     const S* in = static_cast<const S*>(p.distributions);
-    const auto [xcd, lds] = node_launch<S>(p, true);
+    const auto [xcd, lds] = node_launch<S>(p, true, true);
     if (p.fluidMask && xcd)
         hipLaunchKernelGGL((k17_box_into_kernel<S, EVEN, BUF, true, true>), grid, dim3(bx), lds, s, in, out, a, r);
     else if (p.fluidMask)
