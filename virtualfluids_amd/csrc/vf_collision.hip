@@ -598,26 +598,31 @@ static bool try_launch_row(const vf_lbm_parameter& p, const BoxArgs& a, const K1
 //
 // XCD block ranges (xcd_block): where the spans of a plane share cache lines at their ends (a plane
 // is not a whole number of lines) the ranges keep both sharers in one L2. Beyond the cache they
-// also make eight distant regions of every stream, which costs DRAM efficiency: a 16-bit lattice
-// (its spans half as long) is better off in launch order, and so is an FP32 lattice of more
-// than twice the cache at two resident workgroups per CU. Measured on MI355X, us per step in
-// place, ranges against launch order, each at its best cap:
+// also make eight distant regions of every stream, which costs DRAM efficiency: an unmasked 16-bit
+// lattice (its spans half as long) is better off in launch order from 9/8 of the cache, and so is an FP32
+// lattice of more than twice the cache at two resident workgroups per CU. Measured on MI355X, us
+// per step in place, ranges against launch order, each at its best cap:
 //   cache-resident   66^3 FP32 11.8 / 12.9, FP16 10.0 / 12.3; 130 x 70 x 70 FP32 22.9 / 26.2;
-//                    194 x 98 x 98 FP32 63.0 / 68.6; 258 x 130 x 130 FP16 90 / 98
+//                    194 x 98 x 98 FP32 63.0 / 68.6; 258 x 130 x 130 FP16 90 / 98; 191 x 126 x 213 BF16 130 / 146
 //   streaming FP32   258 x 130 x 130 187 / 196; 251 x 187 x 133 280 / 271; 300 x 301 x 150 582 / 569;
 //                    333 x 200 x 290 855 / 805; 150 x 300 x 310 601 / 580
 //   streaming 16-bit 251 x 187 x 133 183 / 158; 300 x 301 x 150 332 / 327; 333 x 200 x 290 502 / 462
-// A 16-bit level that fits by itself inside a hierarchy that does not (258 x 130 x 130 FP16 in the
-// two-level step) takes the ranges: 315 us per coarse step against 319 in launch order.
+// Streaming 16-bit lattices differ among themselves: over 35 sizes from 300 to 1500 MiB launch order took
+// 0.88 to 1.09 times the ranges, 0.99 in the mean. With solid nodes (their lines are written in part) it
+// took 0.91 to 1.08 times and 1.02 in the mean over 40, so those keep the ranges. A 16-bit level that
+// fits by itself inside a hierarchy that does not (258 x 130 x 130 FP16 in the two-level step) takes the
+// ranges: 315 us per coarse step against 319 in launch order.
 //
 // Resident workgroups per CU (0: as many as registers allow, eight): fewer concurrent spans per
 // stream serve HBM better, until the loads in flight no longer cover its latency. Eight against
 // the cap here: FP32 in place 258 x 130 x 130 192 -> 188 (4), 333 x 200 x 290 1006 -> 805 (2); out of
 // place 255 -> 198 (3, masked), 333 x 200 x 290 945 -> 900 (3); 16-bit in place 333 x 200 x 290 500 ->
-// 462 (4), out of place 542 -> 498 (4). Up to 5/4 of the cache four lead in FP32 in place as within it
-// (256 to 295 MiB, whole planes: two 1.06 to 1.19 times, four 0.97 to 1.00 times the time of eight; from
-// 349 MiB two 0.93 to 1.01). Lattices of less than half the cache are latency-bound
-// (26 MB: 9.7 -> 10.7 at 4) and take every wave.
+// 462 (4), out of place 542 -> 498 (4). 16-bit lattices of whole planes (64 x 934 x 439) keep six, which
+// is within 1 % of eight in place and the best out of place (four: 618 and 659 us, six: 557 and 612), and
+// so do those with solid nodes beyond the cache (0.97 to 1.03 of four, 0.99 in the mean). Up to 5/4 of the cache four lead
+// in FP32 in place as within it (256 to 295 MiB, whole planes: two 1.06 to 1.19 times, four 0.97 to 1.00
+// times the time of eight; from 349 MiB two 0.93 to 1.01). Lattices of less than half the cache are
+// latency-bound (26 MB: 9.7 -> 10.7 at 4) and take every wave.
 struct NodeLaunch {
     bool xcd;
     size_t lds; // reserved at launch to impose the cap
@@ -627,11 +632,15 @@ template <class S> static NodeLaunch node_launch(const vf_lbm_parameter& p, bool
 {
     const uint64_t own = 27 * p.numberOfNodes * sizeof(S);
     const int choice = p.kernelChoice.rowXcdRanges;
-    const bool ordered = !into && own > (sizeof(S) == 4 ? 2 * kCacheResidentBytes : kCacheResidentBytes);
-    const bool xcd = ranges && (choice == 1 || choice == 2 ? choice == 1
-                                                           : xcd_planes(p.nx, p.ny, sizeof(S), 0) && !ordered);
+    const bool half = sizeof(S) == 2, masked = p.fluidMask != nullptr;
+    const bool shared = xcd_planes(p.nx, p.ny, sizeof(S), 0); // planes share lines at their ends
+    const bool ordered = !into && (half ? !masked && own > kCacheResidentBytes / 8 * 9 : own > 2 * kCacheResidentBytes);
+    const bool xcd = ranges && (choice == 1 || choice == 2 ? choice == 1 : shared && !ordered);
     int cap = 0;
-    if (own > kCacheResidentBytes / 2) cap = sizeof(S) == 2 ? 4 : into ? 3 : xcd || own <= kNearCacheBytes ? 4 : 2;
+    if (own > kCacheResidentBytes / 2) {
+        if (half) cap = !shared || (masked && !into && own > kCacheResidentBytes) ? 6 : 4;
+        else cap = into ? 3 : xcd || own <= kNearCacheBytes ? 4 : 2;
+    }
     return {xcd, lds_reserve_for(cap)};
 }
 
