@@ -394,24 +394,33 @@ void launch_row_b(const AdjBoxArgs& a, const K17Rates& r, const S* f, float* lam
 
 template <class S, bool EVEN, bool BUF>
 void launch_scalar_b(const AdjBoxArgs& a, const K17Rates& r, const S* f, float* lam, bool mask, bool shift, dim3 grid,
-                     hipStream_t s, bool xcd)
+                     hipStream_t s, bool xcd, size_t lds)
 {
     const dim3 block(kAdjBlock);
-    if (xcd && mask && !shift) hipLaunchKernelGGL((k17_adjoint_box_kernel<S, EVEN, true, false, BUF, true>), grid, block, 0, s, f, lam, a, r);
-    else if (xcd && !mask && !shift) hipLaunchKernelGGL((k17_adjoint_box_kernel<S, EVEN, false, false, BUF, true>), grid, block, 0, s, f, lam, a, r);
-    else if (mask && shift) hipLaunchKernelGGL((k17_adjoint_box_kernel<S, EVEN, true, true, BUF>), grid, block, 0, s, f, lam, a, r);
-    else if (mask) hipLaunchKernelGGL((k17_adjoint_box_kernel<S, EVEN, true, false, BUF>), grid, block, 0, s, f, lam, a, r);
-    else if (shift) hipLaunchKernelGGL((k17_adjoint_box_kernel<S, EVEN, false, true, BUF>), grid, block, 0, s, f, lam, a, r);
-    else hipLaunchKernelGGL((k17_adjoint_box_kernel<S, EVEN, false, false, BUF>), grid, block, 0, s, f, lam, a, r);
+    if (xcd && mask && !shift) hipLaunchKernelGGL((k17_adjoint_box_kernel<S, EVEN, true, false, BUF, true>), grid, block, lds, s, f, lam, a, r);
+    else if (xcd && !mask && !shift) hipLaunchKernelGGL((k17_adjoint_box_kernel<S, EVEN, false, false, BUF, true>), grid, block, lds, s, f, lam, a, r);
+    else if (mask && shift) hipLaunchKernelGGL((k17_adjoint_box_kernel<S, EVEN, true, true, BUF>), grid, block, lds, s, f, lam, a, r);
+    else if (mask) hipLaunchKernelGGL((k17_adjoint_box_kernel<S, EVEN, true, false, BUF>), grid, block, lds, s, f, lam, a, r);
+    else if (shift) hipLaunchKernelGGL((k17_adjoint_box_kernel<S, EVEN, false, true, BUF>), grid, block, lds, s, f, lam, a, r);
+    else hipLaunchKernelGGL((k17_adjoint_box_kernel<S, EVEN, false, false, BUF>), grid, block, lds, s, f, lam, a, r);
 }
 template <class S, bool EVEN>
 void launch_scalar(const AdjBoxArgs& a, const K17Rates& r, const S* f, float* lam, bool mask, bool shift, dim3 grid,
                    hipStream_t s, const vf_kernel_choice& kc, bool xcd = false)
 {
+    // Two resident workgroups per CU (of the three that registers allow) where state and adjoint together
+    // exceed twice the cache: the third only adds concurrent streams (us, three / two: 546 x 243 x 211 FP16
+    // 1808 / 1507, 304 x 262 x 140 675 / 610, 406 x 235 x 102 FP32 656 / 619, 1024 x 147 x 113 1119 / 1069; at
+    // 327 MiB of both 105 / 107). With solid nodes FP32 does so from four times the cache (400 x 400 x 200 2304 /
+    // 2038, 330 x 200 x 193 850 / 809; 286 x 99 x 111 208 / 216), 16-bit not at all (450 x 200 x 250 1173 / 1215), nor the
+    // shift's adjoint.
+    const uint64_t both = 27 * a.N * (sizeof(S) + sizeof(float));
+    const bool streams = mask ? sizeof(S) == 4 && both > (1024ull << 20) : both > (512ull << 20);
+    const size_t lds = lds_reserve_for(streams && !shift && !xcd ? 2 : 0);
     // the buffer form needs kRowSplit slots of the adjoint (the larger element) within 32-bit offsets
     if (slots_fit_buffers(a.N, sizeof(float)) && kc.rowAddressing != VF_ROW_ADDRESSING_GLOBAL)
-        launch_scalar_b<S, EVEN, true>(a, r, f, lam, mask, shift, grid, s, xcd);
-    else launch_scalar_b<S, EVEN, false>(a, r, f, lam, mask, shift, grid, s, xcd);
+        launch_scalar_b<S, EVEN, true>(a, r, f, lam, mask, shift, grid, s, xcd, lds);
+    else launch_scalar_b<S, EVEN, false>(a, r, f, lam, mask, shift, grid, s, xcd, lds);
 }
 
 template <class S, bool EVEN>
@@ -428,7 +437,9 @@ void launch_box(const vf_lbm_parameter& p, float* lam, float* shift, float* padj
     // leave too few workgroups to overlap loads and arithmetic (384 x 192 x 128 FP32 789 / 600, 512 x
     // 128 x 128 630 / 529), and
     // rows that are not whole waves idle lanes (258 x 130 x 130 FP16 524 / 250): those take the
-    // scalar kernel, whose plane-flat workgroups keep every lane busy.
+    // scalar kernel, whose plane-flat workgroups keep every lane busy. So do rows of three waves with solid
+    // nodes: spread over the box these break up the row kernel's non-temporal lines (one node in ten,
+    // 192 x 97 x 168 FP16 231 / 172, 192 x 458 x 176 FP32 1293 / 1051; walls only, 192 x 436 x 357 FP16 1490 / 1594).
     // kernelChoice.adjointKernel pins the scalar kernel, whole rows (ROW_WHOLE), or the row kernel
     // over the whole waves of any row with the scalar kernel on the columns beyond (ROW: a row
     // whose last wave would carry fewer than 32 lanes is split there, 258 = 256 + 2).
@@ -438,7 +449,7 @@ void launch_box(const vf_lbm_parameter& p, float* lam, float* shift, float* padj
     if (p.nx > 64 && p.nx % 64 != 0 && p.nx % 64 < 32 && kc.adjointKernel == VF_ADJOINT_KERNEL_ROW)
         rowEnd = p.nx - p.nx % 64;
     const int waves = (int)((rowEnd + 63) / 64);
-    const bool wholeWaves = p.nx % 64 == 0 && waves <= 4;
+    const bool wholeWaves = p.nx % 64 == 0 && waves <= 4 && !(waves == 3 && mask);
     if (rowEnd <= (uint32_t)kAdjRowMaxThreads && (wholeWaves || pinnedRow) && kc.adjointKernel != VF_ADJOINT_KERNEL_NODE) {
         // the buffer form needs kRowSplit slots of the adjoint (the larger element) within
         // 32-bit offsets
