@@ -133,29 +133,27 @@ __device__ __forceinline__ double node_energy(const float* vx, const float* vy, 
     return 0.5 * (ux * ux + uy * uy + uz * uz) * ((double)rho[k] + 1.0);
 }
 
-// BOX: nodes numbered over the planes of a dense box (plane_sum_grid), so that the seven neighbours
-// are offsets; their types and the node's fields are loaded together (one by one
-// behind the previous test they are eight memory latencies a node). Bound by HBM: 20 bytes a node.
-// 256^3: 156 us with the chain, a division per coordinate and 2048 workgroups, 66 us so.
+// BOX: a dense box, whose seven neighbours are offsets (the coordinates by reciprocals); their types and
+// the node's fields are loaded together (one by one behind the previous test they are eight memory
+// latencies a node). Bound by HBM: 20 bytes a node. 256^3: 156 us with the chain, a division per
+// coordinate and 2048 workgroups, 73 us so.
 template <bool BOX>
 __global__ __launch_bounds__(kReduceThreads) void kinetic_energy_kernel(Addr a, const uint32_t* nbinv, const uint32_t* geo,
                                                              const float* vx, const float* vy, const float* vz,
-                                                             const float* rho, PlaneDiv plane, double* out)
+                                                             const float* rho, BoxDiv box, double* out)
 {
     __shared__ double part[kReduceThreads / 64][2];
     double e = 0.0, c = 0.0;
+    const uint64_t step = (uint64_t)gridDim.x * blockDim.x;
     if constexpr (BOX) {
-        const uint32_t nx = plane.nx, ny = (uint32_t)a.ny, nz = (uint32_t)a.nz, P = plane.planeNodes;
-        const uint32_t per = (P + kReduceThreads - 1) / kReduceThreads;
-        for (uint64_t i = blockIdx.x; i < (uint64_t)per * nz; i += gridDim.x) {
-            const uint32_t z = (uint32_t)(i / per), t = (uint32_t)(i % per) * kReduceThreads + threadIdx.x;
-            if (t >= P) continue;
-            const uint32_t y = plane_row(t, plane), x = t - y * nx;
+        const uint32_t nx = box.plane.nx, ny = (uint32_t)a.ny, nz = (uint32_t)a.nz, P = box.plane.planeNodes;
+        for (uint64_t kk = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; kk < a.N; kk += step) {
+            const uint32_t k = (uint32_t)kk, z = box_plane(k, box), t = k - P * z;
+            const uint32_t y = plane_row(t, box.plane), x = t - y * nx;
             const uint32_t xp = x + 1 == nx ? t + 1 - nx : t + 1, xm = x == 0 ? t + nx - 1 : t - 1;
             const uint32_t yp = y + 1 == ny ? x : t + nx, ym = y == 0 ? t + (P - nx) : t - nx;
             const uint32_t xym = y == 0 ? xm + (P - nx) : xm - nx;
             const uint32_t zo = P * z, zp = P * (z + 1 == nz ? 0 : z + 1), zm = P * (z == 0 ? nz - 1 : z - 1);
-            const uint32_t k = zo + t;
             const uint32_t g[8] = {geo[k],       geo[zo + xp], geo[zo + xm], geo[zo + yp],
                                    geo[zo + ym], geo[zp + t],  geo[zm + t],  geo[zm + xym]};
             const double en = node_energy(vx, vy, vz, rho, k);
@@ -168,8 +166,7 @@ __global__ __launch_bounds__(kReduceThreads) void kinetic_energy_kernel(Addr a, 
             }
         }
     } else {
-        for (uint64_t kk = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; kk < a.N;
-             kk += (uint64_t)gridDim.x * blockDim.x) {
+        for (uint64_t kk = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; kk < a.N; kk += step) {
             const uint32_t k = (uint32_t)kk;
             if (!interior_fluid(a, nbinv, geo, k)) continue;
             e += node_energy(vx, vy, vz, rho, k);
@@ -186,7 +183,7 @@ __global__ __launch_bounds__(kReduceThreads) void kinetic_energy_kernel(Addr a, 
     __syncthreads();
     if (threadIdx.x < 2) {
         double s = 0.0;
-        for (int w = 0; w < kReduceThreads / 64; ++w) s += part[w][threadIdx.x];
+        for (unsigned w = 0; w < blockDim.x / 64; ++w) s += part[w][threadIdx.x];
         atomicAdd(out + threadIdx.x, s);
     }
 }
@@ -307,15 +304,15 @@ extern "C" int vf_KineticEnergy(const vf_lbm_parameter* p, const uint32_t* neigh
     }
     hipStream_t s = (hipStream_t)stream;
     hipLaunchKernelGGL(zero2_kernel, dim3(1), dim3(64), 0, s, out2);
+    const SumLaunch l = sum_launch(p->numberOfNodes);
     if (!p->neighborX) {
-        const dim3 grid = plane_sum_grid(p->nx, p->ny, p->nz);
-        hipLaunchKernelGGL(kinetic_energy_kernel<true>, grid, dim3(kReduceThreads), 0, s, make_addr(*p), neighborInverse,
+        hipLaunchKernelGGL(kinetic_energy_kernel<true>, l.grid, l.block, 0, s, make_addr(*p), neighborInverse,
                            p->typeOfGridNode, p->velocityX, p->velocityY, p->velocityZ, p->rho,
-                           make_plane_div(p->nx, p->ny), out2);
+                           make_box_div(p->nx, p->ny), out2);
     } else {
-        hipLaunchKernelGGL(kinetic_energy_kernel<false>, flat_sum_grid(p->numberOfNodes), dim3(kReduceThreads), 0, s,
+        hipLaunchKernelGGL(kinetic_energy_kernel<false>, l.grid, l.block, 0, s,
                            make_addr(*p), neighborInverse, p->typeOfGridNode, p->velocityX, p->velocityY,
-                           p->velocityZ, p->rho, PlaneDiv{}, out2);
+                           p->velocityZ, p->rho, BoxDiv{}, out2);
     }
     return check_launch("kineticEnergyKernel execution failed");
 }

@@ -126,13 +126,13 @@ __device__ __forceinline__ bool is_valid_fluid(uint32_t t)
     return t == VF_GEO_FLUID || t == VF_GEO_PM_0 || t == VF_GEO_PM_1 || t == VF_GEO_PM_2;
 }
 
-// The cell nodes of node t of plane z (t = x + nx y) of a dense box
-__device__ __forceinline__ void plane_cell_nodes(const PlaneDiv& p, int ny, int nz, uint32_t t, uint32_t z,
-                                                 uint32_t (&n)[8])
+// The cell nodes of node k of a dense box
+__device__ __forceinline__ void box_cell_nodes(const BoxDiv& b, int ny, int nz, uint32_t k, uint32_t (&n)[8])
 {
-    const uint32_t y = plane_row(t, p), x = t - y * p.nx, P = p.planeNodes;
-    const uint32_t xp = x + 1 == p.nx ? 0 : x + 1;
-    const uint32_t r0 = t - x, r1 = y + 1 == (uint32_t)ny ? 0 : r0 + p.nx;
+    const uint32_t P = b.plane.planeNodes, nx = b.plane.nx;
+    const uint32_t z = box_plane(k, b), t = k - P * z, y = plane_row(t, b.plane), x = t - y * nx;
+    const uint32_t xp = x + 1 == nx ? 0 : x + 1;
+    const uint32_t r0 = t - x, r1 = y + 1 == (uint32_t)ny ? 0 : r0 + nx;
     const uint32_t z0 = P * z, z1 = z + 1 == (uint32_t)nz ? 0 : z0 + P;
     n[0] = z0 + r0 + x; n[1] = z0 + r0 + xp; n[2] = z0 + r1 + x; n[3] = z0 + r1 + xp;
     n[4] = z1 + r0 + x; n[5] = z1 + r0 + xp; n[6] = z1 + r1 + x; n[7] = z1 + r1 + xp;
@@ -165,29 +165,23 @@ __device__ __forceinline__ void node_moments(const float (&f)[27], double& drho,
     }
 }
 
-// BOX: nodes numbered over the planes of a dense box (one per thread, grid.y the plane), populations
-// through buffer descriptors where they reach. Bound by HBM: 27 populations, the type and five
-// fields a node. 256^3 FP32: 429 us with a division per coordinate and every field written twice
-// (zero, then the value).
+// BOX: the cell nodes of a dense box by reciprocals; populations through buffer descriptors where they
+// reach. Bound by HBM: 27 populations, the type and five fields a node. 256^3 FP32: 429 us with a
+// division per coordinate and every field written twice (zero, then the value), 396 so.
 template <class S, bool BOX, bool BUF>
-__global__ __launch_bounds__(256) void macroscopic_kernel(const S* __restrict__ f, Addr a, PlaneDiv plane,
+__global__ __launch_bounds__(256) void macroscopic_kernel(const S* __restrict__ f, Addr a, BoxDiv box,
                                                           const uint32_t* geo, float* rho, float* vx, float* vy,
                                                           float* vz, float* press, int even_flag)
 {
-    uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= a.N) return;
     uint32_t n[8];
-    if constexpr (BOX) {
-        if (k >= plane.planeNodes) return;
-        plane_cell_nodes(plane, a.ny, a.nz, (uint32_t)k, blockIdx.y, n);
-        k = n[0];
-    } else {
-        if (k >= a.N) return;
-    }
     // a node that is not fluid keeps the zeros; one store for both, so that a wave that holds both writes
     // whole lines (448 x 115 x 327 BF16, one solid node in ten: 226 us, 312 with a store of its own for each)
     float drho = 0.0f, ux = 0.0f, uy = 0.0f, uz = 0.0f, pr = 0.0f;
     if (!geo || is_valid_fluid(geo[k])) {
-        if constexpr (!BOX) cell_nodes(a, (uint32_t)k, n);
+        if constexpr (BOX) box_cell_nodes(box, a.ny, a.nz, (uint32_t)k, n);
+        else cell_nodes(a, (uint32_t)k, n);
         const SlotIO<S, BUF> io(f, a.N);
         float fv[27];
         load_cell<S, BUF>(io, n, even_flag != 0, fv);
@@ -230,10 +224,9 @@ __device__ __forceinline__ double wave_sum(double v)
 }
 
 // out[0..3] += sum drho, jx, jy, jz; out[4] += sum 1/2 (1+drho) |u|^2 (when KE).
-// BOX, BUF as in macroscopic_kernel; a workgroup steps through the planes (plane_sum_grid). Bound
-// by HBM: 27 populations and the type a node (256^3 FP32 327 us, FP16 197 -> 174 us).
+// BOX, BUF as in macroscopic_kernel; launched by sum_launch. Bound by HBM: 27 populations and the type a node (256^3 FP32 327 us, FP16 197 -> 174 us).
 template <class S, bool KE, bool BOX, bool BUF>
-__global__ __launch_bounds__(kReduceThreads) void moments_reduce_kernel(const S* __restrict__ f, Addr a, PlaneDiv plane,
+__global__ __launch_bounds__(kReduceThreads) void moments_reduce_kernel(const S* __restrict__ f, Addr a, BoxDiv box,
                                                              const uint32_t* geo, int even_flag, double* out)
 {
     constexpr int NV = KE ? 5 : 4;
@@ -256,22 +249,11 @@ __global__ __launch_bounds__(kReduceThreads) void moments_reduce_kernel(const S*
         }
     };
     uint32_t n[8];
-    if constexpr (BOX) {
-        const uint32_t per = (plane.planeNodes + kReduceThreads - 1) / kReduceThreads;
-        for (uint64_t i = blockIdx.x; i < (uint64_t)per * (uint32_t)a.nz; i += gridDim.x) {
-            const uint32_t z = (uint32_t)(i / per), t = (uint32_t)(i % per) * kReduceThreads + threadIdx.x;
-            if (t >= plane.planeNodes) continue;
-            plane_cell_nodes(plane, a.ny, a.nz, t, z, n);
-            if (geo && geo[n[0]] != VF_GEO_FLUID) continue;
-            add(n);
-        }
-    } else {
-        for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k < a.N;
-             k += (uint64_t)gridDim.x * blockDim.x) {
-            if (geo && geo[k] != VF_GEO_FLUID) continue;
-            cell_nodes(a, (uint32_t)k, n);
-            add(n);
-        }
+    for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k < a.N; k += (uint64_t)gridDim.x * blockDim.x) {
+        if (geo && geo[k] != VF_GEO_FLUID) continue;
+        if constexpr (BOX) box_cell_nodes(box, a.ny, a.nz, (uint32_t)k, n);
+        else cell_nodes(a, (uint32_t)k, n);
+        add(n);
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
@@ -282,7 +264,7 @@ __global__ __launch_bounds__(kReduceThreads) void moments_reduce_kernel(const S*
     __syncthreads();
     if (threadIdx.x < NV) {
         double s = 0.0;
-        for (int w = 0; w < kReduceThreads / 64; ++w) s += part[w][threadIdx.x];
+        for (unsigned w = 0; w < blockDim.x / 64; ++w) s += part[w][threadIdx.x];
         atomicAdd(out + threadIdx.x, s);
     }
 }
@@ -314,23 +296,20 @@ template <class S> struct InitNeqL {
                            p.isEvenTimestep);
     }
 };
-// whether the plane-numbered forms serve a lattice: a dense box whose planes fit grid.y
-static bool plane_box(const vf_lbm_parameter& p) { return !p.neighborX && p.nz <= 65535; }
-
 template <class S> struct MacroL {
     template <bool BOX, bool BUF> static void go(const vf_lbm_parameter& p, hipStream_t s)
     {
-        const dim3 grid = BOX ? dim3(plane_blocks(p.nx, p.ny), p.nz) : dim3((unsigned)((p.numberOfNodes + 255) / 256));
+        const dim3 grid((unsigned)((p.numberOfNodes + 255) / 256));
         // FP32 beyond the cache: four resident workgroups per CU (415 -> 402 us at 256^3); a 16-bit
         // lattice needs every wave (234 -> 253 us at four)
         const bool cap = BOX && sizeof(S) == 4 && 27 * p.numberOfNodes * sizeof(S) > (256ull << 20);
         hipLaunchKernelGGL((macroscopic_kernel<S, BOX, BUF>), grid, dim3(256), lds_reserve_for(cap ? 4 : 0), s, (const S*)p.distributions,
-                           make_addr(p), BOX ? make_plane_div(p.nx, p.ny) : PlaneDiv{}, p.typeOfGridNode, p.rho,
+                           make_addr(p), BOX ? make_box_div(p.nx, p.ny) : BoxDiv{}, p.typeOfGridNode, p.rho,
                            p.velocityX, p.velocityY, p.velocityZ, p.pressure, p.isEvenTimestep);
     }
     static void run(const vf_lbm_parameter& p, hipStream_t s)
     {
-        if (!plane_box(p)) go<false, false>(p, s);
+        if (p.neighborX) go<false, false>(p, s);
         else if (slots_fit_buffers(p.numberOfNodes, sizeof(S))) go<true, true>(p, s);
         else go<true, false>(p, s);
     }
@@ -338,14 +317,14 @@ template <class S> struct MacroL {
 template <class S> struct ReduceL {
     template <bool KE, bool BOX, bool BUF> static void go(const vf_lbm_parameter& p, double* out, hipStream_t s)
     {
-        const dim3 grid = BOX ? plane_sum_grid(p.nx, p.ny, p.nz) : flat_sum_grid(p.numberOfNodes);
-        hipLaunchKernelGGL((moments_reduce_kernel<S, KE, BOX, BUF>), grid, dim3(kReduceThreads), 0, s, (const S*)p.distributions,
-                           make_addr(p), BOX ? make_plane_div(p.nx, p.ny) : PlaneDiv{}, p.typeOfGridNode,
+        const SumLaunch l = sum_launch(p.numberOfNodes);
+        hipLaunchKernelGGL((moments_reduce_kernel<S, KE, BOX, BUF>), l.grid, l.block, 0, s, (const S*)p.distributions,
+                           make_addr(p), BOX ? make_box_div(p.nx, p.ny) : BoxDiv{}, p.typeOfGridNode,
                            p.isEvenTimestep, out);
     }
     template <bool KE> static void pick(const vf_lbm_parameter& p, double* out, hipStream_t s)
     {
-        if (!plane_box(p)) go<KE, false, false>(p, out, s);
+        if (p.neighborX) go<KE, false, false>(p, out, s);
         else if (slots_fit_buffers(p.numberOfNodes, sizeof(S))) go<KE, true, true>(p, out, s);
         else go<KE, true, false>(p, out, s);
     }
