@@ -85,7 +85,7 @@ typedef struct vf_kernel_choice {
     int32_t rowWidth;           /* 0: automatic; 1, 2 or 4 nodes per lane (2 and 4 for FP16/BF16) */
     int32_t rowWorkgroupsPerCU; /* 0: automatic; -1: no cap; k > 0: at most k row workgroups per CU */
     int32_t rowAddressing;      /* enum vf_row_addressing (row kernels; GLOBAL: every collision and adjoint
-                                   kernel but the indexed adjoint) */
+                                   kernel but the indexed adjoint, fields and sums of boxes) */
     int32_t rowXcdRanges;       /* 0: automatic; 1: contiguous row ranges per XCD; 2: launch order (WriteMacroVars
                                    and the bounce-back epilogue without a mask: always launch order) */
     int32_t adjointKernel;      /* enum vf_adjoint_kernel */

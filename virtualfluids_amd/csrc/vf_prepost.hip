@@ -296,6 +296,12 @@ template <class S> struct InitNeqL {
                            p.isEvenTimestep);
     }
 };
+// Buffer descriptors where 14 slots lie within 4 GiB, unless 64-bit addresses are pinned
+template <class S> static bool buffers(const vf_lbm_parameter& p)
+{
+    return slots_fit_buffers(p.numberOfNodes, sizeof(S)) && p.kernelChoice.rowAddressing != VF_ROW_ADDRESSING_GLOBAL;
+}
+
 template <class S> struct MacroL {
     template <bool BOX, bool BUF> static void go(const vf_lbm_parameter& p, hipStream_t s)
     {
@@ -310,7 +316,7 @@ template <class S> struct MacroL {
     static void run(const vf_lbm_parameter& p, hipStream_t s)
     {
         if (p.neighborX) go<false, false>(p, s);
-        else if (slots_fit_buffers(p.numberOfNodes, sizeof(S))) go<true, true>(p, s);
+        else if (buffers<S>(p)) go<true, true>(p, s);
         else go<true, false>(p, s);
     }
 };
@@ -325,7 +331,7 @@ template <class S> struct ReduceL {
     template <bool KE> static void pick(const vf_lbm_parameter& p, double* out, hipStream_t s)
     {
         if (p.neighborX) go<KE, false, false>(p, out, s);
-        else if (slots_fit_buffers(p.numberOfNodes, sizeof(S))) go<KE, true, true>(p, out, s);
+        else if (buffers<S>(p)) go<KE, true, true>(p, out, s);
         else go<KE, true, false>(p, out, s);
     }
     static void run(const vf_lbm_parameter& p, double* out, bool ke, hipStream_t s)
