@@ -139,3 +139,24 @@ def test_gradient_forwards_return_when_their_steps_are_done(gpu, case):
     for _ in range(3):
         call()
         assert torch.cuda.current_stream().query()
+
+
+@pytest.mark.gpu
+def test_one_step_of_one_launch_builds_no_list(gpu, monkeypatch):
+    """A run of one step whose step is one launch makes that launch; every other run is enqueued."""
+    from virtualfluids_amd.lattice import Lattice
+    from virtualfluids_amd.simulation import Simulation
+
+    g = cavity(9)
+    L = Lattice(g, 1.7)
+    z = np.zeros(g.N)
+    L.init_equilibrium(z, z, z, z)
+    sim = Simulation(L, _factory(True))
+    sim.run(1)
+    built = []
+    add = Simulation.add_launches
+    monkeypatch.setattr(Simulation, "add_launches", lambda self, *a, **k: built.append(1) or add(self, *a, **k))
+    sim.run(1)
+    assert not built and sim.t == 2 and L.even
+    sim.run(2)
+    assert built and sim.t == 4 and L.even

@@ -403,7 +403,7 @@ class Simulation:
         itself (virtualfluids_amd.launches): the same kernels with the same arguments, without a host
         round trip per launch; without an explicit stream a run of three or more steps returns once
         they are done. graphs=False launches every kernel from Python."""
-        if not graphs:
+        if not graphs or steps == 1 and self.fused is not None:  # one launch: 8.3 us so, 11.1 as a list
             for _ in range(steps):
                 self.step(stream)
             return
