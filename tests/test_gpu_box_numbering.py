@@ -1,5 +1,5 @@
 """Macroscopic fields, moment sums and kinetic energy of boxes whose planes are thin or many (nodes
-numbered flat, coordinates by reciprocals) against the neighbour-array forms of the same lattice."""
+numbered flat, their coordinates by multiplication) against the neighbour-array forms of the same lattice."""
 import numpy as np
 import pytest
 

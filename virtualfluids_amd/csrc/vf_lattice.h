@@ -67,34 +67,6 @@ inline unsigned plane_blocks(int nx, int ny)
     return (unsigned)(((uint64_t)nx * (uint64_t)ny + kPlaneBlock - 1) / kPlaneBlock);
 }
 VF_PLANE_HD uint32_t plane_row(uint32_t t, const PlaneDiv& p) { return (uint32_t)(((double)t + 0.5) * p.invNx); }
-// Flat numbering of a box's nodes, k = x + nx (y + ny z), for kernels that walk the whole box whatever its
-// planes are: z = k / (nx ny) by the same reciprocal.
-struct BoxDiv {
-    PlaneDiv plane;
-    double invPlane; // 1 / (nx ny)
-};
-inline BoxDiv make_box_div(int nx, int ny)
-{
-    const PlaneDiv p = make_plane_div(nx, ny);
-    return BoxDiv{p, 1.0 / (double)p.planeNodes};
-}
-VF_PLANE_HD uint32_t box_plane(uint32_t k, const BoxDiv& b) { return (uint32_t)(((double)k + 0.5) * b.invPlane); }
-
-// A reduction over a lattice ends in one FP64 atomic per workgroup and sum on the same few words,
-// about 10 ns a workgroup one after the other (64^3 moment sums: 18.4 us with 1024 workgroups, 10.6
-// with 256). So the sums take one workgroup of 16 waves per CU, as few as keep HBM busy, and up to 48 k
-// nodes workgroups of four waves, which start and end sooner (moment sums of 20^3 nodes 7.0 -> 5.8 us).
-constexpr int kReduceThreads = 1024;
-constexpr unsigned kReduceGroups = 256;
-struct SumLaunch {
-    dim3 grid, block;
-};
-inline SumLaunch sum_launch(uint64_t nodes)
-{
-    const unsigned threads = nodes <= 48 * 1024 ? 256 : kReduceThreads;
-    const uint64_t pieces = (nodes + threads - 1) / threads;
-    return {dim3((unsigned)(pieces < kReduceGroups ? pieces : kReduceGroups)), dim3(threads)};
-}
 // (x, y) of this thread's node in its plane (blockIdx.y); false for threads beyond the plane
 __device__ __forceinline__ bool plane_xy(const PlaneDiv& p, int& x, int& y)
 {
@@ -104,6 +76,85 @@ __device__ __forceinline__ bool plane_xy(const PlaneDiv& p, int& x, int& y)
     y = (int)r;
     x = (int)(t - r * p.nx);
     return true;
+}
+
+// Flat numbering of a box's nodes, k = x + nx (y + ny z), for kernels that walk the whole box whatever its
+// planes are. k / d of k < 2^30 (numberOfNodes is checked) by a multiplication: with 2^(s-1) < d <= 2^s and
+// m = floor(2^(30+s) / d) + 1, m d exceeds 2^(30+s) by at most d <= 2^s, so k m / 2^(30+s) exceeds k / d by
+// less than 1 / d and has the same integer part.
+struct Divider {
+    uint32_t d, m;
+    int s;
+};
+inline Divider make_divider(uint32_t d)
+{
+    int s = 0;
+    while ((1u << s) < d) ++s;
+    return Divider{d, (uint32_t)((1ull << (30 + s)) / d + 1), s};
+}
+VF_PLANE_HD uint32_t divide(uint32_t k, const Divider& v) { return (uint32_t)(((uint64_t)(k << 2) * v.m) >> 32) >> v.s; }
+struct BoxDiv {
+    Divider plane, row; // by nx ny and by nx
+};
+inline BoxDiv make_box_div(int nx, int ny)
+{
+    return BoxDiv{make_divider((uint32_t)nx * (uint32_t)ny), make_divider((uint32_t)nx)};
+}
+
+// A reduction over a lattice ends in one FP64 atomic per workgroup and sum on the same few words,
+// about 10 ns a workgroup one after the other (64^3 moment sums: 18.4 us with 1024 workgroups, 10.6
+// with 256). So the sums take one workgroup of 16 waves per CU, as few as keep HBM busy, and up to 48 k
+// nodes workgroups of four waves, which start and end sooner (moment sums of 20^3 nodes 7.0 -> 5.8 us).
+// A box is walked in pieces of a workgroup's size: of its planes (SUM_PLANES: the plane is the same for all
+// lanes, and so are the offsets to its neighbours: kinetic energy of 448 x 69 x 231 33.8 us, 38.1 flat) where
+// these fill their last pieces to 9/10 in the mean, else of the flat numbering (2 x 2 x 9000: 5.6, 20.7 by planes).
+constexpr int kReduceThreads = 1024;
+constexpr unsigned kReduceGroups = 256;
+enum SumForm { SUM_INDEXED, SUM_FLAT, SUM_PLANES };
+struct SumLaunch {
+    SumForm form;
+    uint32_t groups, threads; // the launch, also as kernel arguments (reading blockDim costs a load before all else)
+    BoxDiv box;
+};
+inline SumLaunch sum_launch(const vf_lbm_parameter& p)
+{
+    const uint64_t n = p.numberOfNodes;
+    const unsigned threads = n <= 48 * 1024 ? 256 : kReduceThreads;
+    SumForm form = SUM_INDEXED;
+    uint64_t pieces = (n + threads - 1) / threads;
+    if (!p.neighborX) {
+        const uint64_t planes = ((uint64_t)p.nx * p.ny + threads - 1) / threads * p.nz;
+        form = planes * threads * 9 <= n * 10 ? SUM_PLANES : SUM_FLAT;
+        if (form == SUM_PLANES) pieces = planes;
+    }
+    return {form, (uint32_t)(pieces < kReduceGroups ? pieces : kReduceGroups), threads,
+            form == SUM_INDEXED ? BoxDiv{} : make_box_div(p.nx, p.ny)};
+}
+// f(k, z, t) for this thread's nodes k = t + nx ny z of a box (z, t: 0 and k on neighbour arrays)
+template <SumForm FORM, class F> __device__ __forceinline__ void sum_nodes(const Addr& a, const SumLaunch& l, F f)
+{
+    const BoxDiv& b = l.box;
+    if constexpr (FORM == SUM_PLANES) {
+        const uint32_t P = b.plane.d, nz = (uint32_t)a.nz, per = (P + l.threads - 1) / l.threads;
+        // piece i of plane z, and the step to this workgroup's next one
+        uint32_t z = blockIdx.x / per, i = blockIdx.x - z * per;
+        const uint32_t dz = l.groups / per, di = l.groups - dz * per;
+        while (z < nz) {
+            const uint32_t t = i * l.threads + threadIdx.x;
+            if (t < P) f(P * z + t, z, t);
+            z += dz;
+            i += di;
+            if (i >= per) {
+                i -= per;
+                ++z;
+            }
+        }
+    } else {
+        for (uint64_t kk = (uint64_t)blockIdx.x * l.threads + threadIdx.x; kk < a.N; kk += (uint64_t)l.groups * l.threads) {
+            const uint32_t k = (uint32_t)kk, z = FORM == SUM_FLAT ? divide(k, b.plane) : 0;
+            f(k, z, k - b.plane.d * z);
+        }
+    }
 }
 
 template <class S> __device__ __forceinline__ S* slot_ptr(S* f, uint64_t N, int d, bool even)

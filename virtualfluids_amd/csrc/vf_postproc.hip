@@ -126,53 +126,49 @@ __device__ __forceinline__ bool interior_fluid(const Addr& a, const uint32_t* nb
            fl(a.nby[a.nbx[m]]);
 }
 
-__device__ __forceinline__ double node_energy(const float* vx, const float* vy, const float* vz, const float* rho,
-                                              uint32_t k)
+__device__ __forceinline__ double node_energy(float vx, float vy, float vz, float rho)
 {
-    const double ux = vx[k], uy = vy[k], uz = vz[k];
-    return 0.5 * (ux * ux + uy * uy + uz * uz) * ((double)rho[k] + 1.0);
+    const double ux = vx, uy = vy, uz = vz;
+    return 0.5 * (ux * ux + uy * uy + uz * uz) * ((double)rho + 1.0);
 }
 
-// BOX: a dense box, whose seven neighbours are offsets (the coordinates by reciprocals); their types and
-// the node's fields are loaded together (one by one behind the previous test they are eight memory
-// latencies a node). Bound by HBM: 20 bytes a node. 256^3: 156 us with the chain, a division per
-// coordinate and 2048 workgroups, 73 us so.
-template <bool BOX>
+// FORM: sum_launch. The seven neighbours of a box's node are offsets; their types and the node's fields
+// are loaded together (one by one behind the previous test they are eight memory latencies a node).
+// Bound by HBM: 20 bytes a node. 256^3: 155 us with the chain, a division per coordinate and 2048
+// workgroups, 72 us so.
+template <SumForm FORM>
 __global__ __launch_bounds__(kReduceThreads) void kinetic_energy_kernel(Addr a, const uint32_t* nbinv, const uint32_t* geo,
                                                              const float* vx, const float* vy, const float* vz,
-                                                             const float* rho, BoxDiv box, double* out)
+                                                             const float* rho, SumLaunch l, double* out)
 {
     __shared__ double part[kReduceThreads / 64][2];
     double e = 0.0, c = 0.0;
-    const uint64_t step = (uint64_t)gridDim.x * blockDim.x;
-    if constexpr (BOX) {
-        const uint32_t nx = box.plane.nx, ny = (uint32_t)a.ny, nz = (uint32_t)a.nz, P = box.plane.planeNodes;
-        for (uint64_t kk = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; kk < a.N; kk += step) {
-            const uint32_t k = (uint32_t)kk, z = box_plane(k, box), t = k - P * z;
-            const uint32_t y = plane_row(t, box.plane), x = t - y * nx;
+    const uint32_t nx = l.box.row.d, ny = (uint32_t)a.ny, nz = (uint32_t)a.nz, P = l.box.plane.d;
+    sum_nodes<FORM>(a, l, [&](uint32_t k, uint32_t z, uint32_t t) {
+        if constexpr (FORM == SUM_INDEXED) {
+            if (!interior_fluid(a, nbinv, geo, k)) return;
+            e += node_energy(vx[k], vy[k], vz[k], rho[k]);
+            c += 1.0;
+        } else {
+            const uint32_t y = divide(t, l.box.row), x = t - y * nx;
             const uint32_t xp = x + 1 == nx ? t + 1 - nx : t + 1, xm = x == 0 ? t + nx - 1 : t - 1;
             const uint32_t yp = y + 1 == ny ? x : t + nx, ym = y == 0 ? t + (P - nx) : t - nx;
             const uint32_t xym = y == 0 ? xm + (P - nx) : xm - nx;
             const uint32_t zo = P * z, zp = P * (z + 1 == nz ? 0 : z + 1), zm = P * (z == 0 ? nz - 1 : z - 1);
             const uint32_t g[8] = {geo[k],       geo[zo + xp], geo[zo + xm], geo[zo + yp],
                                    geo[zo + ym], geo[zp + t],  geo[zm + t],  geo[zm + xym]};
-            const double en = node_energy(vx, vy, vz, rho, k);
+            float ux = vx[k], uy = vy[k], uz = vz[k], r = rho[k];
+            // needed here: the compiler would move these loads behind the test of the types (256^3 72 -> 95 us)
+            asm volatile("" : "+v"(ux), "+v"(uy), "+v"(uz), "+v"(r));
             bool in = true;
 #pragma unroll
             for (int j = 0; j < 8; ++j) in &= g[j] == VF_GEO_FLUID;
             if (in) {
-                e += en;
+                e += node_energy(ux, uy, uz, r);
                 c += 1.0;
             }
         }
-    } else {
-        for (uint64_t kk = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; kk < a.N; kk += step) {
-            const uint32_t k = (uint32_t)kk;
-            if (!interior_fluid(a, nbinv, geo, k)) continue;
-            e += node_energy(vx, vy, vz, rho, k);
-            c += 1.0;
-        }
-    }
+    });
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     e = wave_sum(e);
     c = wave_sum(c);
@@ -183,7 +179,7 @@ __global__ __launch_bounds__(kReduceThreads) void kinetic_energy_kernel(Addr a, 
     __syncthreads();
     if (threadIdx.x < 2) {
         double s = 0.0;
-        for (unsigned w = 0; w < blockDim.x / 64; ++w) s += part[w][threadIdx.x];
+        for (unsigned w = 0; w < l.threads / 64; ++w) s += part[w][threadIdx.x];
         atomicAdd(out + threadIdx.x, s);
     }
 }
@@ -304,15 +300,13 @@ extern "C" int vf_KineticEnergy(const vf_lbm_parameter* p, const uint32_t* neigh
     }
     hipStream_t s = (hipStream_t)stream;
     hipLaunchKernelGGL(zero2_kernel, dim3(1), dim3(64), 0, s, out2);
-    const SumLaunch l = sum_launch(p->numberOfNodes);
-    if (!p->neighborX) {
-        hipLaunchKernelGGL(kinetic_energy_kernel<true>, l.grid, l.block, 0, s, make_addr(*p), neighborInverse,
-                           p->typeOfGridNode, p->velocityX, p->velocityY, p->velocityZ, p->rho,
-                           make_box_div(p->nx, p->ny), out2);
-    } else {
-        hipLaunchKernelGGL(kinetic_energy_kernel<false>, l.grid, l.block, 0, s,
-                           make_addr(*p), neighborInverse, p->typeOfGridNode, p->velocityX, p->velocityY,
-                           p->velocityZ, p->rho, BoxDiv{}, out2);
-    }
+    const SumLaunch l = sum_launch(*p);
+    const auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(l.groups), dim3(l.threads), 0, s, make_addr(*p), neighborInverse,
+                           p->typeOfGridNode, p->velocityX, p->velocityY, p->velocityZ, p->rho, l, out2);
+    };
+    if (l.form == SUM_INDEXED) launch(kinetic_energy_kernel<SUM_INDEXED>);
+    else if (l.form == SUM_PLANES) launch(kinetic_energy_kernel<SUM_PLANES>);
+    else launch(kinetic_energy_kernel<SUM_FLAT>);
     return check_launch("kineticEnergyKernel execution failed");
 }

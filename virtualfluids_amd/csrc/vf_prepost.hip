@@ -126,11 +126,11 @@ __device__ __forceinline__ bool is_valid_fluid(uint32_t t)
     return t == VF_GEO_FLUID || t == VF_GEO_PM_0 || t == VF_GEO_PM_1 || t == VF_GEO_PM_2;
 }
 
-// The cell nodes of node k of a dense box
-__device__ __forceinline__ void box_cell_nodes(const BoxDiv& b, int ny, int nz, uint32_t k, uint32_t (&n)[8])
+// The cell nodes of node t of plane z (t = x + nx y) of a dense box
+__device__ __forceinline__ void plane_cell_nodes(const BoxDiv& b, int ny, int nz, uint32_t z, uint32_t t, uint32_t (&n)[8])
 {
-    const uint32_t P = b.plane.planeNodes, nx = b.plane.nx;
-    const uint32_t z = box_plane(k, b), t = k - P * z, y = plane_row(t, b.plane), x = t - y * nx;
+    const uint32_t P = b.plane.d, nx = b.row.d;
+    const uint32_t y = divide(t, b.row), x = t - y * nx;
     const uint32_t xp = x + 1 == nx ? 0 : x + 1;
     const uint32_t r0 = t - x, r1 = y + 1 == (uint32_t)ny ? 0 : r0 + nx;
     const uint32_t z0 = P * z, z1 = z + 1 == (uint32_t)nz ? 0 : z0 + P;
@@ -165,7 +165,7 @@ __device__ __forceinline__ void node_moments(const float (&f)[27], double& drho,
     }
 }
 
-// BOX: the cell nodes of a dense box by reciprocals; populations through buffer descriptors where they
+// BOX: the cell nodes of a dense box by multiplication; populations through buffer descriptors where they
 // reach. Bound by HBM: 27 populations, the type and five fields a node. 256^3 FP32: 429 us with a
 // division per coordinate and every field written twice (zero, then the value), 396 so.
 template <class S, bool BOX, bool BUF>
@@ -180,8 +180,12 @@ __global__ __launch_bounds__(256) void macroscopic_kernel(const S* __restrict__ 
     // whole lines (448 x 115 x 327 BF16, one solid node in ten: 226 us, 312 with a store of its own for each)
     float drho = 0.0f, ux = 0.0f, uy = 0.0f, uz = 0.0f, pr = 0.0f;
     if (!geo || is_valid_fluid(geo[k])) {
-        if constexpr (BOX) box_cell_nodes(box, a.ny, a.nz, (uint32_t)k, n);
-        else cell_nodes(a, (uint32_t)k, n);
+        if constexpr (BOX) {
+            const uint32_t z = divide((uint32_t)k, box.plane);
+            plane_cell_nodes(box, a.ny, a.nz, z, (uint32_t)k - box.plane.d * z, n);
+        } else {
+            cell_nodes(a, (uint32_t)k, n);
+        }
         const SlotIO<S, BUF> io(f, a.N);
         float fv[27];
         load_cell<S, BUF>(io, n, even_flag != 0, fv);
@@ -224,9 +228,9 @@ __device__ __forceinline__ double wave_sum(double v)
 }
 
 // out[0..3] += sum drho, jx, jy, jz; out[4] += sum 1/2 (1+drho) |u|^2 (when KE).
-// BOX, BUF as in macroscopic_kernel; launched by sum_launch. Bound by HBM: 27 populations and the type a node (256^3 FP32 327 us, FP16 197 -> 174 us).
-template <class S, bool KE, bool BOX, bool BUF>
-__global__ __launch_bounds__(kReduceThreads) void moments_reduce_kernel(const S* __restrict__ f, Addr a, BoxDiv box,
+// FORM: sum_launch; BUF as in macroscopic_kernel. Bound by HBM: 27 populations and the type a node (256^3 FP32 327 us, FP16 197 -> 174 us).
+template <class S, bool KE, SumForm FORM, bool BUF>
+__global__ __launch_bounds__(kReduceThreads) void moments_reduce_kernel(const S* __restrict__ f, Addr a, SumLaunch l,
                                                              const uint32_t* geo, int even_flag, double* out)
 {
     constexpr int NV = KE ? 5 : 4;
@@ -248,13 +252,13 @@ __global__ __launch_bounds__(kReduceThreads) void moments_reduce_kernel(const S*
             acc[NV - 1] += 0.5 * (jx * jx + jy * jy + jz * jz) / (1.0 + drho);
         }
     };
-    uint32_t n[8];
-    for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k < a.N; k += (uint64_t)gridDim.x * blockDim.x) {
-        if (geo && geo[k] != VF_GEO_FLUID) continue;
-        if constexpr (BOX) box_cell_nodes(box, a.ny, a.nz, (uint32_t)k, n);
-        else cell_nodes(a, (uint32_t)k, n);
+    sum_nodes<FORM>(a, l, [&](uint32_t k, uint32_t z, uint32_t t) {
+        if (geo && geo[k] != VF_GEO_FLUID) return;
+        uint32_t n[8];
+        if constexpr (FORM == SUM_INDEXED) cell_nodes(a, k, n);
+        else plane_cell_nodes(l.box, a.ny, a.nz, z, t, n);
         add(n);
-    }
+    });
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
@@ -264,7 +268,7 @@ __global__ __launch_bounds__(kReduceThreads) void moments_reduce_kernel(const S*
     __syncthreads();
     if (threadIdx.x < NV) {
         double s = 0.0;
-        for (unsigned w = 0; w < blockDim.x / 64; ++w) s += part[w][threadIdx.x];
+        for (unsigned w = 0; w < l.threads / 64; ++w) s += part[w][threadIdx.x];
         atomicAdd(out + threadIdx.x, s);
     }
 }
@@ -321,18 +325,24 @@ template <class S> struct MacroL {
     }
 };
 template <class S> struct ReduceL {
-    template <bool KE, bool BOX, bool BUF> static void go(const vf_lbm_parameter& p, double* out, hipStream_t s)
+    template <bool KE, SumForm FORM, bool BUF>
+    static void go(const vf_lbm_parameter& p, const SumLaunch& l, double* out, hipStream_t s)
     {
-        const SumLaunch l = sum_launch(p.numberOfNodes);
-        hipLaunchKernelGGL((moments_reduce_kernel<S, KE, BOX, BUF>), l.grid, l.block, 0, s, (const S*)p.distributions,
-                           make_addr(p), BOX ? make_box_div(p.nx, p.ny) : BoxDiv{}, p.typeOfGridNode,
-                           p.isEvenTimestep, out);
+        hipLaunchKernelGGL((moments_reduce_kernel<S, KE, FORM, BUF>), dim3(l.groups), dim3(l.threads), 0, s,
+                           (const S*)p.distributions, make_addr(p), l, p.typeOfGridNode, p.isEvenTimestep, out);
+    }
+    template <bool KE, SumForm FORM>
+    static void box(const vf_lbm_parameter& p, const SumLaunch& l, double* out, hipStream_t s)
+    {
+        if (buffers<S>(p)) go<KE, FORM, true>(p, l, out, s);
+        else go<KE, FORM, false>(p, l, out, s);
     }
     template <bool KE> static void pick(const vf_lbm_parameter& p, double* out, hipStream_t s)
     {
-        if (p.neighborX) go<KE, false, false>(p, out, s);
-        else if (buffers<S>(p)) go<KE, true, true>(p, out, s);
-        else go<KE, true, false>(p, out, s);
+        const SumLaunch l = sum_launch(p);
+        if (l.form == SUM_INDEXED) go<KE, SUM_INDEXED, false>(p, l, out, s);
+        else if (l.form == SUM_PLANES) box<KE, SUM_PLANES>(p, l, out, s);
+        else box<KE, SUM_FLAT>(p, l, out, s);
     }
     static void run(const vf_lbm_parameter& p, double* out, bool ke, hipStream_t s)
     {
