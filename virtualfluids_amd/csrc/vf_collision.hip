@@ -571,6 +571,9 @@ template <class S> static int box_row_width(const vf_lbm_parameter& p, bool into
     if (pinned) return V;
     if (ws <= kCacheResidentBytes || (p.nx / V) % 64 != 0) return 0;
     const int waves = p.nx / V / 64;
+    // BF16 rows of five and seven waves with solid nodes: 640 x 228 x 92 with walls 390 in the row kernel, 297 us in
+    // the node kernel, 896 x 100 x 100 212 / 198 (without 640 x 250 x 250 867 / 877, 896 x 100 x 100 188 / 200)
+    if (sizeof(S) == 2 && waves > 4 && p.fluidMask) return 0;
     if (sizeof(S) == 4 && (waves == 1 || (!into && waves > 4 && waves < 8 && ws <= kNearCacheBytes))) return 0;
     return V;
 }
