@@ -434,6 +434,8 @@ class _TwoLevelSteps(torch.autograd.Function):
             n = min(K - i % K, steps - i, (observe_from - i) if observe is not None else steps)
             even = run.run(n, even)
             i += n
+        if any(ctx.needs_input_grad):
+            cells[0].sources(sc.L.grid)  # the backward's tables, while the steps run
         run.close()
         ctx.sc, ctx.sf, ctx.cells, ctx.steps, ctx.K = sc, sf, cells, steps, K
         ctx.in_place = in_place
@@ -843,6 +845,9 @@ class _MultiLevelSteps(torch.autograd.Function):
             n_run = min(K - i % K, steps - i, (observe_from - i) if observe is not None else steps)
             even = run.run(n_run, even)
             i += n_run
+        if any(ctx.needs_input_grad):
+            for (cf, _), L in zip(cells, lats):
+                cf.sources(L.grid)  # the backward's tables, while the steps run
         run.close()
         ctx.meta = meta
         ctx.checkpoints = checkpoints
