@@ -137,13 +137,13 @@ def test_a_given_stream_is_not_waited_for():
 
 
 def test_asking_waits_for_the_steps_that_pay_for_it(monkeypatch):
-    """About 5 ns a node against 2 us a step: long lists ask later than the 512 steps of short ones."""
+    """2 to 5 ns a node against 2 us a step: long lists ask later than the 512 steps of short ones."""
     from virtualfluids_amd import simulation
 
     asked = []
     monkeypatch.setattr(simulation, "paired_launches",
                         lambda lattice, groups: asked.append(1) or [(fn, [(name, bc)]) for name, fn, bc in groups])
-    for nodes, steps in ((100, 512), (100_000, 512), (1_000_000, 5000)):
+    for nodes, steps in ((100, 512), (200_000, 512), (1_000_000, 2500)):
         sim = _channel()
         for _, _, bc in sim._post_groups():
             bc.n = nodes // 2

@@ -367,7 +367,7 @@ class Simulation:
                 return self._paired[1]
             self._paired, self._unpaired_steps = None, 0
         self._unpaired_steps += steps
-        if (self._unpaired_steps < max(512, sum(bc.n for _, _, bc in groups) // 200) or stream is not None
+        if (self._unpaired_steps < max(512, sum(bc.n for _, _, bc in groups) // 400) or stream is not None
                 or self.lattice.device.type == "cuda" and torch.cuda.is_current_stream_capturing()):
             return [(fn, [(name, bc)]) for name, fn, bc in groups]
         self._paired = (groups, paired_launches(self.lattice, groups))
