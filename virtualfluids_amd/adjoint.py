@@ -290,12 +290,12 @@ class _K17Steps(torch.autograd.Function):
             if start in ctx.kept:
                 states, posts = ctx.kept.pop(start)
             else:
-                states = [ckpt]
-                # the post-collision values of the BC nodes, step by step, for the BC adjoints
-                posts = [{name: torch.empty(27 * nb, dtype=torch.float32, device=lam.device) for name, nb in lists}
-                         for _ in range(n)]
+                # the states and the post-collision values of the BC nodes, step by step, for the BC adjoints
+                states, posts = [ckpt], []
                 even = even_start
                 for j in range(n):
+                    posts.append({name: torch.empty(27 * nb, dtype=torch.float32, device=lam.device)
+                                  for name, nb in lists})
                     states.append(stepper.forward(states[-1], even, torch.empty_like(ckpt), stream, save=posts[j]))
                     even = not even
             for j in reversed(range(n)):
@@ -489,12 +489,12 @@ class _TwoLevelSteps(torch.autograd.Function):
             if start in ctx.kept:
                 states, posts = ctx.kept.pop(start)
             else:
-                states = []
-                # the post-collision values of every level's BC nodes, step by step, for the BC
-                # adjoints
-                posts = [(post_buffers(lists_c), post_buffers(lists_f), post_buffers(lists_f)) for _ in range(n)]
+                # the states and the post-collision values of every level's BC nodes, step by step, for the
+                # BC adjoints
+                states, posts = [], []
                 C, F, even = C0, F0, even_start
                 for j in range(n):
+                    posts.append((post_buffers(lists_c), post_buffers(lists_f), post_buffers(lists_f)))
                     st = _two_level_step(sc, sf, cells, C, F, even, stream, posts[j], ctx.in_place)
                     states.append((even, C, F) + st)
                     C, F = st[-2], st[-1]
