@@ -122,3 +122,31 @@ def test_lattices_beyond_two_descriptors(gpu, shape):
     into = torch.zeros_like(f)
     capi.call("vf_k17_run_box_into", P, into.data_ptr(), s)
     assert slots_equal(into, stepped)
+
+
+@pytest.mark.parametrize("storage", ["fp32", "fp16", "bf16"])
+@pytest.mark.parametrize("solid", [False, True])
+def test_write_macro_vars_leaves_the_same_populations(gpu, storage, solid):
+    """A collision that also writes the macroscopic values (64-bit addresses on 16-bit lattices that fit
+    the cache) leaves the populations of the plain one."""
+    import torch
+
+    from virtualfluids_amd.grid import GEO_SOLID
+    from virtualfluids_amd.lattice import Lattice
+
+    g = periodic_box(33, 31, 6)
+    rng = np.random.default_rng(9)
+    if solid:
+        s = rng.random(g.N) < 0.1
+        g.geo = np.where(s, GEO_SOLID, g.geo).astype(np.uint32)
+        g.fluid = np.nonzero(~s)[0].astype(np.uint32)
+    pre = near_equilibrium(rng, g.N, u_amp=0.04, noise=5e-3)
+    for even in (True, False):
+        out = []
+        for macro in (True, False):
+            L = Lattice(g, 1.9, storage=storage)
+            L.even = even
+            L.set_populations(pack_pre(pre, g, even))
+            L.collide(write_macro=macro)
+            out.append(L.f.clone())
+        assert torch.equal(*out)

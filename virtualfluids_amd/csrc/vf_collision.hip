@@ -663,10 +663,21 @@ template <class S> static NodeLaunch node_launch(const vf_lbm_parameter& p, bool
     return {xcd, lds_reserve_for(cap)};
 }
 
-// Buffer descriptors where 14 slots lie within 4 GiB, unless 64-bit addresses are pinned
-template <class S> static bool node_buffers(const vf_lbm_parameter& p)
+// Launches that write macroscopic values near the cache keep 64-bit addresses and no cap, whose registers
+// leave four or five workgroups per CU: with buffers and the cap, us, 512 x 68 x 64 FP32 91 -> 101, 300 x 90 x 90
+// 99 -> 108, 67 x 130 x 266 BF16 57 -> 62, 164 x 87 x 167 FP16 58 -> 62. FP32 lattices that stream gain by them
+// (258 x 130 x 130 234 -> 216), below half the cache and in 16 bits beyond it the forms are even.
+template <class S> static bool macro_near_cache(const vf_lbm_parameter& p, bool macro)
 {
-    return slots_fit_buffers(p.numberOfNodes, sizeof(S)) && p.kernelChoice.rowAddressing != VF_ROW_ADDRESSING_GLOBAL;
+    const uint64_t own = 27 * p.numberOfNodes * sizeof(S);
+    return macro && (sizeof(S) == 2 ? own <= kCacheResidentBytes : own > kCacheResidentBytes / 2 && own <= kNearCacheBytes);
+}
+
+// Buffer descriptors where 14 slots lie within 4 GiB, unless 64-bit addresses are pinned
+template <class S> static bool node_buffers(const vf_lbm_parameter& p, bool macro = false)
+{
+    return slots_fit_buffers(p.numberOfNodes, sizeof(S)) && p.kernelChoice.rowAddressing != VF_ROW_ADDRESSING_GLOBAL &&
+           !macro_near_cache<S>(p, macro);
 }
 
 template <class S, bool EVEN, bool BUF>
@@ -676,7 +687,8 @@ static void launch_node_b(const vf_lbm_parameter& p, const BoxArgs& a, const K17
     const bool mask = p.fluidMask != nullptr;
     const dim3 grid(plane_blocks(p.nx, p.ny), p.nz), bx(kBoxBlock);
     const FusedBB none{};
-    const auto [xcd, lds] = node_launch<S>(p, false, !macro);
+    const auto [xcd, cap] = node_launch<S>(p, false, !macro);
+    const size_t lds = macro_near_cache<S>(p, macro) ? 0 : cap;
     if (mask && macro) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, BUF, true, true>), grid, dim3(bx), lds, s, f, a, r, none);
     else if (mask && xcd) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, BUF, true, false, false, true>), grid, dim3(bx), lds, s, f, a, r, none);
     else if (mask) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, BUF, true, false>), grid, dim3(bx), lds, s, f, a, r, none);
@@ -692,7 +704,7 @@ static void launch_box_t(const vf_lbm_parameter& p, bool macro, hipStream_t s)
               p.porosity, make_plane_div(p.nx, p.ny)};
     const K17Rates r = make_k17_rates(p);
     if (try_launch_row<S, EVEN>(p, a, r, macro, nullptr, s)) return;
-    if (node_buffers<S>(p)) launch_node_b<S, EVEN, true>(p, a, r, macro, s);
+    if (node_buffers<S>(p, macro)) launch_node_b<S, EVEN, true>(p, a, r, macro, s);
     else launch_node_b<S, EVEN, false>(p, a, r, macro, s);
 }
 
@@ -703,7 +715,8 @@ static void launch_node_bb_b(const vf_lbm_parameter& p, const BoxArgs& a, const 
     S* f = static_cast<S*>(p.distributions);
     const bool mask = p.fluidMask != nullptr;
     const dim3 grid(plane_blocks(p.nx, p.ny), p.nz), bx(kBoxBlock);
-    const auto [xcd, lds] = node_launch<S>(p, false, mask && !macro);
+    const auto [xcd, cap] = node_launch<S>(p, false, mask && !macro);
+    const size_t lds = macro_near_cache<S>(p, macro) ? 0 : cap;
     if (mask && macro) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, BUF, true, true, true>), grid, dim3(bx), lds, s, f, a, r, bb);
     else if (mask && xcd) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, BUF, true, false, true, true>), grid, dim3(bx), lds, s, f, a, r, bb);
     else if (mask) hipLaunchKernelGGL((k17_box_kernel<S, EVEN, BUF, true, false, true>), grid, dim3(bx), lds, s, f, a, r, bb);
@@ -720,7 +733,7 @@ static bool launch_box_bb_t(const vf_lbm_parameter& p, bool macro, const FusedBB
     BoxArgs a{p.numberOfNodes, p.nx, p.ny, p.nz, p.fluidMask, p.rho, p.velocityX, p.velocityY, p.velocityZ,
               p.porosity, make_plane_div(p.nx, p.ny)};
     const K17Rates r = make_k17_rates(p);
-    if (node_buffers<S>(p)) launch_node_bb_b<S, EVEN, true>(p, a, r, macro, bb, s);
+    if (node_buffers<S>(p, macro)) launch_node_bb_b<S, EVEN, true>(p, a, r, macro, bb, s);
     else launch_node_bb_b<S, EVEN, false>(p, a, r, macro, bb, s);
     return true;
 }
