@@ -757,7 +757,14 @@ template <class S, bool EVEN>
 static void launch_indexed_t(const vf_lbm_parameter& p, const uint32_t* idx, uint32_t n, bool macro, bool force,
                              hipStream_t s)
 {
-    if (node_buffers<S>(p)) launch_indexed_b<S, EVEN, true>(p, idx, n, macro, force, s);
+    // Buffers serve the plain collision in 16 bits and up to the cache's size in FP32 (us, 64-bit addresses and
+    // buffers: 267 x 233 x 234 BF16 440 / 421, 182 x 113 x 114 FP32 122 / 119). FP32 lattices that stream, and
+    // from a quarter of the cache the templates that read or write more fields, run better with the fewer
+    // workgroups that 64-bit addresses leave on a CU (104 x 397 x 397 FP32 765 / 809; writing the macroscopic
+    // values 147 x 358 x 359 FP16 607 / 636).
+    const uint64_t own = 27 * p.numberOfNodes * sizeof(S);
+    const bool fewer = macro || force ? own > kCacheResidentBytes / 4 : sizeof(S) == 4 && own > kCacheResidentBytes;
+    if (node_buffers<S>(p) && !fewer) launch_indexed_b<S, EVEN, true>(p, idx, n, macro, force, s);
     else launch_indexed_b<S, EVEN, false>(p, idx, n, macro, force, s);
 }
 
