@@ -160,3 +160,32 @@ def test_one_step_of_one_launch_builds_no_list(gpu, monkeypatch):
     assert not built and sim.t == 2 and L.even
     sim.run(2)
     assert built and sim.t == 4 and L.even
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("steps", [2, 3, 7])
+def test_k17_steps_inside_a_captured_graph(gpu, steps):
+    """A caller's graph around k17_steps records its launches: the wait that ends a sweep of three or more
+    steps is left out, every replay gives the eager result."""
+    import torch
+
+    from virtualfluids_amd.adjoint import k17_steps
+    from virtualfluids_amd.graphs import capture
+    from virtualfluids_amd.lattice import Lattice
+
+    g = channel((17, 9, 7), inflow=0.03)
+    L = Lattice(g, 1.7)
+    z = np.zeros(g.N)
+    L.init_equilibrium(z, np.where(g.geo == 19, 0.02, 0.0), z, z)
+    x = L.f.clone()
+    with torch.no_grad():
+        k17_steps(x, L, 2, even=True, bc_factory=_factory(False))
+        out = {}
+        graph = capture(lambda st: out.update(y=k17_steps(x, L, steps, even=True, bc_factory=_factory(False))),
+                        torch.cuda.Stream())
+        for i in range(3):
+            graph.replay()
+            ref = k17_steps(x, L, steps, even=True, bc_factory=_factory(False))
+            assert torch.equal(out["y"], ref), f"replay {i}"
+            x.copy_(ref)
+    torch.cuda.synchronize()

@@ -125,6 +125,6 @@ class StepLaunches:
 
     def close(self):
         """Wait for the steps, as Simulation.run does: a sweep of three or more native steps has
-        returned when they are done."""
-        if self.enqueued >= 3:
+        returned when they are done. Inside a caller's capture there is nothing to wait for."""
+        if self.enqueued >= 3 and not torch.cuda.is_current_stream_capturing():
             torch.cuda.current_stream().synchronize()
