@@ -508,11 +508,11 @@ template <class S> static int row_width(int nx, const vf_kernel_choice& kc)
 // streams from HBM (fewer concurrent direction streams per memory channel), as long as at least
 // eight waves are resident: measured on MI355X, us per step, rows of one wave (64 x 300 x 300) 532
 // at 2, 311 at 4, 232 at 8, 238 without a cap; of two (128 x 300 x 300) 588 at 2, 438 at 4, 457
-// without; of four (256 x 200 x 200) 396 at 2, 389 at 4, 404 without; of eight (512^3) 6394 at 1, 5021
-// at 2, 5901 at 4, 5857 without. A working set that fits the 256 MB infinity cache is
-// latency-bound instead and takes every wave. The 16-bit kernels are bound by VALU issue and need
-// every wave they can get. The cap is imposed by reserving LDS at launch;
-// kernelChoice.rowWorkgroupsPerCU pins it.
+// without; of four (256 x 200 x 200) 396 at 2, 389 at 4, 404 without (17 lattices: 4 over 2 0.947 to
+// 1.027, mean 0.994; 256^3 622.1 to 620.3); of eight (512^3) 6394 at 1, 5021 at 2, 5901 at 4, 5857
+// without. A working set that fits the 256 MB infinity cache is latency-bound instead and takes
+// every wave. The 16-bit kernels are bound by VALU issue and need every wave they can get. The cap
+// is imposed by reserving LDS at launch; kernelChoice.rowWorkgroupsPerCU pins it.
 constexpr uint64_t kCacheResidentBytes = 256ull << 20;
 constexpr uint64_t kNearCacheBytes = kCacheResidentBytes / 4 * 5; // the cache still serves a good part
 template <class S, int V, int SPLIT> static int row_wgs_per_cu(uint64_t workingSet, int waves, const vf_kernel_choice& kc)

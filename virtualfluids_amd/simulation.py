@@ -355,10 +355,10 @@ class Simulation:
         paired_launches once enough steps have been asked for, until then a launch per group. A shared
         launch saves 2 to 4 us a step. Finding out whether the lists allow it takes 0.2 ms of host time
         and 1 to 5 ns a node (87 000 nodes 0.4 ms, 615 000 1.2 ms), so it waits for 512 steps and
-        for a step per 200 nodes; it also waits for the current stream's work, so calls with a stream of
-        their own or inside a capture do not ask. A pair whose lists are written to afterwards (as torch
-        counts; a program that writes them through raw pointers takes a new Simulation) is given up, and
-        asked for again after as many steps."""
+        for a step per 400 nodes (per 200 cost a two-level run 0.9 %); it also waits for the current
+        stream's work, so calls with a stream of their own or inside a capture do not ask. A pair whose
+        lists are written to afterwards (as torch counts; a program that writes them through raw
+        pointers takes a new Simulation) is given up, and asked for again after as many steps."""
         import torch
 
         groups = self._post_groups()
